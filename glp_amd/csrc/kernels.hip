@@ -1115,28 +1115,28 @@ __device__ __forceinline__ void hub_part_count(const StepArgs& a, const HubArgs&
     if (threadIdx.x == 0 && best) atomicMax(&h.hs.best[j.hub], (unsigned long long)best);
 }
 
-// One workgroup per batch of kPartBatch parts: each wave sums the run
+// One workgroup per batch of part_batch parts: each wave sums the run
 // lengths of a quarter of them, the non-empty ones are listed in LDS and
 // counted one after another.  Once labels converge nearly every bucket is
 // empty, and a launch of one workgroup per part would spend its time
 // starting and ending them; while labels are diverse every bucket is full,
 // and a long batch would count its parts in series on one CU.  16 parts per
 // workgroup measured best over both (hub_part on RMAT-25: diverse steps 2.8
-// -> 1.8 ms against 256 parts, converged 0.11 -> 0.085 ms).
-constexpr int kPartBatch = 16;
+// -> 1.8 ms against 256 parts, converged 0.11 -> 0.085 ms) where that still
+// fills the chip; fewer parts take shorter batches (hub_part_batch).
 
 template <class H>
 __device__ __forceinline__ void hub_part_batch_body(const StepArgs& a, const HubArgs& h,
                                                     uint32_t blk) {
     extern __shared__ __align__(16) uint32_t s_dyn[];
-    __shared__ PartJob s_jobs[kPartBatch];
+    __shared__ PartJob s_jobs[kPartBatchMax];
     __shared__ unsigned long long s_red[kHubThreads / 64];
     __shared__ uint32_t s_n, s_distinct, s_over;
     if (threadIdx.x == 0) s_n = 0u;
     __syncthreads();
     const int lane = lane_id();
-    for (int k = threadIdx.x >> 6; k < kPartBatch; k += kHubThreads / 64) {
-        const int32_t p = (int32_t)blk * kPartBatch + k;
+    for (int k = threadIdx.x >> 6; k < h.part_batch; k += kHubThreads / 64) {
+        const int32_t p = (int32_t)blk * h.part_batch + k;
         if (p >= h.nparts) break;  // wave-uniform
         const int2 hp = h.parts[p];
         const int32_t v = h.hubs[hp.x];
@@ -1406,7 +1406,8 @@ void job_blocks(const Plan& p, int32_t* blocks) {
     blocks[kLaunchWave] = (int32_t)((p.wave.size() + 4 * kWaveNV - 1) / (4 * kWaveNV));
     for (int c = 0; c < p.nclasses; ++c) blocks[kLaunchBlock0 + c] = (int32_t)p.block[c].size();
     blocks[kLaunchHubAgg] = (int32_t)p.hub_chunks.size();
-    blocks[kLaunchHubPart] = (int32_t)((p.hub_parts.size() + kPartBatch - 1) / kPartBatch);
+    const int32_t pb = hub_part_batch((int64_t)p.hub_parts.size());
+    blocks[kLaunchHubPart] = (int32_t)((p.hub_parts.size() + pb - 1) / pb);
     blocks[kLaunchHubFinal] = (int32_t)((p.hubs.size() + 255) / 256);
 }
 
@@ -2027,6 +2028,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
         h.part_limit = p.tune.part_limit;
         h.nhubs = (int32_t)p.hubs.size();
         h.nparts = (int32_t)p.hub_parts.size();
+        h.part_batch = hub_part_batch(h.nparts);
         h.hs = hs;
         const unsigned nc = (unsigned)p.hub_chunks.size();
         const unsigned np = (unsigned)p.hub_parts.size();
@@ -2035,7 +2037,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
                            hub_agg_lds(h.chunk, p.hub_max_buckets), s, a, h);
         mark(GLP_TIER_HUB, 1);
         mark(GLP_TIER_AUX, 0);
-        hipLaunchKernelGGL((k_hub_part<H>), dim3((np + kPartBatch - 1) / kPartBatch), dim3(kHubThreads),
+        hipLaunchKernelGGL((k_hub_part<H>), dim3((np + h.part_batch - 1) / h.part_batch), dim3(kHubThreads),
                            lds_part, s, a, h);
         hipLaunchKernelGGL((k_hub_final<H>), dim3(grid_for(h.nhubs, 256)), dim3(256), 0, s, a, h);
         if (H::kFrontier && a.act_w)

@@ -488,6 +488,7 @@ int glp_server::step_jobs(const std::vector<ServerJob*>& jobs, hipStream_t s, Ti
         h.part_limit = p.tune.part_limit;
         h.nhubs = (int32_t)p.hubs.size();
         h.nparts = (int32_t)p.hub_parts.size();
+        h.part_batch = hub_part_batch(h.nparts);
         h.hs = j->hs;
         job_blocks(p, d.blocks);
     }

@@ -126,6 +126,18 @@ def test_hub_partition_and_halving(limit):
     assert_steps_equal(dump, O.classic(off, nbr, 5))
 
 
+@pytest.mark.parametrize("n", [1500, 5000, 9000, 20000, 41000])
+def test_hub_part_batches(n):
+    """Every vertex a one-part hub: the part counts lie in each batch length
+    of the counting pass (1, 2, 4, 8 and 16 parts per workgroup)."""
+    with G.tuning(pack_max_deg=2, half_max_deg=0, wave_max_deg=2, block_max_deg=2, hub_chunk=256, part_keys=256):
+        g = G.Graph.planted(n, max(1, n // 500), 10.0, 2.0, seed=5)
+        off, nbr, _ = g.csr()
+        _, dump, timing = G.run(g, 3, dump=True)
+    assert timing["tier_vertices"]["hub"] > 0.95 * n
+    assert_steps_equal(dump, O.classic(off, nbr, 3))
+
+
 def test_hub_weighted_small_tiers():
     with G.tuning(pack_max_deg=4, wave_max_deg=8, block_max_deg=16, hub_chunk=256, part_keys=256):
         g = G.Graph.rmat(13, 16, seed=22, wmax=8)

@@ -37,9 +37,9 @@
 // the packed maximum with a 64-bit atomic max, a third commits).  Frequent and buffer: one lane per
 // vertex up to kTableLaneMaxDeg edges (the lane walks its table slot by
 // slot), one wavefront per vertex above, with table slot i held by lane i
-// and each edge applied by the whole wavefront in CSR order: the order the
-// semantics fix, so both forms give the same table.  The vertices above the
-// thresholds are listed once per session.
+// and the edges applied in CSR order, the order the semantics fix, several at
+// once where that gives the same table, so both forms agree.  The vertices
+// above the thresholds are listed once per session.
 
 #include "device.h"
 #include "device_prims.h"
@@ -420,19 +420,398 @@ __device__ __forceinline__ uint32_t wave_min_dpp(uint32_t x) {
     return min(min(r0, r1), min(r2, r3));
 }
 
-// One wavefront per vertex of `verts` (degrees above kTableLaneMaxDeg):
-// slot i of the vertex's table is lane i's (K, C); lanes >= cap hold the key
-// 0xffffffff, which no edge carries (keys are labels + 1 <= 2^31), so they
-// never match and are never free.  Edges are applied one after another in
-// CSR order; a table's keys are distinct, so at most one lane hits.  The
-// vertex and its edge range are wave-uniform (scalar loop control), and
-// edges come in chunks of 64, one per lane: while chunk c is applied, chunk
-// c+1's labels and chunk c+2's neighbour ids are in flight.  Lanes past the
-// last edge load the last edge again (in bounds, never applied), so the
-// loads need no branches and stay in flight across the chunk.
+// A wide table: slot i is lane i's (K, A).  A slot's count is A - off, so a
+// drop of every slot is one scalar addition to `off`; `fr` holds the free
+// slots (key 0).  Lanes >= cap hold the key 0xffffffff, which no edge carries
+// (keys are labels + 1 <= 2^31), and the largest A: they never match, are
+// never free and never the smallest.  A and off stay below 2^31 (the host
+// checks the largest frequency sum).
+struct WideTable {
+    uint32_t K, A;
+    uint32_t off;  // wave-uniform
+    uint64_t fr;   // wave-uniform
+};
+
+// Applies a chunk's edges (lane l: key, frequency f; `all` the lanes with an
+// edge) at once where that gives what applying them in order gives: no edge
+// misses, or the table is full and its smallest count exceeds what all the
+// misses together take off, so no slot can empty between them.  False (and
+// nothing applied) otherwise.  `sum` is the wave's LDS.
+template <bool W>
+__device__ __forceinline__ bool table_bulk(uint32_t key, uint32_t f, uint64_t all, int32_t cap, WideTable& t,
+                                           uint32_t* sum) {
+    const int lane = lane_id();
+    int32_t at = -1;  // the slot holding this edge's key
+#pragma unroll 4
+    for (int32_t s = 0; s < cap; ++s)
+        at = key == (uint32_t)__builtin_amdgcn_readlane((int)t.K, s) ? s : at;
+    const bool in = (all >> lane) & 1u;
+    const uint64_t miss = __ballot(in && at < 0);
+    uint32_t drop = 0u;
+    if (miss) {
+        if (t.fr) return false;
+        drop = W ? wave_sum_u32(in && at < 0 ? f : 0u) : (uint32_t)__popcll(miss);
+        drop = (uint32_t)__builtin_amdgcn_readfirstlane((int)drop);
+        if (__ballot(t.A <= t.off + drop)) return false;
+    }
+    sum[lane] = 0u;
+    wave_lds_sync();
+    if (in && at >= 0) atomicAdd(&sum[at], W ? f : 1u);
+    wave_lds_sync();
+    t.A += sum[lane];
+    t.off += drop;
+    wave_lds_sync();
+    return true;
+}
+
+// Lane src's 64-bit value, held as two words.
+__device__ __forceinline__ uint64_t readlane_u64(uint32_t lo, uint32_t hi, int src) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, src) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)lo, src);
+}
+// Set bits of m below this lane.
+__device__ __forceinline__ uint32_t rank_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+constexpr int kTableBlk = 4;               // most chunks of 64 edges loaded together
+constexpr uint32_t kNoEdge = 0xfffffffeu;  // key of a lane past the last edge
+
+// For each of a block's chunks (lane l: edge l's key) the edge lanes whose
+// key may occur more than once in the chunk: every one that does, and the few
+// that share a hash bit.  The block's chunks go through LDS together, so its
+// latency is paid once.
+constexpr uint32_t kDupWords = 128;
+struct TableLds {
+    uint32_t bits[kTableBlk][2][kDupWords];  // per chunk 4,096 bits: a key hashed here; another one did
+};
+template <int B>
+__device__ __forceinline__ void table_repeats(const uint32_t* key, uint64_t* dup, TableLds& t) {
+    const int lane = lane_id();
+    uint32_t* flat = &t.bits[0][0][0];
+#pragma unroll
+    for (uint32_t i = 0; i < B * 2 * kDupWords; i += 64) flat[i + (uint32_t)lane] = 0u;
+    wave_lds_sync();
+    uint32_t w[B], bit[B], old[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        const uint32_t h = (key[u] * 0x9e3779b1u) >> 20;
+        static_assert(kDupWords * 32 == 1u << (32 - 20), "one bit per hash value");
+        w[u] = h >> 5;
+        // lanes past the last edge set no bit
+        bit[u] = key[u] != kNoEdge ? 1u << (h & 31u) : 0u;
+        old[u] = atomicOr(&t.bits[u][0][w[u]], bit[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) atomicOr(&t.bits[u][1][w[u]], old[u] & bit[u]);
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < B; ++u) old[u] = t.bits[u][1][w[u]];
+#pragma unroll
+    for (int u = 0; u < B; ++u) dup[u] = __ballot((old[u] & bit[u]) != 0u);
+    wave_lds_sync();
+}
+
+// Applies an unweighted chunk (lane l: edge l's key; `all` the lanes with an
+// edge, the others' key kNoEdge; `dup` the lanes whose key may repeat) as if
+// its edges came one after another: a key in the table gains one, else it
+// takes a free slot with one, else (full) every slot drops by one, emptied
+// slots are freed and the key is dropped.  (Which free slot a key takes does
+// not matter: the winner is a maximum over the table.  Every count is >= 1
+// and every frequency 1, so frequent and buffer agree.)
+// Between two changes of the key set hits only add up, so the chunk is
+// applied event by event instead of edge by edge.  An entry is a table slot
+// (lane i: K, A) or, entered in this chunk, its first edge's lane (key, An);
+// mo and mn are the lane's masks of the chunk's later edges with its key, so
+// an entry's count at edge p is A + (mask bits below p) - off.  `miss` holds
+// the edges not yet applied whose key has no entry:
+//  * with free slots the first misses enter, all at once while their keys
+//    occur once in the chunk (`run`), else one at a time, its later edges
+//    becoming hits;
+//  * full, the next miss drops every entry (off + 1) and frees the emptied
+//    ones, whose later edges miss again; if it empties none, no miss before
+//    the cmin-th can (cmin the smallest count), so those are skipped;
+//  * a run that fills the f free slots loses those entries again to its next
+//    miss, f + 1 misses a turn, as long as no older entry empties: such turns
+//    are skipped together.
+// While labels are diverse a chunk takes about three events; one edge at a
+// time it took 64 ballots, each followed by a dependent update.  The chain
+// of events of the largest hub sets the step: latency bound, one wavefront.
+__device__ __forceinline__ void table_chunk(uint32_t key, uint64_t all, uint64_t dup, int32_t cap, WideTable& t,
+                                            uint32_t* lds) {
+    const int lane = lane_id();
+    uint32_t mo_lo = 0u, mo_hi = 0u, mn_lo = 0u, mn_hi = 0u, An = 0u;
+    const uint64_t slots = cap == 64 ? ~0ull : (1ull << cap) - 1ull;
+    uint64_t live_o = slots & ~t.fr, live_n = 0ull;
+    const int top = live_o ? 64 - (int)__builtin_clzll(live_o) : 0;  // past the highest slot in use
+    int at = -1;  // the slot holding this edge's key
+    for (int s = 0; s < top; s += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            // a free slot's key is 0, lanes without a slot hold 0xffffffff: no edge carries either
+            at = key == (uint32_t)__builtin_amdgcn_readlane((int)t.K, s + u) ? s + u : at;
+        }
+    }
+    const uint64_t hit = __ballot(at >= 0);
+    if (hit) {
+        lds[lane] = 0u;
+        lds[64 + lane] = 0u;
+        wave_lds_sync();
+        if (at >= 0) atomicOr(&lds[at + (lane & 32 ? 64 : 0)], 1u << (lane & 31));
+        wave_lds_sync();
+        mo_lo = lds[lane];
+        mo_hi = lds[64 + lane];
+        wave_lds_sync();
+    }
+    uint64_t miss = all & ~hit;
+    uint32_t off = t.off, nfree = (uint32_t)__popcll(t.fr);
+    while (miss) {  // every pass applies at least the first miss
+        if (nfree) {
+            const uint64_t low = miss & (0ull - miss);
+            if (dup & low) {
+                const int p = (int)__builtin_ctzll(miss);
+                const uint32_t kk = (uint32_t)__builtin_amdgcn_readlane((int)key, p);
+                const uint64_t m = __ballot(key == kk) & (0ull - low);  // from p on
+                const uint64_t later = m & ~low;
+                const bool mine = lane == p;
+                An = mine ? off + 1u : An;
+                mn_lo = mine ? (uint32_t)later : mn_lo;
+                mn_hi = mine ? (uint32_t)(later >> 32) : mn_hi;
+                live_n |= low;
+                miss &= ~m;
+                --nfree;
+            } else {
+                // the misses before the first whose key may repeat
+                const uint64_t d = miss & dup;
+                uint64_t run = miss & ((d & (0ull - d)) - 1ull);  // d = 0: all of them
+                uint32_t n = (uint32_t)__popcll(run);
+                if (n > nfree) {
+                    const uint32_t r = rank_below(run);
+                    uint32_t skip = 0u;
+                    if (live_n == 0ull) {
+                        uint32_t turns = 0u, left = n;
+                        for (; left > nfree; left -= nfree + 1u) ++turns;
+                        if ((__ballot(t.A <= off + turns) & live_o) == 0ull) {
+                            skip = n - left;
+                            n = left;
+                            off += turns;
+                        }
+                    }
+                    const uint64_t gone = run & __ballot(r < skip);
+                    run = run & ~gone & __ballot(r < skip + nfree);
+                    miss &= ~gone;
+                    n = min(n, nfree);
+                }
+                const bool mine = __builtin_amdgcn_inverse_ballot_w64(run);
+                An = mine ? off + 1u : An;
+                mn_lo = mine ? 0u : mn_lo;
+                mn_hi = mine ? 0u : mn_hi;
+                live_n |= run;
+                miss &= ~run;
+                nfree -= n;
+            }
+            if (nfree || miss == 0ull) continue;
+        }
+        const uint64_t low = miss & (0ull - miss), below = low - 1ull;
+        const uint32_t b_lo = (uint32_t)below, b_hi = (uint32_t)(below >> 32);
+        const uint32_t co = t.A + (uint32_t)(__popc(mo_lo & b_lo) + __popc(mo_hi & b_hi));
+        const uint32_t cn = An + (uint32_t)(__popc(mn_lo & b_lo) + __popc(mn_hi & b_hi));
+        const uint64_t dead_o = __ballot(co == off + 1u) & live_o;
+        const uint64_t dead_n = __ballot(cn == off + 1u) & live_n;
+        if ((dead_o | dead_n) == 0ull) {
+            const uint32_t lo_o = __builtin_amdgcn_inverse_ballot_w64(live_o) ? co : 0xffffffffu;
+            const uint32_t lo_n = __builtin_amdgcn_inverse_ballot_w64(live_n) ? cn : 0xffffffffu;
+            const uint32_t cmin = wave_min_dpp(min(lo_o, lo_n)) - off;  // >= 2
+            const uint32_t skip = min(cmin - 1u, (uint32_t)__popcll(miss));
+            for (uint32_t k = 0u; k < skip; ++k) miss &= miss - 1ull;
+            off += skip;
+            continue;
+        }
+        ++off;
+        miss &= ~low;
+        const uint64_t after = ~(below | low);  // the edges past this miss
+        const uint32_t a_lo = (uint32_t)after, a_hi = (uint32_t)(after >> 32);
+        const bool d_o = __builtin_amdgcn_inverse_ballot_w64(dead_o), d_n = __builtin_amdgcn_inverse_ballot_w64(dead_n);
+        const uint32_t back_lo = ((d_o ? mo_lo : 0u) | (d_n ? mn_lo : 0u)) & a_lo;
+        const uint32_t back_hi = ((d_o ? mo_hi : 0u) | (d_n ? mn_hi : 0u)) & a_hi;
+        for (uint64_t q = __ballot((back_lo | back_hi) != 0u); q; q &= q - 1ull)
+            miss |= readlane_u64(back_lo, back_hi, (int)__builtin_ctzll(q));
+        live_o &= ~dead_o;
+        live_n &= ~dead_n;
+        nfree = (uint32_t)(__popcll(dead_o) + __popcll(dead_n));
+    }
+    t.off = off;
+    t.A += (uint32_t)(__popc(mo_lo) + __popc(mo_hi));  // 0 for lanes without a slot
+    t.fr = slots & ~live_o;
+    if (__builtin_amdgcn_inverse_ballot_w64(t.fr)) t.K = 0u;
+    if (live_n) {  // this chunk's entries move to free slots
+        const uint32_t cnt = (uint32_t)__popcll(live_n);
+        uint32_t* ks = lds;
+        uint32_t* as = lds + 64;
+        if (__builtin_amdgcn_inverse_ballot_w64(live_n)) {
+            const uint32_t r = rank_below(live_n);
+            ks[r] = key;
+            as[r] = An + (uint32_t)(__popc(mn_lo) + __popc(mn_hi));
+        }
+        wave_lds_sync();
+        const uint32_t r = rank_below(t.fr);
+        const bool takes = __builtin_amdgcn_inverse_ballot_w64(t.fr) && r < cnt;
+        if (takes) {
+            t.K = ks[r];
+            t.A = as[r];
+        }
+        t.fr &= ~__ballot(takes);
+        wave_lds_sync();
+    }
+}
+
+// Applies one weighted edge: a key in the table gains the frequency, else it
+// takes the lowest free slot, else (full) every counter drops and emptied
+// slots are freed.  Buffer drops by min(counter, frequency) and the key is
+// dropped; frequent drops by d = min(frequency, smallest counter) and what is
+// left of the frequency enters the first freed slot.
+template <bool BUF>
+__device__ __forceinline__ void table_edge(uint32_t kk, uint32_t ff, WideTable& t) {
+    const uint64_t hm = __ballot(t.K == kk);
+    if (hm) {
+        t.A += __builtin_amdgcn_inverse_ballot_w64(hm) ? ff : 0u;
+        return;
+    }
+    if (t.fr) {
+        const uint64_t low = t.fr & (0ull - t.fr);
+        const bool mine = __builtin_amdgcn_inverse_ballot_w64(low);
+        t.K = mine ? kk : t.K;
+        t.A = mine ? t.off + ff : t.A;
+        t.fr ^= low;
+        return;
+    }
+    const uint32_t to = t.off + ff;
+    const uint64_t gone = __ballot(t.A <= to);
+    if (gone == 0ull) {
+        t.off = to;
+        return;
+    }
+    if constexpr (BUF) {
+        t.off = to;
+        t.fr = gone;
+        t.K = __builtin_amdgcn_inverse_ballot_w64(gone) ? 0u : t.K;
+    } else {
+        const uint32_t least = wave_min_dpp(t.A);  // off + the smallest counter
+        const uint32_t left = ff - (least - t.off);
+        t.off = least;
+        t.fr = __ballot(t.A == least);
+        t.K = __builtin_amdgcn_inverse_ballot_w64(t.fr) ? 0u : t.K;
+        if (left) {
+            const uint64_t low = t.fr & (0ull - t.fr);
+            const bool mine = __builtin_amdgcn_inverse_ballot_w64(low);
+            t.K = mine ? kk : t.K;
+            t.A = mine ? t.off + left : t.A;
+            t.fr ^= low;
+        }
+    }
+}
+
+// Applies the edges [b, e) (e > b) of a vertex to its table.  Edges come in
+// chunks of 64, one per lane, applied at once where table_bulk can, else by
+// table_chunk (weighted: edge by edge); the bulk form is tried after it
+// worked and on every fourth chunk, so that diverse labels, where it does
+// not, pay little for it.  B chunks' loads are issued together, a block
+// ahead (the neighbour ids two blocks ahead): a chunk applied at once takes
+// less time than its loads.  Lanes past the last edge load the last edge
+// again (in bounds, never applied), so the loads need no branches and stay in
+// flight across the block.
+template <bool W, bool BUF, int B>
+__device__ __forceinline__ void table_run(const StepArgs& a, int32_t b, int32_t e, int32_t cap, WideTable& t,
+                                          TableLds& lds) {
+    const int lane = lane_id();
+    uint32_t* words = &lds.bits[0][0][0];  // scratch of one chunk
+    const int32_t last = e - 1;
+    // this lane's edge of chunk u of the block at j (an int64 j: the blocks
+    // loaded ahead may lie past 2^31)
+    auto edge = [&](int64_t j, int u) { return (int32_t)min(j + 64 * u + lane, (int64_t)last); };
+    bool calm = false;  // the last chunk was applied at once
+    uint32_t chunk = 0u;
+    int32_t id[B];
+    uint32_t lab[B], f[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) id[u] = a.nbr[edge(b, u)];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        lab[u] = (uint32_t)a.L[id[u]];
+        f[u] = W ? a.w[edge(b, u)] : 1u;
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u) id[u] = a.nbr[edge((int64_t)b + 64 * B, u)];
+    for (int64_t j0 = b; j0 < e; j0 += 64 * B) {
+        const int64_t j1 = j0 + 64 * B, j2 = j1 + 64 * B;
+        uint32_t nlab[B], nf[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            nlab[u] = (uint32_t)a.L[id[u]];
+            nf[u] = W ? a.w[edge(j1, u)] : 1u;
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) id[u] = a.nbr[edge(j2, u)];
+        uint32_t key[B];
+        uint64_t dup[B] = {};
+        bool have = false;  // dup is known
+#pragma unroll
+        for (int u = 0; u < B; ++u) key[u] = j0 + 64 * u + lane < e ? lab[u] + 1u : kNoEdge;
+        // one chunk's code for all of them: the block's registers rotate
+#pragma unroll 1
+        for (int u = 0; u < B; ++u) {
+            const int32_t cnt = (int32_t)min((int64_t)64, (int64_t)e - j0 - 64 * u);
+            if (cnt <= 0) break;
+            const uint64_t all = cnt == 64 ? ~0ull : (1ull << cnt) - 1ull;
+            calm = (calm || chunk++ % 4u == 3u) && table_bulk<W>(key[0], f[0], all, cap, t, words);
+            if (!calm) {
+                if constexpr (W) {
+                    auto apply = [&](int k) {
+                        table_edge<BUF>((uint32_t)__builtin_amdgcn_readlane((int)key[0], k),
+                                        (uint32_t)__builtin_amdgcn_readlane((int)f[0], k), t);
+                    };
+                    if (cnt == 64) {
+#pragma unroll 64
+                        for (int k = 0; k < 64; ++k) apply(k);
+                    } else {
+                        for (int k = 0; k < cnt; ++k) apply(k);
+                    }
+                } else {
+                    if (!have) table_repeats<B>(key, dup, lds);
+                    have = true;
+                    table_chunk(key[0], all, dup[0], cap, t, words);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k + 1 < B; ++k) {
+                key[k] = key[k + 1];
+                f[k] = f[k + 1];
+                dup[k] = dup[k + 1];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            lab[u] = nlab[u];
+            f[u] = nf[u];
+        }
+    }
+}
+
+// One wavefront per vertex of `verts` (degrees above kTableLaneMaxDeg), its
+// table a WideTable; the vertex and its edge range are wave-uniform (scalar
+// loop control).  Up to kTableShort edges the loads of four chunks at a time
+// would mostly be clamped ones (planted graph of 100,000 vertices of degree
+// 48, 4 steps: 0.95 ms, with one chunk at a time 0.59).  The chain of edges
+// of the largest hub sets the step, not bandwidth: R-MAT scale 21, 16 slots,
+// 3 steps from L0, 20.4 ms with every edge applied on its own (64 ns an
+// edge), 8.0 ms with table_chunk (22 ns); weighted at scale 20 (frequent)
+// 23.9 -> 17.7 ms with the offset in place of a drop per slot and the chunk
+// unrolled.
+constexpr int32_t kTableShort = 256;
 template <bool W, bool BUF>
 __global__ __launch_bounds__(256) void k_table_wave(StepArgs a, const int32_t* __restrict__ verts, int32_t nv,
                                                     int32_t cap) {
+    __shared__ TableLds s_lds[4];
     const int lane = lane_id();
     const int32_t i = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (i >= nv) return;  // wave-uniform
@@ -440,82 +819,11 @@ __global__ __launch_bounds__(256) void k_table_wave(StepArgs a, const int32_t* _
     const int32_t b = __builtin_amdgcn_readfirstlane(a.off[v]);
     const int32_t e = __builtin_amdgcn_readfirstlane(a.off[v + 1]);
     const bool slot = lane < cap;
-    const uint64_t slots = __ballot(slot);
-    uint32_t K = slot ? 0u : 0xffffffffu, C = 0u;
-    const int32_t last = e - 1;  // e > b: these vertices have more than 32 edges
-    int32_t jn = b + lane;
-    int32_t id = a.nbr[min(jn, last)];
-    uint32_t lab = (uint32_t)a.L[id];
-    uint32_t f = W ? a.w[min(jn, last)] : 1u;
-    jn += 64;
-    id = a.nbr[min(jn, last)];
-    for (int32_t j0 = b; j0 < e; j0 += 64) {
-        const uint32_t nlab = (uint32_t)a.L[id];
-        const uint32_t nf = W ? a.w[min(jn, last)] : 1u;
-        jn += 64;
-        id = a.nbr[min(jn, last)];
-        const int32_t cnt = __builtin_amdgcn_readfirstlane(min(64, e - j0));  // held in a scalar register
-        if constexpr (!W) {
-            // Unweighted, without branches: the key's slot (the one holding
-            // it, else the lowest free one) gains one and holds it, else
-            // (full) every slot drops by one and the emptied ones are freed.
-            // Frequent and buffer agree here (every count >= 1, frequency 1).
-            // The two slot sets are wave-uniform masks, read back per lane.
-            // A full chunk runs unrolled (no loop control per edge).
-            const uint32_t key = lab + 1u;
-            auto apply = [&](uint32_t kk) {
-                const uint64_t hm = __ballot(K == kk), fm = __ballot(K == 0u);
-                const uint64_t upm = hm ? hm : fm & (0ull - fm);
-                const uint64_t dnm = hm | fm ? 0ull : slots;
-                const bool up = __builtin_amdgcn_inverse_ballot_w64(upm);
-                const bool dn = __builtin_amdgcn_inverse_ballot_w64(dnm);
-                C = C + (uint32_t)up - (uint32_t)dn;
-                K = up ? kk : K;
-                K = dn && C == 0u ? 0u : K;
-            };
-            if (cnt == 64) {
-#pragma unroll
-                for (int k = 0; k < 64; ++k) apply((uint32_t)__builtin_amdgcn_readlane((int)key, k));
-            } else {
-                for (int32_t k = 0; k < cnt; ++k) apply((uint32_t)__builtin_amdgcn_readlane((int)key, k));
-            }
-        } else {
-            for (int32_t k = 0; k < cnt; ++k) {
-                const uint32_t kk = (uint32_t)__builtin_amdgcn_readlane((int)lab, k) + 1u;
-                const uint32_t ff = (uint32_t)__builtin_amdgcn_readlane((int)f, k);
-                const bool hit = K == kk;
-                if (__ballot(hit)) {  // present: it gains the frequency
-                    if (hit) C += ff;
-                    continue;
-                }
-                const uint64_t fr = __ballot(K == 0u);
-                if (fr) {  // the first free slot takes it
-                    if (lane == __builtin_ctzll(fr)) {
-                        K = kk;
-                        C = ff;
-                    }
-                    continue;
-                }
-                // full: every counter drops (buffer: by the frequency;
-                // frequent: by min(frequency, smallest counter)), emptied
-                // slots are freed
-                uint32_t d = ff;
-                if (!BUF) d = min(ff, wave_min_dpp(slot ? C : 0xffffffffu));
-                if (slot) C = BUF ? (C > ff ? C - ff : 0u) : C - d;
-                const bool emptied = slot && C == 0u;
-                if (emptied) K = 0u;
-                if (!BUF && ff > d) {  // frequent: what is left enters the first freed slot
-                    if (lane == __builtin_ctzll(__ballot(emptied))) {
-                        K = kk;
-                        C = ff - d;
-                    }
-                }
-            }
-        }
-        lab = nlab;
-        f = nf;
-    }
-    const uint64_t best = wave_max_u64(slot && K ? pack_score((int32_t)min(C, 0x7fffffffu), K) : 0ull);
+    WideTable t{slot ? 0u : 0xffffffffu, slot ? 0u : 0xffffffffu, 0u, __ballot(slot)};
+    TableLds& lds = s_lds[threadIdx.x >> 6];
+    if (e - b <= kTableShort) table_run<W, BUF, 1>(a, b, e, cap, t, lds);
+    else table_run<W, BUF, kTableBlk>(a, b, e, cap, t, lds);
+    const uint64_t best = wave_max_u64(slot && t.K ? pack_score((int32_t)(t.A - t.off), t.K) : 0ull);
     if (lane == 0) {
         const int32_t old = a.keep[v];
         const int32_t nl = best ? packed_label(best) : old;

@@ -322,6 +322,33 @@ def test_tables_weighted(rmat13w, cap):
         assert np.array_equal(labels, prev)
 
 
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("cap", [1, 2, 7, 16, 33, 64])
+def test_tables_apply_chunks_in_order(cap, weighted):
+    """Neighbour lists in random order with repeats, from alphabets around the
+    table's capacity (slots empty and refill all the time) to far above it, at
+    degrees around the chunk and block lengths of the wide tables."""
+    rng = np.random.default_rng(cap)
+    n, nbrs, deg = 700, [], []
+    for d in (33, 63, 64, 65, 128, 129, 255, 256, 257, 320, 513, 2000):
+        for alphabet in (1, 2, cap, cap + 1, 2 * cap, 600):
+            p = rng.random(alphabet) ** 4
+            x = rng.choice(alphabet, size=d, p=p / p.sum()) if rng.random() < 0.7 else np.arange(d) // 2 % alphabet
+            nbrs.append(x.astype(np.int32))
+            deg.append(d)
+    deg += [0] * (n - len(deg))
+    off = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    nbr = np.concatenate(nbrs)
+    w = rng.choice([1, 1, 2, 5, 40], size=len(nbr)).astype(np.uint32) if weighted else None
+    g = G.Graph.from_csr(off, nbr, w)
+    for method, buf in ((G.FREQUENT, 0), (G.BUFFER, 1)):
+        _, dump, _ = G.run(g, 3, dump=True, method=method, table_cap=cap, weighted=weighted)
+        prev = np.arange(n, dtype=np.int32)
+        for t in range(3):
+            prev = O.table_step(off, nbr, prev, cap, buf, w=w)
+            assert np.array_equal(dump[t], prev), "step %d" % (t + 1)
+
+
 # --------------------------------------------------------------- user hooks ----
 
 def test_user_hooks_are_classic(rmat14):

@@ -71,6 +71,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
         dg->off = base->off;
         dg->nbr = base->nbr;
         dg->w = base->w;
+        dg->ascending = base->ascending;
         dg->owns_csr = false;
         int r = device_plan_upload(dg.get(), stream);
         if (r != GLP_OK) return r;
@@ -123,6 +124,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
         dg->off = base->off;
         dg->nbr = base->nbr;
         dg->w = base->w;
+        dg->ascending = base->ascending;
         if ((rc = device_plan_upload(dg.get(), stream)) != GLP_OK) return rc;
         dg->owns_csr = true;
         base->owns_csr = false;

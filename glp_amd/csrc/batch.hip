@@ -88,8 +88,12 @@ extern "C" int glp_batch_create(int32_t ngraphs, glp_graph* const* graphs, const
     }
     u.finish();
     // a disjoint union is symmetric when every part is
-    u.symmetric = 1;
-    for (int32_t i = 0; i < ngraphs; ++i) u.symmetric = std::min(u.symmetric, graphs[i]->csr.symmetric);
+    // (and its lists ascend when every part's do)
+    u.symmetric = u.ascending = 1;
+    for (int32_t i = 0; i < ngraphs; ++i) {
+        u.symmetric = std::min(u.symmetric, graphs[i]->csr.symmetric);
+        u.ascending = std::min(u.ascending, graphs[i]->csr.ascending);
+    }
     int rc = session_create(b->uni.get(), p, &b->sess);
     if (rc != GLP_OK) return rc;
     *out = b.release();

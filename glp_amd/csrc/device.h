@@ -98,6 +98,7 @@ struct DeviceGraph {
     InverseIndex inv;
     double upload_ms = 0, plan_ms = 0;
     size_t bytes = 0;
+    bool ascending = false;  // every neighbour list is strictly ascending (no repeats)
     bool owns_csr = true;   // false: off/nbr/w borrowed from another DeviceGraph
     bool owns_plan = true;  // false: the d_* plan arrays live in memory the graph does not own
     ~DeviceGraph();
@@ -186,8 +187,9 @@ struct JobDesc {
 };
 
 // LayeredVol: layered LP with gamma > 0 scored in the table slots from the
-// (label, volume) records of StepArgs::LV (LayeredVolHooks).
-enum class Method { Classic, Layered, LayeredVol, Slpa, User, Seeded };
+// (label, volume) records of StepArgs::LV (LayeredVolHooks).  First: the step
+// from L_0 of classic, layered and SLPA LP (FirstHooks).
+enum class Method { Classic, Layered, LayeredVol, Slpa, User, Seeded, First };
 
 // One-time kernel attribute set-up (LDS limits); call before any capture.
 void init_kernels();
@@ -208,6 +210,9 @@ int inverse_index_build(const int32_t* nbr, int32_t n, int64_t m, int32_t* curso
 // Most in-edges of changed sources for which a frontier gather pushes
 // (frontier control word 7); above it the gather rewrites every edge.
 int32_t push_edge_limit(int64_t m);
+// Whether every neighbour list of the device CSR is strictly ascending
+// (synchronises s).
+int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s, bool* yes);
 // Random-read calibration: `reads` 4-byte reads of T (entries a power of
 // two) at uniform hashed indices; out holds out_entries int32 sums.
 int launch_calib_read(const int32_t* T, int64_t entries, int64_t reads, uint32_t seed, int32_t* out,

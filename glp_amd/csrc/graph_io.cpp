@@ -243,9 +243,18 @@ extern "C" int glp_graph_from_csr(int32_t n, int64_t m, const int32_t* offsets,
         return set_error(GLP_E_FORMAT, "offsets must start at 0 and end at m");
     for (int32_t v = 0; v < n; ++v)
         if (offsets[v + 1] < offsets[v]) return set_error(GLP_E_FORMAT, "offsets not monotone at %d", v);
-    for (int64_t j = 0; j < m; ++j)
-        if (neighbors[j] < 0 || neighbors[j] >= n)
-            return set_error(GLP_E_FORMAT, "neighbor %d at %lld out of range", neighbors[j], (long long)j);
+    int64_t descents = 0;  // edges not above the one before them
+    int32_t before = -1;
+    for (int64_t j = 0; j < m; ++j) {
+        const int32_t u = neighbors[j];
+        if (u < 0 || u >= n) return set_error(GLP_E_FORMAT, "neighbor %d at %lld out of range", u, (long long)j);
+        descents += u <= before;
+        before = u;
+    }
+    for (int32_t v = 1; v < n; ++v) {  // those between two lists say nothing
+        const int64_t j = offsets[v];
+        if (offsets[v + 1] > j && j > 0) descents -= neighbors[j] <= neighbors[j - 1];
+    }
     auto g = std::make_unique<glp_graph>();
     g->csr.n = n;
     g->csr.m = m;
@@ -257,6 +266,7 @@ extern "C" int glp_graph_from_csr(int32_t n, int64_t m, const int32_t* offsets,
             if (w == 0) return set_error(GLP_E_FORMAT, "zero edge weight");
     }
     g->csr.finish();
+    g->csr.ascending = descents == 0 ? 1 : 0;
     *out = g.release();
     return GLP_OK;
 }
@@ -356,6 +366,7 @@ extern "C" int glp_graph_degree_sort(const glp_graph* g, glp_graph** out, int32_
     }
     d.finish();
     d.symmetric = c.symmetric;  // a relabelling keeps (a)symmetry
+    d.ascending = c.ascending == 1 ? 1 : -1;  // sorted lists; repeats would stay
     if (perm_out) std::memcpy(perm_out, perm.data(), sizeof(int32_t) * n);
     *out = ng.release();
     return GLP_OK;

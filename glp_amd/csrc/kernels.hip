@@ -180,6 +180,25 @@ __device__ __forceinline__ void count_edges(const StepArgs& a, int32_t v, int32_
     }
 }
 
+// Best packed score of an edge of [b, e) (first steps, whose labels all
+// differ), STRIDE threads cooperating, K edges' loads in flight per thread
+// (an index past the end is clamped to the last edge: counting it twice
+// changes no maximum).
+template <class H, bool W, bool G, int K, int STRIDE>
+__device__ __forceinline__ uint64_t best_edge(const StepArgs& a, int32_t v, int32_t b, int32_t e, int tid) {
+    uint64_t best = 0ull;
+    for (int64_t j0 = (int64_t)b + tid; j0 < e; j0 += STRIDE * K) {
+        uint32_t key[K], fr[K];
+        int32_t vol;
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+            key[i] = load_edge<H, W, G>(a, v, (int32_t)min(j0 + i * STRIDE, (int64_t)e - 1), &fr[i], &vol);
+#pragma unroll
+        for (int i = 0; i < K; ++i) best = max_u64(best, H::label_score(a, v, key[i], W ? fr[i] : 1u));
+    }
+    return best;
+}
+
 // Whether v sets its bit in the changed-vertex bitmap (frontier gather
 // only): its new label differs from the previous step's, or, with the
 // two-step lookahead, from the label of two steps back, which the buffer
@@ -355,7 +374,12 @@ __device__ __forceinline__ uint32_t packed_finish(const StepArgs& a, const Packe
     const bool live = lane < s.nE && s.key != 0u;
     uint64_t best = 0ull;  // on vertex lanes: the vertex's best packed score
     bool decided = false;  // the whole group was decided without the table
-    if constexpr (count_score_of<H>::value && !W) {
+    if (!W && labels_distinct<H>(a)) {
+        // every edge counts once: the highest label, the list's last, wins
+        const uint32_t top = shfl_u32(s.key, max(s.ve - 1, 0));
+        if (s.ve > s.vb) best = H::label_score(a, s.v0 + lane, top, 1u);
+        decided = true;
+    } else if constexpr (count_score_of<H>::value && !W) {
         // majority shortcut: a label on more than half of a vertex's counted
         // edges wins outright.  Candidates per vertex: the labels of its
         // first and of its last edge (one of them is the majority label
@@ -394,7 +418,10 @@ __device__ __forceinline__ uint32_t packed_finish(const StepArgs& a, const Packe
         wave_lds_sync();  // the clear, or the previous group's clears, are done
         uint32_t h = 0u;
         bool claimed = false;  // this lane created the (owner, label) slot
-        if (live) {
+        if (labels_distinct<H>(a)) {  // every edge is its label's only one
+            if (live)
+                atomicMax(&t.best[s.own], (unsigned long long)H::label_score(a, s.v0 + s.own, s.key, W ? s.fr : 1u));
+        } else if (live) {
             const unsigned long long k64 = ((unsigned long long)(uint32_t)(s.own + 1) << 32) | s.key;
             h = fmix32(s.key ^ ((uint32_t)s.own * 0x9e3779b9u)) & (kPackSlots - 1u);
             for (;;) {
@@ -551,7 +578,14 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
         // its score
         uint64_t fast = 0ull;
         bool peel = true;  // merge lanes of a shared label before the table
-        if constexpr (count_score_of<H>::value) {
+        if (labels_distinct<H>(a)) {
+            // every edge is its label's only one: the best edge wins
+#pragma unroll
+            for (int i = 0; i < EPL; ++i)
+                if (key[p][i]) fast = max_u64(fast, H::label_score(a, v[p], key[p][i], W ? fr[p][i] : 1u));
+#pragma unroll
+            for (int d = S / 2; d >= 1; d >>= 1) fast = max_u64(fast, shfl_u64(fast, lane ^ d));
+        } else if constexpr (count_score_of<H>::value) {
             const uint32_t lead = shfl_u32(key[p][0], g0);
             const uint32_t lead2 = shfl_u32(key[p][0], g0 + S / 2);
             uint32_t c = 0u, c2 = 0u, tot = 0u;
@@ -711,7 +745,14 @@ __device__ __forceinline__ void wave_body(const StepArgs& a, const int4* __restr
         uint64_t best = 0ull;
         bool decided = false;  // wave-uniform
         bool peel = true;      // merge lanes of a shared label before the table
-        if constexpr (count_score_of<H>::value) {
+        if (labels_distinct<H>(a)) {
+            // every edge is its label's only one: the best edge wins
+#pragma unroll
+            for (int i = 0; i < EPL; ++i)
+                if (key[k][i]) best = max_u64(best, H::label_score(a, v[k], key[k][i], W ? fr[k][i] : 1u));
+            best = wave_max_u64(best);
+            decided = true;
+        } else if constexpr (count_score_of<H>::value) {
             // majority shortcut: the label of the first edge, or of the
             // 33rd, wins outright when it holds more than half of the
             // counted frequency
@@ -813,12 +854,17 @@ __device__ __forceinline__ void block_body(const StepArgs& a, const int32_t* __r
     const int32_t b = a.off[v], e = a.off[v + 1];
     const uint32_t cap = min(max(next_pow2(2u * (uint32_t)(e - b)), 64u), cap_max);
     const uint32_t mask = cap - 1u;
-    for (uint32_t i = threadIdx.x; i < cap; i += NT) T[i] = 0ull;
-    __syncthreads();
-    constexpr bool S = slot_score_of<H>::value;
-    count_edges<H, W, G, K, NT, S>(a, v, b, e, threadIdx.x, T, mask);
-    __syncthreads();
-    uint64_t best = table_best<H, S>(a, v, T, cap, threadIdx.x, NT, false);
+    uint64_t best = 0ull;
+    if (labels_distinct<H>(a)) {  // uniform
+        best = best_edge<H, W, G, K, NT>(a, v, b, e, threadIdx.x);
+    } else {
+        for (uint32_t i = threadIdx.x; i < cap; i += NT) T[i] = 0ull;
+        __syncthreads();
+        constexpr bool S = slot_score_of<H>::value;
+        count_edges<H, W, G, K, NT, S>(a, v, b, e, threadIdx.x, T, mask);
+        __syncthreads();
+        best = table_best<H, S>(a, v, T, cap, threadIdx.x, NT, false);
+    }
     best = block_max_u64<NT>(best, s_red);
     if (threadIdx.x < 64) {
         bool changed = false;
@@ -932,6 +978,12 @@ __device__ __forceinline__ void hub_agg_body(const StepArgs& a, const HubArgs& h
     const int32_t e = min(b + h.chunk, ve);
     const uint32_t cap = min(max(next_pow2(2u * (uint32_t)(e - b)), 64u), cap_max);
     const uint32_t mask = cap - 1u;
+    if (labels_distinct<H>(a)) {  // uniform: no pairs to sum, k_hub_part is not launched
+        __shared__ unsigned long long s_red[NT / 64];
+        const uint64_t best = block_max_u64<NT>(best_edge<H, W, G, K, NT>(a, v, b, e, threadIdx.x), s_red);
+        if (threadIdx.x == 0) atomicMax(&h.hs.best[hc.x], (unsigned long long)best);
+        return;
+    }
     for (uint32_t i = threadIdx.x; i < cap; i += NT) T[i] = 0ull;
     for (uint32_t q = threadIdx.x; q < P; q += NT) s_hist[q] = 0u;
     __syncthreads();
@@ -1906,7 +1958,8 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
         if (ev) (void)hipEventRecord(ev[2 * tier + edge], s);
     };
     mark(GLP_TIER_PACKED, 0);
-    const int32_t ng = (int32_t)(H::kSkipIsolated ? p.groups_with_edges : (int64_t)p.groups.size());
+    const int32_t ng = (int32_t)(H::kSkipIsolated && !a.write_isolated ? p.groups_with_edges
+                                                                       : (int64_t)p.groups.size());
     if (p.tune.fused_small > 0 && hs.work) {
         // packed and half tiers in one persistent launch
         SmallTiers st;
@@ -2037,8 +2090,9 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
                            hub_agg_lds(h.chunk, p.hub_max_buckets), s, a, h);
         mark(GLP_TIER_HUB, 1);
         mark(GLP_TIER_AUX, 0);
-        hipLaunchKernelGGL((k_hub_part<H>), dim3((np + h.part_batch - 1) / h.part_batch), dim3(kHubThreads),
-                           lds_part, s, a, h);
+        if (!(first_of<H>::value && a.ascending))
+            hipLaunchKernelGGL((k_hub_part<H>), dim3((np + h.part_batch - 1) / h.part_batch), dim3(kHubThreads),
+                               lds_part, s, a, h);
         hipLaunchKernelGGL((k_hub_final<H>), dim3(grid_for(h.nhubs, 256)), dim3(256), 0, s, a, h);
         if (H::kFrontier && a.act_w)
             hipLaunchKernelGGL((k_hub_mark<H>), dim3(nc), dim3(256), 0, s, a, h);
@@ -2099,7 +2153,12 @@ void init_kernels() {
     GLP_SETLDS4(SlpaHooks)
     GLP_SETLDS4(UserHooks)
     GLP_SETLDS4(SeededHooks)
-    // slot-scored layered LP runs fused only (no gathered instantiation)
+    // first steps and slot-scored layered LP run fused only (no gathered instantiation)
+    GLP_SETLDS(FirstHooks, false, false)
+    GLP_SETLDS(FirstHooks, true, false)
+    GLP_SETLDS_HUB(FirstHooks, false, false)
+    GLP_SETLDS_HUB(FirstHooks, true, false)
+    (void)hipFuncSetAttribute((const void*)k_hub_part<FirstHooks>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
     GLP_SETLDS(LayeredVolHooks, false, false)
     GLP_SETLDS(LayeredVolHooks, true, false)
     GLP_SETLDS_HUB(LayeredVolHooks, false, false)
@@ -2131,6 +2190,10 @@ int launch_step(Method method, bool weighted, bool gathered, const DeviceGraph& 
                 const HubScratch& hs, const StepArgs& a, hipStream_t s, hipEvent_t* ev) {
     switch (method) {
         case Method::Classic: return launch_hooks<ClassicHooks>(weighted, gathered, g, hs, a, s, ev);
+        case Method::First:
+            if (gathered) return set_error(GLP_E_UNSUPPORTED, "first steps read the neighbour ids themselves");
+            return weighted ? launch_tiers<FirstHooks, true, false>(g, hs, a, s, ev)
+                            : launch_tiers<FirstHooks, false, false>(g, hs, a, s, ev);
         case Method::Layered: return launch_hooks<LayeredHooks>(weighted, gathered, g, hs, a, s, ev);
         case Method::LayeredVol:
             if (gathered || !a.LV)
@@ -2266,6 +2329,48 @@ int launch_iota(int32_t* p, int64_t count, hipStream_t s) {
     hipLaunchKernelGGL(k_iota, dim3(grid), dim3(256), 0, s, p, count);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "iota launch: %s", hipGetErrorString(e));
+}
+
+// Whether every neighbour list is strictly ascending: the positions j with
+// nbr[j] >= nbr[j + 1] (out[0]) must all be the last of their list (out[1]
+// counts those).  Two streaming passes, once per graph.
+__global__ __launch_bounds__(256) void k_descents(const int32_t* __restrict__ off, const int32_t* __restrict__ nbr,
+                                                  int32_t n, int64_t m, unsigned long long* __restrict__ out) {
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    uint32_t all = 0u, ends = 0u;
+    for (int64_t j = t0; j + 1 < m; j += stride) all += nbr[j] >= nbr[j + 1] ? 1u : 0u;
+    for (int64_t v = t0; v < n; v += stride) {
+        const int64_t e = off[v + 1];
+        if (e > off[v] && e < m) ends += nbr[e - 1] >= nbr[e] ? 1u : 0u;
+    }
+    all = wave_sum_u32(all);
+    ends = wave_sum_u32(ends);
+    if (lane_id() == 0) {
+        if (all) atomicAdd(&out[0], (unsigned long long)all);
+        if (ends) atomicAdd(&out[1], (unsigned long long)ends);
+    }
+}
+
+int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s, bool* yes) {
+    *yes = true;
+    if (m < 2) return GLP_OK;
+    unsigned long long* out = nullptr;
+    unsigned long long got[2] = {0, 0};
+    GLP_HIP(hipMalloc(&out, sizeof got));
+    int rc = launch_zero_bytes(out, sizeof got, s);
+    hipError_t e = hipSuccess;
+    if (!rc) {
+        const unsigned grid = (unsigned)std::min<int64_t>(grid_for(m, 256), 256 * 32);
+        hipLaunchKernelGGL(k_descents, dim3(grid), dim3(256), 0, s, off, nbr, n, m, out);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipMemcpyAsync(got, out, sizeof got, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) rc = set_error(GLP_E_HIP, "neighbour order check: %s", hipGetErrorString(e));
+    }
+    (void)hipFree(out);
+    *yes = got[0] == got[1];
+    return rc;
 }
 
 // Random 4-byte reads of a table with uniform fmix32 indices (the label

@@ -47,6 +47,7 @@ struct glp_session {
     int32_t* d_ctr = nullptr;              // device-side step counter
     int cur = 0;                           // index of the current label buffer
     int32_t t = 0;                         // steps enqueued
+    bool at_l0 = false;                    // the labels are L_0[v] = v: the next step can be a first step
     int32_t pending_steps = 0;
     size_t bytes = 0;                      // device bytes owned (graph excluded)
     std::vector<std::array<hipEvent_t, 2 * GLP_NTIERS>> ev_pool;  // profiled steps' events
@@ -70,7 +71,8 @@ int session_step(glp_session* s, int32_t steps);
 int session_step_graph(glp_session* s, int32_t steps);
 int session_sync(glp_session* s);
 int session_labels(glp_session* s, int32_t* out);
-int enqueue_step(glp_session* s, hipEvent_t* ev);
+// replayed: the step is being captured, to be replayed from any later state
+int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed = false);
 // count-min / frequent / buffer steps (counting.hip)
 int enqueue_counting_step(glp_session* s);
 int counting_wide_list(glp_session* s);

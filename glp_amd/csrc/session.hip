@@ -85,6 +85,8 @@ int device_graph_upload(const HostCSR& g, Plan&& plan, hipStream_t s, DeviceGrap
     if ((rc = upload(&dg->off, g.offsets.data(), (size_t)g.n + 1, s, bytes))) return rc;
     if ((rc = upload(&dg->nbr, g.neighbors.data(), (size_t)g.m, s, bytes))) return rc;
     if (g.weighted() && (rc = upload(&dg->w, g.weights.data(), (size_t)g.m, s, bytes))) return rc;
+    if (g.ascending >= 0) dg->ascending = g.ascending == 1;
+    else if ((rc = neighbours_ascending(dg->off, dg->nbr, g.n, g.m, s, &dg->ascending))) return rc;
     if ((rc = device_plan_upload(dg.get(), s))) return rc;
     double t2 = now_ms();
     dg->upload_ms = t2 - t1;
@@ -346,6 +348,8 @@ int session_reset(glp_session* s) {
     const int64_t n = s->n;
     s->cur = 0;
     s->t = 0;
+    s->at_l0 = s->method == Method::Layered || s->method == Method::Slpa ||
+               (s->method == Method::Classic && !counting_method(s->p.method));
     s->timing.steps = 0;
     s->timing.steps_ms = 0;
     for (int i = 0; i < GLP_NTIERS; ++i) {
@@ -449,7 +453,7 @@ static StepArgs step_args(glp_session* s) {
 }
 
 // Enqueues one step.  ev: per-tier events or null.
-int enqueue_step(glp_session* s, hipEvent_t* ev) {
+int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     if (counting_method(s->p.method)) return enqueue_counting_step(s);
     if (s->method == Method::Seeded && !s->seeds_set)
         return set_error(GLP_E_STATE, "a seeded session needs its seeds (glp_session_set_seeds)");
@@ -462,7 +466,14 @@ int enqueue_step(glp_session* s, hipEvent_t* ev) {
     // layered with gamma > 0: each neighbour's label travels with its
     // label's volume, and the tables accumulate scores (LayeredVolHooks)
     Method method = s->method;
-    if (s->method == Method::Layered && s->LV && s->p.gamma_num > 0) {
+    // from L_0 no label is gathered (the frontier gather counts on the adj
+    // its steps fill, so gather sessions keep their form)
+    const bool first = s->at_l0 && !replayed && !s->p.gather;
+    if (first) {
+        method = Method::First;
+        a.ascending = s->g->dev->ascending ? 1 : 0;
+        a.write_isolated = s->method == Method::Slpa ? 1 : 0;
+    } else if (s->method == Method::Layered && s->LV && s->p.gamma_num > 0) {
         method = Method::LayeredVol;
         a.LV = s->LV;
         if ((rc = launch_label_volumes(a.L, a.Vr, s->LV, s->n, s->stream))) return rc;
@@ -472,7 +483,7 @@ int enqueue_step(glp_session* s, hipEvent_t* ev) {
     // this step's changed-vertex bits start clear (they held two steps back)
     if (s->chg[0] && (rc = launch_zero_bytes(s->chg[s->cur ^ 1], s->chg_bytes, s->stream))) return rc;
     if (ev) (void)hipEventRecord(ev[2 * GLP_TIER_PICK], s->stream);
-    if (s->method == Method::Slpa || s->method == Method::User) {
+    if ((s->method == Method::Slpa && !first) || s->method == Method::User) {
         if ((rc = launch_pick(s->method, a, s->shown, s->stream))) return rc;
     }
     if (ev) (void)hipEventRecord(ev[2 * GLP_TIER_PICK + 1], s->stream);
@@ -490,6 +501,7 @@ int enqueue_step(glp_session* s, hipEvent_t* ev) {
     if ((rc = launch_end_step(s->d_acc, s->d_ring, s->d_ctr, kChangeRing, s->stream, s->fctl))) return rc;
     if (s->method != Method::Slpa) s->cur ^= 1;
     s->t += 1;
+    if (!replayed) s->at_l0 = false;
     return GLP_OK;
 }
 
@@ -557,7 +569,7 @@ int session_step_graph(glp_session* s, int32_t steps) {
         const int save_cur = s->cur, save_t = s->t;
         s->cur = parity;
         GLP_HIP(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-        int rc = enqueue_step(s, nullptr);
+        int rc = enqueue_step(s, nullptr, true);
         hipGraph_t graph = nullptr;
         hipError_t e = hipStreamEndCapture(s->stream, &graph);
         s->cur = save_cur;
@@ -572,7 +584,13 @@ int session_step_graph(glp_session* s, int32_t steps) {
         if (e != hipSuccess) return set_error(GLP_E_HIP, "instantiate: %s", hipGetErrorString(e));
     }
     if (s->pending_steps == 0) GLP_HIP(hipEventRecord(s->ev_start, s->stream));
-    for (int32_t i = 0; i < steps; ++i) {
+    int32_t i = 0;
+    if (s->at_l0) {  // the first step has launches of its own
+        int rc = enqueue_step(s, nullptr);
+        if (rc != GLP_OK) return rc;
+        i = 1;
+    }
+    for (; i < steps; ++i) {
         GLP_HIP(hipGraphLaunch(s->graph_exec[s->cur], s->stream));
         s->cur ^= 1;
         s->t += 1;
@@ -815,6 +833,7 @@ extern "C" int glp_session_load(glp_session* s, const void* state, size_t state_
     }
     s->cur = 0;
     s->t = h.t;
+    s->at_l0 = false;  // the labels are the caller's
     GLP_HIP(hipMemcpy(s->d_ctr, &h.t, 4, hipMemcpyHostToDevice));
     return GLP_OK;
 }

@@ -317,3 +317,64 @@ def test_profile_mode_matches():
     labels, t = G.run(g, 3, profile=True)
     assert np.array_equal(labels, O.classic(off, nbr, 3)[-1])
     assert t["tier_launches"]["packed"] == 3
+
+
+@pytest.mark.parametrize("order", ["ascending", "one_swap", "descending", "repeats"])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_first_step_by_neighbour_order(order, weighted):
+    """The step from L0 gathers no labels, and with strictly ascending lists
+    needs no tables: every tier of a graph whose lists ascend, one with a
+    single pair swapped, one descending and one with repeated neighbours, for
+    each method with such a step, eager and replayed, and a restored state of
+    step 0 whose labels are not L0."""
+    g = G.Graph.rmat(13, 16, seed=5, wmax=8)
+    off, nbr, w = g.csr()
+    nbr = nbr.copy()
+    if order == "one_swap":
+        v = int(np.flatnonzero(np.diff(off) > 300)[-1])
+        nbr[off[v + 1] - 2:off[v + 1]] = nbr[off[v + 1] - 2:off[v + 1]][::-1].copy()
+    elif order == "descending":
+        for v in range(len(off) - 1):
+            nbr[off[v]:off[v + 1]] = nbr[off[v]:off[v + 1]][::-1].copy()
+    elif order == "repeats":
+        for v in range(0, len(off) - 1, 3):
+            if off[v + 1] - off[v] >= 2:
+                nbr[off[v + 1] - 1] = nbr[off[v + 1] - 2]
+    ww = w if weighted else None
+    with G.tuning(block_max_deg=512, hub_chunk=256, part_keys=256):
+        g = G.Graph.from_csr(off, nbr, w)
+        want = O.classic(off, nbr, 3, w=ww)
+        assert_steps_equal(gpu_steps(g, 3, weighted=weighted), want)
+        for gamma in ((0, 1), (1, 4)):
+            assert_steps_equal(gpu_steps(g, 3, method=G.LAYERED, gamma=gamma, weighted=weighted),
+                               O.layered(off, nbr, 3, gamma[0], gamma[1], w=ww)[0])
+        with G.Session(g, method=G.SLPA, slpa_T=3, weighted=weighted) as s:
+            s.step(3)
+            assert np.array_equal(s.slpa_memory(4), O.slpa(off, nbr, 1, 3, w=ww))
+        with G.Session(g, weighted=weighted) as s:
+            s.step(3, graph=True)
+            assert np.array_equal(s.labels(), want[2])
+            s.reset()
+            s.step(2, graph=True)
+            assert np.array_equal(s.labels(), want[1])
+            s.reset()
+            state = bytearray(s.save())
+            lab = np.random.default_rng(1).integers(0, len(off) - 1, len(off) - 1).astype(np.int32)
+            state[-4 * len(lab):] = lab.tobytes()
+            s.load(bytes(state))
+            s.step(1)
+            assert np.array_equal(s.labels(), O.classic_step(off, nbr, lab, ww))
+
+
+def test_first_step_of_a_loaded_file(tmp_path):
+    """A .bin graph's lists are in file order with repeats: the order is
+    checked on the device copy."""
+    rng = np.random.default_rng(3)
+    pairs = rng.integers(0, 300, (3000, 2)).astype(np.int32)
+    pairs.tofile(tmp_path / "g.bin")
+    chain = np.stack([np.arange(299), np.arange(1, 300)], 1).astype(np.int32)  # ascending lists
+    chain.tofile(tmp_path / "c.bin")
+    for name in ("g.bin", "c.bin"):
+        g = G.Graph.load_bin(str(tmp_path / name))
+        off, nbr, _ = g.csr()
+        assert_steps_equal(gpu_steps(g, 3), O.classic(off, nbr, 3))

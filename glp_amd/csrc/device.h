@@ -233,8 +233,19 @@ int launch_label_volumes(const int32_t* L, const int32_t* V, int2* LV, int32_t n
 int launch_volume(const int32_t* L, int32_t* V, int32_t n, hipStream_t s);
 // p[i] = seeds[i] ? i : -1 (seeded LP's initial labels).
 int launch_seed_labels(int32_t* p, const uint8_t* seeds, int64_t count, hipStream_t s);
+// dom_ctl (may be null): chooses the next step's dominant label from the
+// labels dom_L over the m > 0 edges of dom_nbr, {1 when there is none, 0, it}.
 int launch_end_step(unsigned long long* acc, unsigned long long* ring, int32_t* step_ctr,
-                    int32_t ring_size, hipStream_t s, int32_t* fctl = nullptr);
+                    int32_t ring_size, hipStream_t s, int32_t* fctl = nullptr, const int32_t* dom_nbr = nullptr,
+                    const int32_t* dom_L = nullptr, int64_t dom_m = 0, int32_t* dom_ctl = nullptr);
+// Settles the vertices that a.fctl's dominant label decides (unweighted
+// classic counting on the labels a.L; nothing without such a label): writes
+// their labels and act[v] = 0, act[v] = 1 for the others with edges.  bits
+// (dominant_bytes(n) + dominant_bytes(n / 64 + 1)) and ebits
+// (dominant_bytes(m)) are scratch.
+int launch_dominant(const DeviceGraph& g, const StepArgs& a, uint32_t* bits, uint32_t* ebits, uint8_t* act,
+                    hipStream_t s);
+inline size_t dominant_bytes(int64_t count) { return ((size_t)count + 63) / 64 * 8; }
 // Fills count bytes (count a multiple of 4, p 4-byte aligned) with zero.
 inline int launch_zero_bytes(void* p, int64_t count, hipStream_t s) {
     return launch_fill_i32(static_cast<int32_t*>(p), 0, count / 4, s);

@@ -42,7 +42,9 @@ struct StepArgs {
     int32_t t;               // step number (1-based)
     const int32_t* mem;      // SLPA memory, (T+1) x n
     uint64_t seed;           // SLPA stream seed
-    // frontier (classic only; null when off): act_r[v] = some neighbour of v
+    // vertices to recompute (null: all of them).  With a dominant label:
+    // act_r[v] = 0 for the vertices it decides, fctl[0] = 0 in steps with one.
+    // Frontier (classic only): act_r[v] = some neighbour of v
     // changed in the previous step; act_w collects that for the next step;
     // fctl[0] = 1: this step recomputes every vertex, fctl[1] = 1: this step
     // marks act_w (both set on the device by k_end_step)

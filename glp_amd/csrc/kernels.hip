@@ -294,6 +294,7 @@ struct PackedGroup {
     int32_t v0, vc, base, ve, vb, nE, own, old;
     uint32_t key, fr;
     int32_t vol;  // the label's volume (slot-scoring hook sets)
+    bool act;     // vertex lanes: the vertex is recomputed
 };
 
 // Per-wave LDS of the packed count.
@@ -331,6 +332,7 @@ __device__ __forceinline__ void packed_load_fast(const StepArgs& a, int2 gr, Pac
     const int32_t end = a.off[s.v0 + li + 1];
     s.old = a.keep[s.v0 + li];
     s.ve = lane < s.vc ? end - s.base : 0;
+    s.act = true;
     packed_segments(s, lane);
     s.key = load_edge<H, W, G>(a, s.v0 + s.own, s.base + min(lane, s.nE - 1), &s.fr, &s.vol);
     if (lane >= s.nE) {
@@ -345,9 +347,10 @@ __device__ __forceinline__ bool packed_load_safe(const StepArgs& a, int2 gr, Pac
     const int lane = lane_id();
     s.v0 = gr.x;
     s.vc = gr.y;
+    s.act = true;
     if (frontier_on<H>(a)) {
-        const bool act = lane < s.vc && a.act_r[s.v0 + lane] != 0;
-        if (__ballot(act) == 0ull) return false;  // no vertex of the group needs work
+        s.act = lane < s.vc && a.act_r[s.v0 + lane] != 0;
+        if (__ballot(s.act) == 0ull) return false;  // no vertex of the group needs work
     }
     s.base = a.off[s.v0];
     s.ve = 0;
@@ -458,7 +461,7 @@ __device__ __forceinline__ uint32_t packed_finish(const StepArgs& a, const Packe
         t.best[lane] = 0ull;
     }
     bool changed = false, gch = false;
-    if (lane < s.vc && !is_fixed<H>(a, s.v0 + lane)) {
+    if (lane < s.vc && s.act && !is_fixed<H>(a, s.v0 + lane)) {
         const int32_t v = s.v0 + lane;
         // no edge, or no counted label: the vertex keeps its label
         const int32_t nl = best ? packed_label(best) : s.old;
@@ -545,6 +548,12 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
     for (int p = 0; p < NP; ++p) {
         run[p] = run[p] && is_active<H>(a, v[p]) && !is_fixed<H>(a, v[p]);
         old[p] = a.keep[v[p]];
+    }
+    if (frontier_on<H>(a)) {  // most waves of a converged step have nothing to do
+        bool any = false;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) any |= run[p];
+        if (__ballot(any) == 0ull) return;
     }
     // every tier vertex has >= 1 edge, so e-1 is a valid index; a vertex not
     // run loads its first edge only
@@ -727,6 +736,12 @@ __device__ __forceinline__ void wave_body(const StepArgs& a, const int4* __restr
     for (int k = 0; k < kWaveNV; ++k) {
         run[k] = i0 + k < nv && is_active<H>(a, v[k]) && !is_fixed<H>(a, v[k]);
         old[k] = a.keep[v[k]];
+    }
+    if (frontier_on<H>(a)) {  // as in the half tier
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < kWaveNV; ++k) any |= run[k];
+        if (!any) return;  // wave-uniform
     }
     // every tier vertex has >= 1 edge, so e-1 is a valid index; a vertex not
     // run loads its first edge only (one line for the whole wave)
@@ -970,10 +985,8 @@ __device__ __forceinline__ void hub_agg_body(const StepArgs& a, const HubArgs& h
     const uint32_t P = hub_buckets(ve - vb, h.part_keys);
     uint32_t* hist = h.hs.hist + h.hist_base[hc.x];      // [bucket][chunk]: run lengths
     uint32_t* lstart = h.hs.lstart + h.hist_base[hc.x];  // [bucket][chunk]: run starts in the chunk region
-    if (!is_active<H>(a, v) || is_fixed<H>(a, v)) {  // block-uniform: the hub keeps its label
-        for (uint32_t q = threadIdx.x; q < P; q += NT) hist[(int64_t)q * nch + hc.y] = 0u;
-        return;
-    }
+    // block-uniform: the hub keeps its label (k_hub_part skips its parts too)
+    if (!is_active<H>(a, v) || is_fixed<H>(a, v)) return;
     const int32_t b = vb + hc.y * h.chunk;
     const int32_t e = min(b + h.chunk, ve);
     const uint32_t cap = min(max(next_pow2(2u * (uint32_t)(e - b)), 64u), cap_max);
@@ -1192,6 +1205,7 @@ __device__ __forceinline__ void hub_part_batch_body(const StepArgs& a, const Hub
         if (p >= h.nparts) break;  // wave-uniform
         const int2 hp = h.parts[p];
         const int32_t v = h.hubs[hp.x];
+        if (!is_active<H>(a, v) || is_fixed<H>(a, v)) continue;  // wave-uniform
         const int32_t d = a.off[v + 1] - a.off[v];
         const uint32_t nch = (uint32_t)((d + h.chunk - 1) / h.chunk);
         const uint32_t* cnt = h.hs.hist + h.hist_base[hp.x] + (int64_t)hp.y * nch;
@@ -1874,9 +1888,43 @@ __global__ void k_iota(int32_t* p, int64_t count) {
 // the next step recomputes everything unless this step marked, and marks
 // when this step changed at most `threshold` labels; the frontier gather's
 // words 3-5 are set up for the next step.
+// With dom.ctl set, the next step's dominant label (see k_dominant_edges):
+// kChangeSlots edges spread evenly over the CSR show their neighbours' new
+// labels, and a label on at least kDomShare of them is it (its share of the
+// edges to within 2%; which label is taken changes no result).
+// dom.ctl = {1 when there is none, 0, the label}.
+struct DominantSample {
+    const int32_t* nbr;
+    const int32_t* L;  // the labels this step wrote
+    int64_t m;         // > 0
+    int32_t* ctl;
+};
+constexpr uint32_t kDomShare = kChangeSlots / 2;
 __global__ __launch_bounds__(kChangeSlots) void k_end_step(unsigned long long* acc,
                                                            unsigned long long* ring, int32_t* ctr,
-                                                           int32_t ring_size, int32_t* fctl) {
+                                                           int32_t ring_size, int32_t* fctl,
+                                                           DominantSample dom) {
+    if (dom.ctl) {  // uniform
+        __shared__ unsigned long long T[2 * kChangeSlots], s_red[kChangeSlots / 64];
+        T[threadIdx.x] = 0ull;
+        T[threadIdx.x + kChangeSlots] = 0ull;
+        const int32_t u = dom.nbr[(int64_t)threadIdx.x * dom.m / kChangeSlots];
+        const uint32_t key = (uint32_t)dom.L[u] + 1u;
+        __syncthreads();
+        const uint32_t at = kc_insert(T, 2 * kChangeSlots - 1, key, 1u) & ~kClaimed;
+        __syncthreads();
+        const uint64_t top =
+            block_max_u64<kChangeSlots>(((uint64_t)(uint32_t)T[at] << 32) | threadIdx.x, s_red);
+        if (threadIdx.x == 0) {
+            s_red[0] = top;
+            if ((uint32_t)(top >> 32) < kDomShare) dom.ctl[0] = 1;
+        }
+        __syncthreads();
+        if ((uint32_t)s_red[0] == threadIdx.x && (uint32_t)(s_red[0] >> 32) >= kDomShare) {
+            dom.ctl[0] = 0;
+            dom.ctl[2] = (int32_t)key - 1;
+        }
+    }
     __shared__ unsigned long long part[kChangeSlots / 64];
     unsigned long long x = acc[threadIdx.x];
     acc[threadIdx.x] = 0ull;
@@ -1901,6 +1949,212 @@ __global__ __launch_bounds__(kChangeSlots) void k_end_step(unsigned long long* a
             fctl[6] = sum <= (unsigned long long)fctl[7] ? 1 : 0;
         }
     }
+}
+
+// The dominant label of a step.  Once an R-MAT graph's labels converge, one
+// label D shows on most edges, yet every edge still fetched its neighbour's
+// 4-byte label, a random 128-byte line; those lines bound the tiers.  Three
+// passes over bits settle the vertices that have D on more than half of their
+// edges, whatever the other labels; the tiers recompute the rest (act = 1):
+//  k_dominant_bits    bit v: vertex v shows D (n/8 bytes)
+//  k_dominant_edges   bit j: edge j's neighbour shows D (m/8 bytes), a stream
+//                     over the CSR whose lookups mostly stay in LDS
+//  k_dominant_decide  a vertex's count is the population count of its edges'
+//                     bits
+// Without a dominant label (ctl[0] = 1) all three return at once.
+// (and bit b of `blocks`: all of vertices [64 b, 64 b + 64) do)
+__global__ __launch_bounds__(256) void k_dominant_bits(const int32_t* __restrict__ L, int32_t n,
+                                                       const int32_t* __restrict__ ctl,
+                                                       unsigned long long* __restrict__ bits,
+                                                       uint32_t* __restrict__ blocks) {
+    if (ctl[0]) return;
+    const int32_t label = __builtin_amdgcn_readfirstlane(ctl[2]);
+    constexpr int kRows = 8;  // loads in flight per lane
+    const int lane = lane_id();
+    const int64_t words = ((int64_t)n + 63) / 64;
+    // a wave takes 32 words of bits, one of blocks
+    const int64_t w0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 32;
+    if (w0 >= words) return;
+    uint32_t full = 0u;
+#pragma unroll
+    for (int r = 0; r < 32; r += kRows) {
+        int32_t l[kRows];
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) l[i] = L[min((w0 + r + i) * 64 + lane, (int64_t)n - 1)];
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const unsigned long long b = __ballot(l[i] == label);
+            if (lane == 0 && w0 + r + i < words) bits[w0 + r + i] = b;  // (bits past n are never read)
+            full |= b == ~0ull ? 1u << (r + i) : 0u;
+        }
+    }
+    if (lane == 0) blocks[w0 >> 5] = full;
+}
+
+// One 1,024-thread workgroup per CU holds in LDS the bits of the first
+// fine * 32 vertices (on degree-sorted graphs the ones most edges name) and
+// one bit per block of 64 for all of them, and streams its share of the
+// edges, four per lane and load.  Only a vertex outside both, in a block that
+// does not show D throughout, has its bit looked up in L2: such a lookup
+// costs a line fill in L1 as its label did.  Converged step of R-MAT scale
+// 25 (1.05G edges): every lookup in L2 5.4 ms a step; the first 1.05M
+// vertices in LDS 1.58 ms for this pass, and with the blocks 0.94 (4.6 TB/s,
+// what a copy reaches).
+constexpr int kDomThreads = 1024;
+constexpr int kDomLdsWords = 152 * 256;  // of 160 KB per CU
+constexpr int kDomU = 2;  // loads in flight per lane (and as many of the next round)
+// ALL: fine covers every vertex; else `nblocks` words of blocks follow (0:
+// the graph has too many, every vertex past fine is looked up).
+template <bool ALL>
+__global__ __launch_bounds__(kDomThreads) void k_dominant_edges(const int32_t* __restrict__ nbr, int64_t m,
+                                                                const uint32_t* __restrict__ bits,
+                                                                const uint32_t* __restrict__ blocks, int32_t fine,
+                                                                int32_t nblocks, const int32_t* __restrict__ ctl,
+                                                                uint32_t* __restrict__ ebits) {
+    if (ctl[0]) return;
+    extern __shared__ __align__(16) uint32_t s_dyn[];
+    for (int32_t i = threadIdx.x; i < fine; i += kDomThreads) s_dyn[i] = bits[i];
+    if constexpr (!ALL) {
+        // without blocks one word of zeros stands for them
+        for (int32_t i = threadIdx.x; i < nblocks; i += kDomThreads) s_dyn[fine + i] = blocks[i];
+        if (nblocks == 0 && threadIdx.x == 0) s_dyn[fine] = 0u;
+    }
+    __syncthreads();
+    const int lane = lane_id();
+    const uint32_t in_lds = (uint32_t)fine, last_block = (uint32_t)max(nblocks, 1) - 1u;
+    const v4i32* nb4 = reinterpret_cast<const v4i32*>(nbr);
+    const int64_t nvec = (m + 3) / 4;  // groups of four edges; the last may be short
+    const int64_t stride = (int64_t)gridDim.x * kDomThreads;
+    auto load = [&](int64_t i0, v4i32* u) {
+#pragma unroll
+        for (int k = 0; k < kDomU; ++k) {
+            const int64_t i = i0 + k * stride + lane;
+            if (i * 4 + 4 <= m) {
+                u[k] = __builtin_nontemporal_load(&nb4[i]);
+            } else {  // past the end, or the short group: its edges, then any vertex
+                const int64_t j = min(i * 4, m - 1);
+                u[k].x = nbr[j];
+                u[k].y = nbr[min(j + 1, m - 1)];
+                u[k].z = nbr[min(j + 2, m - 1)];
+                u[k].w = nbr[min(j + 3, m - 1)];
+            }
+        }
+    };
+    // whole waves stay in the loop together (the words below join lanes)
+    int64_t i0 = (int64_t)blockIdx.x * kDomThreads + (threadIdx.x & ~63);
+    v4i32 u[kDomU];
+    if (i0 < nvec) load(i0, u);
+    while (i0 < nvec) {
+        const int64_t i1 = i0 + stride * kDomU;
+        v4i32 next[kDomU];
+        if (i1 < nvec) load(i1, next);
+        // all LDS lookups, then all L2 lookups (lanes that need none read
+        // word 0 together), each issued before any is used
+        uint32_t x[4 * kDomU];
+#pragma unroll
+        for (int k = 0; k < 4 * kDomU; ++k) {
+            const uint32_t v = (uint32_t)u[k >> 2][k & 3], w = v >> 5;
+            if constexpr (ALL) x[k] = s_dyn[w];
+            else x[k] = s_dyn[w < in_lds ? w : in_lds + min(v >> 11, last_block)];
+        }
+#pragma unroll
+        for (int k = 0; k < 4 * kDomU; ++k) {
+            const uint32_t v = (uint32_t)u[k >> 2][k & 3];
+            x[k] = (x[k] >> (ALL || (v >> 5) < in_lds ? v & 31u : (v >> 6) & 31u)) & 1u;
+        }
+        if constexpr (!ALL) {
+            uint32_t y[4 * kDomU];
+            uint32_t any = 0u;
+#pragma unroll
+            for (int k = 0; k < 4 * kDomU; ++k) {
+                const uint32_t w = (uint32_t)u[k >> 2][k & 3] >> 5;
+                y[k] = w >= in_lds && !x[k] ? w : 0u;  // (word 0 is in LDS)
+                any |= y[k];
+            }
+            if (__ballot(any != 0u)) {  // wave-uniform
+                uint32_t z[4 * kDomU];
+#pragma unroll
+                for (int k = 0; k < 4 * kDomU; ++k) z[k] = bits[y[k]];
+#pragma unroll
+                for (int k = 0; k < 4 * kDomU; ++k)
+                    if (y[k]) x[k] = (z[k] >> (u[k >> 2][k & 3] & 31)) & 1u;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kDomU; ++k) {
+            // this lane's four bits in place, then joined over groups of
+            // eight lanes (quad neighbours, quad pairs, half-row mirror)
+            uint32_t z = (x[4 * k] | x[4 * k + 1] << 1 | x[4 * k + 2] << 2 | x[4 * k + 3] << 3) << (4 * (lane & 7));
+            z |= (uint32_t)__builtin_amdgcn_update_dpp((int)z, (int)z, 0xB1, 0xf, 0xf, false);
+            z |= (uint32_t)__builtin_amdgcn_update_dpp((int)z, (int)z, 0x4E, 0xf, 0xf, false);
+            z |= (uint32_t)__builtin_amdgcn_update_dpp((int)z, (int)z, 0x141, 0xf, 0xf, false);
+            const int64_t i = i0 + k * stride + lane;
+            if ((lane & 7) == 0 && i < nvec) ebits[i >> 3] = z;  // (bits past m are never counted)
+        }
+#pragma unroll
+        for (int k = 0; k < kDomU; ++k) u[k] = next[k];
+        i0 = i1;
+    }
+}
+
+// Set bits among bits [b, e) of ebits, `stride` threads cooperating.
+__device__ __forceinline__ uint32_t count_bits(const uint32_t* __restrict__ ebits, int32_t b, int32_t e, int tid,
+                                               int stride) {
+    uint32_t c = 0u;
+    const int32_t w1 = (int32_t)(((uint32_t)e + 31u) >> 5);
+    for (int32_t w = (b >> 5) + tid; w < w1; w += stride) {
+        uint32_t x = ebits[w];
+        if (w == (b >> 5)) x &= 0xffffffffu << (b & 31);
+        if (w == (e >> 5)) x &= (1u << (e & 31)) - 1u;  // (not met when e is a multiple of 32)
+        c += (uint32_t)__popc(x);
+    }
+    return c;
+}
+// Workgroups [0, nhubs) take a hub each; the others 256 vertices each, one
+// lane per vertex up to kDomLaneDeg edges, a wave above (hubs left out).
+constexpr int32_t kDomLaneDeg = 256;
+__global__ __launch_bounds__(256) void k_dominant_decide(StepArgs a, const uint32_t* __restrict__ ebits,
+                                                         const int32_t* __restrict__ hubs, int32_t nhubs,
+                                                         int32_t hub_deg, uint8_t* __restrict__ act) {
+    if (a.fctl[0]) return;
+    const int32_t label = __builtin_amdgcn_readfirstlane(a.fctl[2]);
+    const int lane = lane_id();
+    // act of vertex v with d edges, c of them showing the label; true when
+    // the vertex is decided and its label changes
+    auto settle = [&](int32_t v, int32_t d, uint32_t c) {
+        const bool won = 2u * c > (uint32_t)d;
+        act[v] = d > 0 && !won ? 1 : 0;
+        if (!won) return false;
+        a.Lw[v] = label;
+        return a.keep[v] != label;
+    };
+    bool changed = false;
+    if ((int32_t)blockIdx.x < nhubs) {
+        __shared__ uint32_t s_c[4];
+        const int32_t v = hubs[blockIdx.x];
+        const int32_t b = a.off[v], e = a.off[v + 1];
+        const uint32_t c = wave_sum_u32(count_bits(ebits, b, e, threadIdx.x, 256));
+        if (lane == 0) s_c[threadIdx.x >> 6] = c;
+        __syncthreads();
+        if (threadIdx.x == 0) changed = settle(v, e - b, s_c[0] + s_c[1] + s_c[2] + s_c[3]);
+        if (threadIdx.x < 64) count_changes(a, changed);
+        return;
+    }
+    const int64_t v0 = (int64_t)(blockIdx.x - (uint32_t)nhubs) * 256 + (threadIdx.x & ~63);
+    const int64_t v = v0 + lane;
+    int32_t b = 0, e = 0;
+    if (v < a.n) {
+        b = a.off[v];
+        e = a.off[v + 1];
+    }
+    if (v < a.n && e - b <= kDomLaneDeg) changed = settle((int32_t)v, e - b, count_bits(ebits, b, e, 0, 1));
+    for (unsigned long long q = __ballot(e - b > kDomLaneDeg && e - b <= hub_deg); q; q &= q - 1ull) {
+        const int src = (int)__builtin_ctzll(q);
+        const int32_t vb = shfl_i32(b, src), ve = shfl_i32(e, src);
+        const uint32_t c = wave_sum_u32(count_bits(ebits, vb, ve, lane, 64));
+        if (lane == src) changed = settle((int32_t)v, ve - vb, c);
+    }
+    count_changes(a, changed);
 }
 
 // ---------------------------------------------------------------- launch ----
@@ -1939,12 +2193,13 @@ static void launch_half(const StepArgs& a, const int4* verts, int32_t nh, hipStr
     }
 }
 
-// Workgroups of `threads` threads of `fn` that the device holds at once.
-static int64_t resident_blocks(const void* fn, int threads) {
+// Workgroups of `threads` threads of `fn` with `lds` bytes of dynamic LDS
+// that the device holds at once.
+static int64_t resident_blocks(const void* fn, int threads, size_t lds = 0) {
     int per_cu = 0, cus = 0, dev = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0) != hipSuccess || per_cu < 1 ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds) != hipSuccess || per_cu < 1 ||
         cus < 1)
         return 1024;
     return (int64_t)per_cu * cus;
@@ -2124,6 +2379,8 @@ void init_kernels() {
     done = true;
     init_counting_kernels();
     const int lim = 160 * 1024 - 1024;
+    (void)hipFuncSetAttribute((const void*)k_dominant_edges<true>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
+    (void)hipFuncSetAttribute((const void*)k_dominant_edges<false>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
 #define GLP_SETLDS(HK, W, G)                                                                    \
     (void)hipFuncSetAttribute((const void*)k_block<HK, W, G, 256>,                              \
                               hipFuncAttributeMaxDynamicSharedMemorySize, lim);                 \
@@ -2402,10 +2659,38 @@ int launch_calib_read(const int32_t* T, int64_t entries, int64_t reads, uint32_t
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "calibration launch: %s", hipGetErrorString(e));
 }
 
+int launch_dominant(const DeviceGraph& g, const StepArgs& a, uint32_t* bits, uint32_t* ebits, uint8_t* act,
+                    hipStream_t s) {
+    if (g.n <= 0 || g.m <= 0) return GLP_OK;
+    const int64_t words = ((int64_t)g.n + 31) / 32;
+    uint32_t* blocks = bits + dominant_bytes(g.n) / 4;
+    hipLaunchKernelGGL(k_dominant_bits, dim3(grid_for(g.n, 4 * 2048)), dim3(256), 0, s, a.L, g.n, a.fctl,
+                       reinterpret_cast<unsigned long long*>(bits), blocks);
+    static const int64_t resident = resident_blocks((const void*)k_dominant_edges<false>, kDomThreads, kDomLdsWords * 4);
+    const dim3 grid((unsigned)std::min<int64_t>(grid_for(g.m, 4 * kDomThreads), resident));
+    if (words <= kDomLdsWords) {
+        hipLaunchKernelGGL((k_dominant_edges<true>), grid, dim3(kDomThreads), (size_t)words * 4, s, a.nbr, g.m, bits,
+                           blocks, (int32_t)words, 0, a.fctl, ebits);
+    } else {
+        // blocks take at most half of LDS (up to 38M vertices)
+        int32_t nblocks = (int32_t)((words + 63) / 64);
+        if (nblocks > kDomLdsWords / 2) nblocks = 0;
+        const int32_t fine = kDomLdsWords - std::max(nblocks, 1);
+        hipLaunchKernelGGL((k_dominant_edges<false>), grid, dim3(kDomThreads), (size_t)kDomLdsWords * 4, s, a.nbr, g.m,
+                           bits, blocks, fine, nblocks, a.fctl, ebits);
+    }
+    const int32_t nh = (int32_t)g.plan.hubs.size();
+    hipLaunchKernelGGL(k_dominant_decide, dim3((unsigned)nh + grid_for(g.n, 256)), dim3(256), 0, s, a, ebits, g.d_hubs,
+                       nh, nh ? g.plan.tune.block_max_deg : INT32_MAX, act);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "dominant label launch: %s", hipGetErrorString(e));
+}
+
 int launch_end_step(unsigned long long* acc, unsigned long long* ring, int32_t* step_ctr,
-                    int32_t ring_size, hipStream_t s, int32_t* fctl) {
+                    int32_t ring_size, hipStream_t s, int32_t* fctl, const int32_t* dom_nbr, const int32_t* dom_L,
+                    int64_t dom_m, int32_t* dom_ctl) {
     hipLaunchKernelGGL(k_end_step, dim3(1), dim3(kChangeSlots), 0, s, acc, ring, step_ctr, ring_size,
-                       fctl);
+                       fctl, DominantSample{dom_nbr, dom_L, dom_m, dom_ctl});
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "end_step launch: %s", hipGetErrorString(e));
 }

@@ -38,6 +38,10 @@ struct glp_session {
     int64_t act_bytes = 0;
     uint32_t* chg[2] = {nullptr, nullptr};  // frontier gather: changed-vertex bitmaps
     void* push = nullptr;                   // frontier gather: push entries of a step
+    uint32_t* dom_bits = nullptr;          // dominant label: the vertices showing it,
+    uint32_t* dom_ebits = nullptr;         // the edges whose neighbour does,
+    uint8_t* dom_act = nullptr;            // the vertices it leaves open
+    int32_t* domctl = nullptr;             // and {1 when there is none, 0, the label, 0}
     uint8_t* seeds = nullptr;              // seeded LP: n bytes, nonzero = seed
     bool seeds_set = false;
     int64_t chg_bytes = 0;

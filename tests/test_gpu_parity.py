@@ -378,3 +378,41 @@ def test_first_step_of_a_loaded_file(tmp_path):
         g = G.Graph.load_bin(str(tmp_path / name))
         off, nbr, _ = g.csr()
         assert_steps_equal(gpu_steps(g, 3), O.classic(off, nbr, 3))
+
+
+@pytest.mark.parametrize("sort", [False, True])
+def test_dominant_label_settles_the_same_labels(sort):
+    """A graph large enough for the dominant label's passes (2^24 edges,
+    hubs): the labels and change counts of each step, while labels are
+    diverse, converge and have converged, equal those of the separate gather,
+    which has no such passes; classic and layered gamma 0, replayed, after a
+    restore and across gammas."""
+    g = G.Graph.rmat(20, 20, seed=11, degree_sort=sort)
+    assert g.m >= 1 << 24
+    steps = 8
+    want = gpu_steps(g, steps, gather=True)
+    _, nbr, _ = g.csr()
+    assert np.bincount(want[steps - 2][nbr]).max() > 0.55 * g.m  # the last step has a dominant label
+    assert_steps_equal(gpu_steps(g, steps), want)
+    assert_steps_equal(gpu_steps(g, steps, method=G.LAYERED, gamma=(0, 1)), want)
+    L0 = np.arange(g.n, dtype=np.int32)
+    with G.Session(g) as s:
+        s.step(steps, graph=True)
+        assert np.array_equal(s.labels(), want[-1])
+        assert s.changes().tolist() == [int((want[t] != (want[t - 1] if t else L0)).sum()) for t in range(steps)]
+        s.reset()
+        s.step(5)
+        state = s.save()
+        s.step(2)
+        s.load(state)
+        s.step(3)
+        assert np.array_equal(s.labels(), want[-1])
+    # gamma 0, 1/4, 0: the label chosen before the switch may have moved on
+    dumps = []
+    for gather in (False, True):
+        with G.Session(g, method=G.LAYERED, gamma=(0, 1), gather=gather) as s:
+            for gamma, k in (((0, 1), 6), ((1, 4), 2), ((0, 1), 2)):
+                s.set_gamma(*gamma)
+                s.step(k)
+            dumps.append(s.labels())
+    assert np.array_equal(dumps[0], dumps[1])

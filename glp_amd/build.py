@@ -16,8 +16,10 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = os.environ.get("GLP_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["kernels.hip", "counting.hip", "session.hip", "batch.hip", "server.hip", "plan.hip",
-               "autotune.hip", "gen_device.hip", "noalloc.hip"]
+# (the tier kernels, the longest to compile, first)
+HIP_SOURCES = ["tiers_multi.hip", "tiers_classic.hip", "tiers_layered.hip", "tiers_slpa.hip", "tiers_user.hip",
+               "tiers_seeded.hip", "tiers_layered_vol.hip", "tiers_first.hip", "kernels.hip", "counting.hip",
+               "session.hip", "batch.hip", "server.hip", "plan.hip", "autotune.hip", "gen_device.hip", "noalloc.hip"]
 CPP_SOURCES = ["graph_io.cpp", "gen.cpp"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]

@@ -197,6 +197,25 @@ void init_kernels();
 // calls it.
 void init_counting_kernels();
 
+// The tier kernels' launches per hook set (tiers_*.hip), and their set-up.
+#define GLP_DECLARE_TIERS(name)                                                                   \
+    int launch_tiers_##name(bool weighted, bool gathered, const DeviceGraph& g, const HubScratch& hs, \
+                            const StepArgs& a, hipStream_t s, hipEvent_t* ev);                    \
+    void init_tiers_##name();
+GLP_DECLARE_TIERS(classic)
+GLP_DECLARE_TIERS(layered)
+GLP_DECLARE_TIERS(slpa)
+GLP_DECLARE_TIERS(user)
+GLP_DECLARE_TIERS(seeded)
+#undef GLP_DECLARE_TIERS
+int launch_tiers_layered_vol(bool weighted, const DeviceGraph& g, const HubScratch& hs, const StepArgs& a,
+                             hipStream_t s, hipEvent_t* ev);
+int launch_tiers_first(bool weighted, const DeviceGraph& g, const HubScratch& hs, const StepArgs& a, hipStream_t s,
+                       hipEvent_t* ev);
+void init_tiers_layered_vol();
+void init_tiers_first();
+void init_tiers_multi();
+
 // Enqueues the counting part of one step (all tiers) on stream s.
 // ev (may be null) holds 2*GLP_NTIERS events for per-tier timing.
 int launch_step(Method method, bool weighted, bool gathered, const DeviceGraph& g,

@@ -32,6 +32,7 @@
 #include "device_prims.h"
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace glp {
 using namespace dev;
@@ -1360,6 +1361,61 @@ __global__ __launch_bounds__(256) void k_hub_mark(StepArgs a, HubArgs h) {
     hub_mark_body<H>(a, h, blockIdx.x);
 }
 
+// All tiers of a step's counting but the hubs' second and third passes in one
+// launch of 512-thread workgroups: workgroup ranges, the longest-running
+// first (hub chunks, block classes from the largest table down, wave-tier
+// units of 4 and 2 edges per lane, half-tier units, packed groups).  On small
+// graphs every tier's launch takes 4-12 us, most of it starting and draining;
+// together they take about what the longest does.  A tier's registers and LDS
+// are the largest tier's, so a launch that fills the chip by itself is better
+// off alone (one_launch).
+constexpr int kTiersThreads = 512;
+constexpr int kTiersWaves = kTiersThreads / 64;
+constexpr size_t kTiersWaveLds = kWaveCap * 8;  // a wave's area (the wave tier's table)
+static_assert(sizeof(PackedLds) <= kTiersWaveLds && sizeof(HalfLds<32>) <= kTiersWaveLds, "wave areas");
+struct TierWork {
+    const int2* groups;
+    const int4* half;
+    const int4* wave;  // the first wave_short of degree <= 128
+    const int32_t* block[kMaxBlockClasses];
+    uint32_t class_cap[kMaxBlockClasses];
+    int32_t ngroups, nge, nhalf, nwave_short, nwave;
+    uint32_t end_hub;                      // cumulative workgroups
+    uint32_t end_block[kMaxBlockClasses];  // class kMaxBlockClasses - 1 first
+    uint32_t end_wave, end_wave_short, end_half;
+};
+template <class H, bool W>
+__global__ __launch_bounds__(kTiersThreads) void k_tiers(StepArgs a, TierWork w, HubArgs h) {
+    constexpr bool G = false;  // sessions with a separate gather keep their launches
+    extern __shared__ __align__(16) uint32_t s_dyn[];
+    const uint32_t blk = blockIdx.x;
+    if (blk < w.end_hub) {
+        hub_agg_body<H, W, G, kTiersThreads, 4>(a, h, blk);
+        return;
+    }
+    uint32_t at = w.end_hub;
+#pragma unroll
+    for (int c = kMaxBlockClasses - 1; c >= 0; --c) {
+        if (blk < w.end_block[c]) {
+            block_body<H, W, G, kTiersThreads, 4>(a, w.block[c], w.class_cap[c], blk - at);
+            return;
+        }
+        at = w.end_block[c];
+    }
+    const int wv = threadIdx.x >> 6;
+    char* lds = reinterpret_cast<char*>(s_dyn) + wv * kTiersWaveLds;
+    auto unit = [&](uint32_t first) { return (blk - first) * kTiersWaves + wv; };
+    if (blk < w.end_wave)
+        wave_body<H, W, G, 4>(a, w.wave + w.nwave_short, w.nwave - w.nwave_short, unit(at),
+                              reinterpret_cast<unsigned long long*>(lds));
+    else if (blk < w.end_wave_short)
+        wave_body<H, W, G, 2>(a, w.wave, w.nwave_short, unit(w.end_wave), reinterpret_cast<unsigned long long*>(lds));
+    else if (blk < w.end_half)
+        half_body<H, W, G, 1>(a, w.half, w.nhalf, unit(w.end_wave_short), *reinterpret_cast<HalfLds<32>*>(lds));
+    else
+        packed_body<H, W, G, 1>(a, w.groups, w.ngroups, w.nge, unit(w.end_half), *reinterpret_cast<PackedLds*>(lds));
+}
+
 // Folded jobs: cum[j] is the first workgroup of job j in this launch
 // (cum[njobs] = grid size); a workgroup finds its job by binary search.
 __device__ __forceinline__ int32_t job_of(const int32_t* __restrict__ cum, int32_t njobs,
@@ -1421,6 +1477,85 @@ static int64_t resident_blocks(const void* fn, int threads, size_t lds = 0) {
     return (int64_t)per_cu * cus;
 }
 
+static HubArgs hub_args(const DeviceGraph& g, const HubScratch& hs) {
+    const Plan& p = g.plan;
+    HubArgs h;
+    h.hubs = g.d_hubs;
+    h.chunks = g.d_hub_chunks;
+    h.parts = g.d_hub_parts;
+    h.chunk0 = g.d_hub_chunk0;
+    h.base = g.d_hub_base;
+    h.hist_base = g.d_hub_hist_base;
+    h.chunk = p.tune.hub_chunk;
+    h.part_keys = p.tune.part_keys;
+    h.part_limit = p.tune.part_limit;
+    h.nhubs = (int32_t)p.hubs.size();
+    h.nparts = (int32_t)p.hub_parts.size();
+    h.part_batch = hub_part_batch(h.nparts);
+    h.hs = hs;
+    return h;
+}
+
+// The work of k_tiers with ng packed groups; returns its workgroups.
+static uint32_t tier_work(const DeviceGraph& g, int32_t ng, TierWork& w, size_t* lds) {
+    const Plan& p = g.plan;
+    auto blocks = [](size_t items, size_t per) { return (uint32_t)((items + per - 1) / per); };
+    w.groups = g.d_groups;
+    w.half = g.d_half;
+    w.wave = g.d_wave;
+    w.ngroups = ng;
+    w.nge = (int32_t)p.groups_with_edges;
+    w.nhalf = (int32_t)p.half.size();
+    w.nwave_short = (int32_t)p.wave_short;
+    w.nwave = (int32_t)p.wave.size();
+    uint32_t at = (uint32_t)p.hub_chunks.size();
+    *lds = kTiersWaves * kTiersWaveLds;
+    if (at) *lds = std::max(*lds, hub_agg_lds(p.tune.hub_chunk, p.hub_max_buckets));
+    w.end_hub = at;
+    for (int c = kMaxBlockClasses - 1; c >= 0; --c) {
+        const bool any = c < p.nclasses && !p.block[c].empty();
+        w.block[c] = any ? g.d_block[c] : nullptr;
+        w.class_cap[c] = any ? (uint32_t)p.class_cap[c] : 0u;
+        if (any) {
+            at += (uint32_t)p.block[c].size();
+            *lds = std::max(*lds, (size_t)p.class_cap[c] * 8);
+        }
+        w.end_block[c] = at;
+    }
+    w.end_wave = at += blocks(p.wave.size() - (size_t)p.wave_short, kTiersWaves * kWaveNV);
+    w.end_wave_short = at += blocks((size_t)p.wave_short, kTiersWaves * kWaveNV);
+    w.end_half = at += blocks(p.half.size(), kTiersWaves * 2);
+    return at + blocks((size_t)ng, kTiersWaves);
+}
+// Whether a plan's tiers go in one launch (k_tiers): each launch saved is
+// worth about 5 us, and each workgroup runs with the largest tier's registers
+// and LDS.  12 steps, separate / together (thousands of workgroups, launches):
+// R-MAT scale 12 510 / 177 us, 16 873 / 437 us, 18 1,123 / 907 us (10, 10),
+// 19 1,737 / 2,362 us (20, 10); LFR 300,000 vertices 1,098 / 953 us (9, 5);
+// planted 65,536 525 / 494 us (2.3, 2), 100,000 of degree 38 463 / 484 us
+// (6, 2).
+constexpr int64_t kTogetherPerLaunch = 3500, kTogetherMax = 16384;
+static bool one_launch(const Plan& p, int32_t ng) {
+    int64_t wgs = (int64_t)p.hub_chunks.size(), launches = p.hub_chunks.empty() ? 0 : 1;
+    for (int c = 0; c < p.nclasses; ++c) {
+        wgs += (int64_t)p.block[c].size();
+        launches += p.block[c].empty() ? 0 : 1;
+    }
+    launches += (ng > 0) + !p.half.empty() + (p.wave_short > 0) + ((int64_t)p.wave.size() > p.wave_short);
+    wgs += ((int64_t)p.wave.size() / kWaveNV + (int64_t)p.half.size() / 2 + ng) / kTiersWaves;
+    return p.tune.fused_small == 0 && launches > 1 &&
+           wgs <= std::min(kTogetherMax, kTogetherPerLaunch * (launches - 1));
+}
+template <class H, bool W>
+static int launch_together(const DeviceGraph& g, const HubScratch& hs, const StepArgs& a, int32_t ng, hipStream_t s) {
+    TierWork w;
+    size_t lds = 0;
+    const uint32_t grid = tier_work(g, ng, w, &lds);
+    if (grid) hipLaunchKernelGGL((k_tiers<H, W>), dim3(grid), dim3(kTiersThreads), lds, s, a, w, hub_args(g, hs));
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "tier launch failed: %s", hipGetErrorString(e));
+}
+
 template <class H, bool W, bool G>
 static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepArgs& a,
                         hipStream_t s, hipEvent_t* ev) {
@@ -1428,10 +1563,19 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
     auto mark = [&](int tier, int edge) {
         if (ev) (void)hipEventRecord(ev[2 * tier + edge], s);
     };
-    mark(GLP_TIER_PACKED, 0);
     const int32_t ng = (int32_t)(H::kSkipIsolated && !a.write_isolated ? p.groups_with_edges
                                                                        : (int64_t)p.groups.size());
-    if (p.tune.fused_small > 0 && hs.work) {
+    bool together = false;
+    if constexpr (!G) {
+        together = !ev && one_launch(p, ng);  // (ev: the tiers are timed one by one)
+        if (together) {
+            const int rc = launch_together<H, W>(g, hs, a, ng, s);
+            if (rc != GLP_OK) return rc;
+        }
+    }
+    mark(GLP_TIER_PACKED, 0);
+    if (together) {
+    } else if (p.tune.fused_small > 0 && hs.work) {
         // packed and half tiers in one persistent launch
         SmallTiers st;
         const int32_t hs_n = (int32_t)p.half_short;
@@ -1477,7 +1621,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
     }
     mark(GLP_TIER_PACKED, 1);
     mark(GLP_TIER_WAVE, 0);
-    if (!p.half.empty() && !(p.tune.fused_small > 0 && hs.work)) {
+    if (!together && !p.half.empty() && !(p.tune.fused_small > 0 && hs.work)) {
         const int32_t nh = (int32_t)p.half.size();
         // 16 lanes per vertex halve the instructions per vertex and double
         // the vertices in flight per wave; they pay off once the launch has
@@ -1493,7 +1637,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
             launch_half<H, W, G, 32>(a, g.d_half, nh, s);
         }
     }
-    if (!p.wave.empty()) {
+    if (!together && !p.wave.empty()) {
         // degrees <= 128 (the list's first wave_short entries) load two edges
         // per lane, the rest four
         const int32_t ns = (int32_t)p.wave_short, nw = (int32_t)p.wave.size();
@@ -1507,7 +1651,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
     mark(GLP_TIER_WAVE, 1);
     mark(GLP_TIER_BLOCK, 0);
     for (int c = 0; c < p.nclasses; ++c) {
-        if (p.block[c].empty()) continue;
+        if (together || p.block[c].empty()) continue;
         const uint32_t cap = (uint32_t)p.class_cap[c];
         const size_t lds = (size_t)cap * 2 * sizeof(uint32_t);
         const unsigned nb = (unsigned)p.block[c].size();
@@ -1540,25 +1684,13 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
     mark(GLP_TIER_BLOCK, 1);
     mark(GLP_TIER_HUB, 0);
     if (!p.hubs.empty()) {
-        HubArgs h;
-        h.hubs = g.d_hubs;
-        h.chunks = g.d_hub_chunks;
-        h.parts = g.d_hub_parts;
-        h.chunk0 = g.d_hub_chunk0;
-        h.base = g.d_hub_base;
-        h.hist_base = g.d_hub_hist_base;
-        h.chunk = p.tune.hub_chunk;
-        h.part_keys = p.tune.part_keys;
-        h.part_limit = p.tune.part_limit;
-        h.nhubs = (int32_t)p.hubs.size();
-        h.nparts = (int32_t)p.hub_parts.size();
-        h.part_batch = hub_part_batch(h.nparts);
-        h.hs = hs;
+        const HubArgs h = hub_args(g, hs);
         const unsigned nc = (unsigned)p.hub_chunks.size();
         const unsigned np = (unsigned)p.hub_parts.size();
         const size_t lds_part = (size_t)next_pow2(2u * (uint32_t)h.part_keys) * 2 * sizeof(uint32_t);
-        hipLaunchKernelGGL((k_hub_agg<H, W, G>), dim3(nc), dim3(kHubAggThreads),
-                           hub_agg_lds(h.chunk, p.hub_max_buckets), s, a, h);
+        if (!together)
+            hipLaunchKernelGGL((k_hub_agg<H, W, G>), dim3(nc), dim3(kHubAggThreads),
+                               hub_agg_lds(h.chunk, p.hub_max_buckets), s, a, h);
         mark(GLP_TIER_HUB, 1);
         mark(GLP_TIER_AUX, 0);
         if (!(first_of<H>::value && a.ascending))
@@ -1605,6 +1737,7 @@ static void set_tier_limits_of() {
     set_lds_limit((const void*)k_block<H, W, G, 1024, 4>);
     set_lds_limit((const void*)k_block<H, W, G, 512, 4>);
     set_lds_limit((const void*)k_hub_agg<H, W, G>);
+    if constexpr (!G) set_lds_limit((const void*)k_tiers<H, W>);
 }
 template <class H, bool GATHERED>
 static void set_tier_limits() {

@@ -416,3 +416,22 @@ def test_dominant_label_settles_the_same_labels(sort):
                 s.step(k)
             dumps.append(s.labels())
     assert np.array_equal(dumps[0], dumps[1])
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(weighted=True), dict(method=G.LAYERED, gamma=(1, 4)),
+                                dict(method=G.LAYERED, gamma=(1, 2), weighted=True), dict(method=G.USER),
+                                dict(method=G.SLPA, slpa_T=4), dict(frontier=1)])
+@pytest.mark.parametrize("tuned", [dict(), dict(pack_max_deg=4, half_max_deg=20, wave_max_deg=40, block_max_deg=300,
+                                                hub_chunk=256, part_keys=256), dict(half_max_deg=0),
+                                   dict(block_max_deg=8192)])
+def test_one_launch_equals_a_launch_per_tier(kw, tuned):
+    """Small graphs count all tiers in one launch; timing the tiers one by one
+    (profile) takes a launch each.  Degrees on both sides of every tier's
+    bound, and a weighted R-MAT graph, with several tier layouts."""
+    with G.tuning(**tuned):
+        n, edges = tier_boundary_graph(seed=7)
+        w = np.random.default_rng(1).integers(1, 9, len(edges)).astype(np.uint32)
+        graphs = [G.Graph.rmat(12, 16, seed=9, wmax=8), G.Graph.from_edges(n, edges, w)]
+        for g in graphs:
+            one = gpu_steps(g, 4, **kw)
+            assert_steps_equal(one, gpu_steps(g, 4, profile=True, **kw))

@@ -981,7 +981,7 @@ int enqueue_counting_step(glp_session* s) {
     a.w = dg.w;
     a.n = s->n;
     a.t = s->t + 1;
-    a.changes = s->d_acc;
+    a.changes = step_counters(s);
     a.L = s->L[s->cur];
     a.keep = s->L[s->cur];
     a.Lw = s->L[s->cur ^ 1];
@@ -1061,7 +1061,7 @@ int enqueue_counting_step(glp_session* s) {
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(GLP_E_HIP, "counting launch: %s", hipGetErrorString(e));
     }
-    int rc = launch_end_step(s->d_acc, s->d_ring, s->d_ctr, kChangeRing, s->stream);
+    int rc = end_step(s, a.nbr, a.Lw, false);
     if (rc != GLP_OK) return rc;
     s->cur ^= 1;
     s->t += 1;

@@ -250,10 +250,29 @@ int launch_label_volumes(const int32_t* L, const int32_t* V, int2* LV, int32_t n
 // V[l] += #{v < n : L[v] = l} (layered LP's volume of the written labels;
 // V zeroed first).
 int launch_volume(const int32_t* L, int32_t* V, int32_t n, hipStream_t s);
-// p[i] = seeds[i] ? i : -1 (seeded LP's initial labels).
-int launch_seed_labels(int32_t* p, const uint8_t* seeds, int64_t count, hipStream_t s);
 // dom_ctl (may be null): chooses the next step's dominant label from the
 // labels dom_L over the m > 0 edges of dom_nbr, {1 when there is none, 0, it}.
+// Sums `rows` rows of kChangeSlots counters into the ring, one step each, and
+// clears them.
+int launch_end_steps(unsigned long long* acc, int32_t rows, unsigned long long* ring, int32_t* step_ctr,
+                     int32_t ring_size, hipStream_t s);
+// What a session's reset writes, in one launch: L_0 in both label buffers
+// (seeds null: v; else v on seeds, -1 elsewhere; unseeded: all -1), and
+// whatever else the session has (null: it has not).
+struct ResetArgs {
+    int32_t* L[2];
+    const uint8_t* seeds;
+    int32_t unseeded;         // seeded LP before its seeds are set
+    int32_t* V[2];            // volumes: 1 and 0
+    int32_t* mem;             // SLPA memory row 0: v
+    int64_t n;
+    int32_t* zero[7];         // arrays of zero_words words to clear
+    int64_t zero_words[7];
+    int32_t* fctl;            // frontier control words, and their values
+    int32_t fctl_words[8];
+    int32_t* domctl;          // dominant label control words: none
+};
+int launch_reset(const ResetArgs& r, hipStream_t s);
 int launch_end_step(unsigned long long* acc, unsigned long long* ring, int32_t* step_ctr,
                     int32_t ring_size, hipStream_t s, int32_t* fctl = nullptr, const int32_t* dom_nbr = nullptr,
                     const int32_t* dom_L = nullptr, int64_t dom_m = 0, int32_t* dom_ctl = nullptr);

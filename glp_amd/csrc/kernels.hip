@@ -394,12 +394,6 @@ int launch_multi_volume(VolumeMode mode, const VolumeJob* jobs, const int32_t* c
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "folded volume launch: %s", hipGetErrorString(e));
 }
 
-// Seeded LP's L_0 (header/kernel.cuh:453-466): v for a seed, -1 otherwise.
-__global__ void k_seed_labels(int32_t* p, const uint8_t* __restrict__ seeds, int64_t count) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride)
-        p[i] = seeds[i] ? (int32_t)i : -1;
-}
 __global__ void k_label_volumes(const int32_t* __restrict__ L, const int32_t* __restrict__ V,
                                 int2* __restrict__ LV, int32_t n) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -413,6 +407,56 @@ __global__ void k_iota(int32_t* p, int64_t count) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += stride)
         p[i] = (int32_t)i;
 }
+// The end of `rows` plain steps (no frontier, no dominant label): wave i sums
+// rows i, i + 16, ... of change counters into the ring.  One launch for the
+// steps of a call (at most kAccRows) instead of one each: on a graph of a
+// thousand vertices it was half of a step's 10 us.
+__global__ __launch_bounds__(1024) void k_end_steps(unsigned long long* acc, int32_t rows, unsigned long long* ring,
+                                                    int32_t* ctr, int32_t ring_size) {
+    const int lane = lane_id();
+    const int32_t t = *ctr;
+    for (int32_t r = threadIdx.x >> 6; r < rows; r += 16) {
+        unsigned long long* row = acc + (size_t)r * kChangeSlots;
+        unsigned long long x = 0ull;
+#pragma unroll
+        for (int i = 0; i < kChangeSlots; i += 64) {
+            x += row[i + lane];
+            row[i + lane] = 0ull;
+        }
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) x += shfl_u64(x, lane ^ d);
+        if (lane == 0) ring[(t + r) % ring_size] = x;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) *ctr = t + rows;
+}
+
+// A session's reset (ResetArgs; seeded labels as header/kernel.cuh:453-466):
+// launch bound on small graphs, one launch
+// instead of seven.
+__global__ __launch_bounds__(256) void k_reset(ResetArgs r) {
+    const int64_t t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t v = t0; v < r.n; v += stride) {
+        const int32_t l = r.unseeded || (r.seeds && !r.seeds[v]) ? -1 : (int32_t)v;
+        r.L[0][v] = l;
+        r.L[1][v] = l;
+        if (r.V[0]) {
+            r.V[0][v] = 1;  // V_0(l) = #{u : L_0[u] = l} = 1
+            r.V[1][v] = 0;
+        }
+        if (r.mem) r.mem[v] = (int32_t)v;  // M_v[0] = v
+    }
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        if (r.zero[k])
+            for (int64_t i = t0; i < r.zero_words[k]; i += stride) r.zero[k][i] = 0;
+    if (t0 == 0 && r.fctl)
+        for (int i = 0; i < 8; ++i) r.fctl[i] = r.fctl_words[i];
+    if (t0 == 0 && r.domctl)
+        for (int i = 0; i < 4; ++i) r.domctl[i] = i == 0 ? 1 : 0;
+}
+
 // Sums and clears the step's change counters into the ring and advances
 // the step counter.  One workgroup of kChangeSlots threads.
 // With a frontier control block fctl = {all_active, mark, threshold, ...}:
@@ -817,14 +861,6 @@ int launch_volume(const int32_t* L, int32_t* V, int32_t n, hipStream_t s) {
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "volume launch: %s", hipGetErrorString(e));
 }
 
-int launch_seed_labels(int32_t* p, const uint8_t* seeds, int64_t count, hipStream_t s) {
-    if (count <= 0) return GLP_OK;
-    const unsigned grid = (unsigned)std::min<int64_t>(grid_for(count, 256), 256 * 32);
-    hipLaunchKernelGGL(k_seed_labels, dim3(grid), dim3(256), 0, s, p, seeds, count);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "seed label launch: %s", hipGetErrorString(e));
-}
-
 int launch_fill_i32(int32_t* p, int32_t value, int64_t count, hipStream_t s) {
     if (count <= 0) return GLP_OK;
     const unsigned grid = (unsigned)std::min<int64_t>(grid_for(count, 256), 256 * 32);
@@ -945,6 +981,22 @@ int launch_dominant(const DeviceGraph& g, const StepArgs& a, uint32_t* bits, uin
                        nh, nh ? g.plan.tune.block_max_deg : INT32_MAX, act);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "dominant label launch: %s", hipGetErrorString(e));
+}
+
+int launch_end_steps(unsigned long long* acc, int32_t rows, unsigned long long* ring, int32_t* step_ctr,
+                     int32_t ring_size, hipStream_t s) {
+    if (rows <= 0) return GLP_OK;
+    hipLaunchKernelGGL(k_end_steps, dim3(1), dim3(1024), 0, s, acc, rows, ring, step_ctr, ring_size);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "end_steps launch: %s", hipGetErrorString(e));
+}
+
+int launch_reset(const ResetArgs& r, hipStream_t s) {
+    int64_t work = r.n;
+    for (int k = 0; k < 7; ++k) work = std::max(work, r.zero[k] ? r.zero_words[k] : 0);
+    hipLaunchKernelGGL(k_reset, dim3((unsigned)std::min<int64_t>(grid_for(work, 256), 256 * 32)), dim3(256), 0, s, r);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "reset launch: %s", hipGetErrorString(e));
 }
 
 int launch_end_step(unsigned long long* acc, unsigned long long* ring, int32_t* step_ctr,

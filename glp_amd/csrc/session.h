@@ -8,6 +8,7 @@
 
 namespace glp {
 constexpr int32_t kChangeRing = 4096;  // per-step change counts kept on the device
+constexpr int32_t kAccRows = 32;       // steps whose change counters are summed together
 }
 
 struct glp_session {
@@ -46,7 +47,8 @@ struct glp_session {
     bool seeds_set = false;
     int64_t chg_bytes = 0;
     glp::HubScratch hs;
-    unsigned long long* d_acc = nullptr;   // change counter of the running step
+    unsigned long long* d_acc = nullptr;   // kAccRows rows of change counters, zero once summed
+    int32_t acc_rows = 0;                  // rows of steps enqueued and not yet summed
     unsigned long long* d_ring = nullptr;  // change count of each finished step
     int32_t* d_ctr = nullptr;              // device-side step counter
     int cur = 0;                           // index of the current label buffer
@@ -77,6 +79,13 @@ int session_sync(glp_session* s);
 int session_labels(glp_session* s, int32_t* out);
 // replayed: the step is being captured, to be replayed from any later state
 int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed = false);
+// Ends an enqueued step: its change counters (row s->acc_rows of d_acc) are
+// summed with those of the following steps by end_steps, or at once where the
+// step's end decides something for the next (frontier, dominant label) or is
+// captured.
+unsigned long long* step_counters(glp_session* s);
+int end_step(glp_session* s, const int32_t* nbr, const int32_t* Lw, bool replayed);
+int end_steps(glp_session* s);
 // count-min / frequent / buffer steps (counting.hip)
 int enqueue_counting_step(glp_session* s);
 int counting_wide_list(glp_session* s);

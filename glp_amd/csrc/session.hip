@@ -272,7 +272,7 @@ size_t session_bytes(const HostCSR& g, const Plan& p, const glp_params& prm) {
     if (prm.frontier == 2 && prm.gather) b += (size_t)g.m * 4;  // the lookahead's second adj
     if (dominant_session(g, p, prm)) b += dominant_bytes(g.n) + dominant_bytes(g.n / 64 + 1) + dominant_bytes(g.m) + n + 16;
     b += hub_scratch_bytes(p, prm.frontier != 0);
-    b += 8 * kChangeSlots + 8 * kChangeRing + 4 + 4;  // change counters and ring, step and unit counters
+    b += 8 * kChangeSlots * kAccRows + 8 * kChangeRing + 4 + 4;  // change counters and ring, step and unit counters
     return b;
 }
 
@@ -353,7 +353,7 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
         GLP_HIP(hipMalloc(&s->domctl, 16));
     }
     GLP_HIP(hipMalloc(&s->hs.work, 4));  // the persistent small-tier launch's counter
-    GLP_HIP(hipMalloc(&s->d_acc, 8 * kChangeSlots));
+    GLP_HIP(hipMalloc(&s->d_acc, 8 * kChangeSlots * kAccRows));
     GLP_HIP(hipMalloc(&s->d_ring, 8 * kChangeRing));
     GLP_HIP(hipMalloc(&s->d_ctr, 4));
     GLP_HIP(hipEventCreate(&s->ev_start));
@@ -369,12 +369,6 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
     return GLP_OK;
 }
 
-// The next step has no dominant label.
-static int clear_dominant(glp_session* s) {
-    int rc = launch_fill_i32(s->domctl, 0, 4, s->stream);
-    return rc ? rc : launch_fill_i32(s->domctl, 1, 1, s->stream);
-}
-
 int session_reset(glp_session* s) {
     const int64_t n = s->n;
     s->cur = 0;
@@ -388,38 +382,65 @@ int session_reset(glp_session* s) {
         s->timing.tier_launches[i] = 0;
     }
     s->host_changes.clear();
-    int rc;
-    // L_0 in both buffers (RS: both label buffers start equal): v, or for
-    // seeded LP v on seeds and -1 elsewhere (all -1 until seeds are set)
+    s->acc_rows = 0;
+    // L_0 in both buffers (RS: both label buffers start equal)
+    ResetArgs r{};
+    r.n = n;
+    int k = 0;
+    auto zero = [&](void* p, int64_t bytes) {
+        r.zero[k] = static_cast<int32_t*>(p);
+        r.zero_words[k++] = bytes / 4;
+    };
     for (int b = 0; b < 2; ++b) {
-        if (s->method != Method::Seeded) rc = launch_iota(s->L[b], n, s->stream);
-        else if (s->seeds_set) rc = launch_seed_labels(s->L[b], s->seeds, n, s->stream);
-        else rc = launch_fill_i32(s->L[b], -1, n, s->stream);
-        if (rc) return rc;
+        r.L[b] = s->L[b];
+        r.V[b] = s->V[b];
     }
-    if (s->V[0]) {
-        // V_0(l) = #{u : L_0[u] = l} = 1
-        if ((rc = launch_fill_i32(s->V[0], 1, n, s->stream))) return rc;
-        if ((rc = launch_fill_i32(s->V[1], 0, n, s->stream))) return rc;
+    if (s->method == Method::Seeded) {
+        r.seeds = s->seeds_set ? s->seeds : nullptr;
+        r.unseeded = s->seeds_set ? 0 : 1;
     }
-    if (s->mem && (rc = launch_iota(s->mem, n, s->stream))) return rc;  // M_v[0] = v
+    r.mem = s->mem;
     if (s->fctl) {
         // the first step recomputes every vertex and does not mark; marking
         // starts after a step that changed at most n/32 labels
         const int32_t ctl[8] = {1, 0, std::max<int32_t>(1, (int32_t)(n / 32)), 0, 0, 0, 0,
                                 push_edge_limit(s->g->csr.m)};
-        GLP_HIP(hipMemcpyAsync(s->fctl, ctl, sizeof ctl, hipMemcpyHostToDevice, s->stream));
-        if ((rc = launch_zero_bytes(s->act[0], s->act_bytes, s->stream))) return rc;
-        if ((rc = launch_zero_bytes(s->act[1], s->act_bytes, s->stream))) return rc;
+        std::memcpy(r.fctl_words, ctl, sizeof ctl);
+        r.fctl = s->fctl;
+        zero(s->act[0], s->act_bytes);
+        zero(s->act[1], s->act_bytes);
     }
-    if (s->domctl && (rc = clear_dominant(s))) return rc;
-    for (uint32_t* c : s->chg)
-        if (c && (rc = launch_zero_bytes(c, s->chg_bytes, s->stream))) return rc;
-    GLP_HIP(hipMemsetAsync(s->d_acc, 0, 8 * kChangeSlots, s->stream));
-    GLP_HIP(hipMemsetAsync(s->d_ring, 0, 8 * kChangeRing, s->stream));
-    GLP_HIP(hipMemsetAsync(s->d_ctr, 0, 4, s->stream));
-    GLP_HIP(hipStreamSynchronize(s->stream));
-    return GLP_OK;
+    if (s->chg[0]) {
+        zero(s->chg[0], s->chg_bytes);
+        zero(s->chg[1], s->chg_bytes);
+    }
+    r.domctl = s->domctl;
+    zero(s->d_acc, 8 * kChangeSlots * kAccRows);
+    zero(s->d_ring, 8 * kChangeRing);
+    zero(s->d_ctr, 4);
+    return launch_reset(r, s->stream);
+}
+
+// The next step has no dominant label.
+static int clear_dominant(glp_session* s) {
+    int rc = launch_fill_i32(s->domctl, 0, 4, s->stream);
+    return rc ? rc : launch_fill_i32(s->domctl, 1, 1, s->stream);
+}
+
+unsigned long long* step_counters(glp_session* s) { return s->d_acc + (size_t)s->acc_rows * kChangeSlots; }
+
+int end_steps(glp_session* s) {
+    const int32_t rows = s->acc_rows;
+    s->acc_rows = 0;
+    return launch_end_steps(s->d_acc, rows, s->d_ring, s->d_ctr, kChangeRing, s->stream);
+}
+
+int end_step(glp_session* s, const int32_t* nbr, const int32_t* Lw, bool replayed) {
+    if (replayed || s->fctl || s->domctl)
+        // (steps with gamma > 0 use no dominant label and choose none)
+        return launch_end_step(step_counters(s), s->d_ring, s->d_ctr, kChangeRing, s->stream, s->fctl, nbr, Lw,
+                               s->g->csr.m, s->p.gamma_num == 0 ? s->domctl : nullptr);
+    return ++s->acc_rows == kAccRows ? end_steps(s) : GLP_OK;
 }
 
 // Builds the argument block of the next step (step number s->t + 1).
@@ -432,7 +453,7 @@ static StepArgs step_args(glp_session* s) {
     a.w = dg.w;
     a.n = s->n;
     a.t = s->t + 1;
-    a.changes = s->d_acc;
+    a.changes = step_counters(s);
     a.seed = s->p.seed;
     const int c = s->cur;
     switch (s->method) {
@@ -537,10 +558,7 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     if ((rc = launch_step(method, s->p.weighted != 0, s->p.gather != 0, *s->g->dev, s->hs, a, s->stream, ev)))
         return rc;
     if (s->method == Method::Layered && (rc = launch_volume(a.Lw, a.Vw, s->n, s->stream))) return rc;
-    // steps with gamma > 0 use no dominant label and choose none
-    if ((rc = launch_end_step(s->d_acc, s->d_ring, s->d_ctr, kChangeRing, s->stream, s->fctl, a.nbr, a.Lw,
-                              s->g->csr.m, s->p.gamma_num == 0 ? s->domctl : nullptr)))
-        return rc;
+    if ((rc = end_step(s, a.nbr, a.Lw, replayed))) return rc;
     if (s->method != Method::Slpa) s->cur ^= 1;
     s->t += 1;
     if (!replayed) s->at_l0 = false;
@@ -581,8 +599,13 @@ int session_step(glp_session* s, int32_t steps) {
             ev = s->ev_pool[s->ev_used++].data();
         }
         int rc = enqueue_step(s, ev);
-        if (rc != GLP_OK) return rc;
+        if (rc != GLP_OK) {
+            (void)end_steps(s);  // of the steps before it
+            return rc;
+        }
     }
+    const int rc = end_steps(s);
+    if (rc != GLP_OK) return rc;
     GLP_HIP(hipEventRecord(s->ev_stop, s->stream));
     s->pending_steps += steps;
     return GLP_OK;
@@ -629,6 +652,7 @@ int session_step_graph(glp_session* s, int32_t steps) {
     int32_t i = 0;
     if (s->at_l0) {  // the first step has launches of its own
         int rc = enqueue_step(s, nullptr);
+        if (rc == GLP_OK) rc = end_steps(s);
         if (rc != GLP_OK) return rc;
         i = 1;
     }
@@ -866,6 +890,7 @@ extern "C" int glp_session_load(glp_session* s, const void* state, size_t state_
     if (s->mem && h.t > s->p.slpa_T) return set_error(GLP_E_FORMAT, "state beyond SLPA memory");
     int rc = session_reset(s);
     if (rc != GLP_OK) return rc;
+    GLP_HIP(hipStreamSynchronize(s->stream));  // the copies below are not on the session's stream
     const int32_t* body = reinterpret_cast<const int32_t*>(static_cast<const char*>(state) + sizeof h);
     const size_t n = (size_t)s->n;
     if (s->mem) {
@@ -908,9 +933,11 @@ static int run_impl(glp_graph* g, const glp_params* p, const uint8_t* seeds, int
     if (rc != GLP_OK) return rc;
     std::unique_ptr<glp_session> guard(s);
     if (q.method == GLP_SEEDED && (rc = glp_session_set_seeds(s, seeds, s->n)) != GLP_OK) return rc;
-    for (int32_t i = 0; i < steps; ++i) {
-        if ((rc = session_step(s, 1)) != GLP_OK) return rc;
-        if (step_dump) {
+    if (!step_dump) {
+        if ((rc = session_step(s, steps)) != GLP_OK) return rc;
+    } else {
+        for (int32_t i = 0; i < steps; ++i) {
+            if ((rc = session_step(s, 1)) != GLP_OK) return rc;
             if ((rc = session_labels(s, step_dump + (size_t)i * s->n)) != GLP_OK) return rc;
         }
     }
@@ -939,7 +966,9 @@ extern "C" int glp_session_set_seeds(glp_session* s, const uint8_t* seeds, int32
     if (!s->seeds) GLP_HIP(hipMalloc(&s->seeds, std::max<size_t>((size_t)n, 1)));
     if (n > 0) GLP_HIP(hipMemcpyAsync(s->seeds, seeds, (size_t)n, hipMemcpyHostToDevice, s->stream));
     s->seeds_set = true;
-    return session_reset(s);  // synchronises the stream (the host buffer may go)
+    const int rc = session_reset(s);
+    GLP_HIP(hipStreamSynchronize(s->stream));  // the host buffer may go
+    return rc;
 }
 
 extern "C" int glp_run_seeded(glp_graph* g, const glp_params* p, const uint8_t* seeds, int32_t steps,

@@ -435,3 +435,23 @@ def test_one_launch_equals_a_launch_per_tier(kw, tuned):
         for g in graphs:
             one = gpu_steps(g, 4, **kw)
             assert_steps_equal(one, gpu_steps(g, 4, profile=True, **kw))
+
+
+@pytest.mark.parametrize("calls", [[1], [31], [32], [33], [70], [20, 0, 13, 1, 64]])
+def test_change_counts_over_many_steps(calls):
+    """The change counters of a call's steps are summed together, 32 steps at
+    a time: counts and labels for calls around that length, eager and
+    replayed, and again after a reset."""
+    g = G.Graph.planted(3000, 30, 6.0, 3.0, seed=4)
+    off, nbr, _ = g.csr()
+    total = sum(calls)
+    want = O.classic(off, nbr, total)
+    prev = np.vstack([np.arange(g.n, dtype=np.int32)[None], want[:-1]])
+    counts = (want != prev).sum(axis=1).tolist()
+    with G.Session(g) as s:
+        for replay in (False, True, False):
+            for k in calls:
+                s.step(k, graph=replay)
+            assert s.changes().tolist() == counts
+            assert np.array_equal(s.labels(), want[-1])
+            s.reset()

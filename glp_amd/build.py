@@ -19,7 +19,8 @@ ARCH = os.environ.get("GLP_OFFLOAD_ARCH", "gfx950")
 # (the tier kernels, the longest to compile, first)
 HIP_SOURCES = ["tiers_multi.hip", "tiers_classic.hip", "tiers_layered.hip", "tiers_slpa.hip", "tiers_user.hip",
                "tiers_seeded.hip", "tiers_layered_vol.hip", "tiers_first.hip", "kernels.hip", "counting.hip",
-               "session.hip", "batch.hip", "server.hip", "plan.hip", "autotune.hip", "gen_device.hip", "noalloc.hip"]
+               "session.hip", "batch.hip", "server.hip", "plan.hip", "autotune.hip", "gen_device.hip", "noalloc.hip",
+               "download.hip"]
 CPP_SOURCES = ["graph_io.cpp", "gen.cpp"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function"]

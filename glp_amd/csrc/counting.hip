@@ -1119,11 +1119,12 @@ int slpa_post(glp_session* s, int32_t kmax, int32_t* dominant, int32_t* nsets, i
     hipLaunchKernelGGL(k_slpa_post, dim3((n + 63) / 64), dim3(64), 0, s->stream, s->mem, n, rows,
                        s->p.slpa_r_num, s->p.slpa_r_den, kmax, d_dom, d_ns, d_sets);
     GLP_HIP(hipGetLastError());
-    GLP_HIP(hipStreamSynchronize(s->stream));
-    if (dominant) GLP_HIP(hipMemcpy(dominant, d_dom, (size_t)n * 4, hipMemcpyDeviceToHost));
-    if (nsets) GLP_HIP(hipMemcpy(nsets, d_ns, (size_t)n * 4, hipMemcpyDeviceToHost));
-    if (kmax > 0 && sets) GLP_HIP(hipMemcpy(sets, d_sets, (size_t)n * kmax * 4, hipMemcpyDeviceToHost));
-    return GLP_OK;
+    int rc = GLP_OK;
+    if (dominant) rc = copy_to_host(s->staging, dominant, d_dom, (size_t)n * 4, s->stream);
+    if (!rc && nsets) rc = copy_to_host(s->staging, nsets, d_ns, (size_t)n * 4, s->stream);
+    if (!rc && kmax > 0 && sets) rc = copy_to_host(s->staging, sets, d_sets, (size_t)n * kmax * 4, s->stream);
+    GLP_HIP(hipStreamSynchronize(s->stream));  // before the arrays go
+    return rc;
 }
 
 }  // namespace glp

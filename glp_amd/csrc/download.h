@@ -1,0 +1,30 @@
+// Copies of results to the caller's memory (download.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <cstddef>
+
+namespace glp {
+
+// Pinned double buffers of one worker.
+struct CopySlots {
+    char* slot[2] = {nullptr, nullptr};
+    hipEvent_t done[2] = {nullptr, nullptr};
+    size_t chunk = 0;
+    int create(size_t chunk);
+    ~CopySlots();
+};
+
+constexpr int kCopyWorkers = 4;
+// A session's buffers, made when copies repeat and kept while it lives (1 MB,
+// and 16 MB once its copies are large).
+struct Staging {
+    CopySlots small, large[kCopyWorkers];
+    bool used = false;  // a copy that could have used them was made
+};
+
+// Copies `bytes` from the device to pageable host memory after the work
+// queued on s; returns when they are there.
+int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s);
+
+}  // namespace glp

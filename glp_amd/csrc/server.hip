@@ -212,7 +212,8 @@ struct glp_server {
     hipStream_t lstream = nullptr;     // job initialisation and light jobs' steps
     hipEvent_t init_ev = nullptr;      // after the latest initialisations on lstream
     hipStream_t up_stream = nullptr;   // private graph uploads
-    hipStream_t dl_stream = nullptr;   // result copies
+    hipStream_t dl_stream = nullptr;   // result copies,
+    Staging staging;                   // and their slots (the completion thread's)
     hipStream_t add_stream = nullptr;  // glp_server_add_* and graph copies (callers' threads)
     std::mutex add_mu;
     DevicePool pool;
@@ -694,9 +695,7 @@ void glp_server::complete_loop() {
         } else {
             const int32_t n = j->rg->dg->n;
             j->result.resize((size_t)n);
-            if (n && (hipMemcpyAsync(j->result.data(), j->L[j->cur], sizeof(int32_t) * n, hipMemcpyDeviceToHost,
-                                     dl_stream) != hipSuccess ||
-                      hipStreamSynchronize(dl_stream) != hipSuccess))
+            if (copy_to_host(staging, j->result.data(), j->L[j->cur], sizeof(int32_t) * (size_t)n, dl_stream) != GLP_OK)
                 st = GLP_E_HIP;
         }
         pool.release(j->block, j->block_cap);

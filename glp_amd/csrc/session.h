@@ -2,6 +2,7 @@
 #pragma once
 
 #include "device.h"
+#include "download.h"
 
 #include <array>
 #include <vector>
@@ -61,6 +62,7 @@ struct glp_session {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     glp_timing timing{};
+    glp::Staging staging;                  // of copies to the caller
     std::vector<int64_t> host_changes;
     ~glp_session();
 };

@@ -683,3 +683,22 @@ def test_calib_random_read_runs():
     ms = G.calib_random_read(1 << 20, 1 << 22, 2)
     assert ms > 0
     assert (1 << 22) / (ms / 1e3) > 1e8   # more than 0.1 G reads/s
+
+
+# ---------------------------------------------------------------- copies out ----
+
+@pytest.mark.parametrize("n", [8191, 524287, 524288, 524289, 1 << 20, (1 << 22) - 1, 1 << 22, (1 << 22) + 1, 9000001])
+def test_label_copies_of_every_size(n):
+    """Copies of labels below, at and above each bound of the ways out
+    (2 MB plain, 16 MB one thread, chunks of 512 KB and 2 MB), the first and
+    repeated ones: an edge-less graph keeps L0."""
+    g = G.Graph.from_csr(np.zeros(n + 1, dtype=np.int32), np.zeros(0, dtype=np.int32))
+    want = np.arange(n, dtype=np.int32)
+    with G.Session(g) as s:
+        s.step(1)
+        for _ in range(3):
+            assert np.array_equal(s.labels(), want)
+    with G.Session(g, method=G.LAYERED, gamma=(1, 2)) as s:
+        s.step(1)
+        assert np.array_equal(s.volume(), np.ones(n, dtype=np.int32))
+        assert np.array_equal(s.labels(), want)

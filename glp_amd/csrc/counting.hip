@@ -73,27 +73,40 @@ __device__ __forceinline__ uint32_t cm_hash(int r, uint32_t k) {
     }
 }
 
-// Cells (row*W + column) a key touches, one entry per increment; the first
-// `rows` entries are used.  All five are computed with constant indices so
-// the array stays in registers.  Aliased rows (d = 3 or 4): row 3's hash
-// lands in row 2, and for d = 4 h3 goes into row 2 again.
-// x mod W by Lemire, Kaser and Kurz's direct remainder ("Faster remainder
-// by direct computation", 2019): with M = floor((2^64 - 1) / W) + 1, the
-// remainder of any 32-bit x is the high 64 bits of (M x mod 2^64) * W.
-__device__ __forceinline__ uint32_t cm_mod(uint32_t x, uint64_t M, uint32_t W) {
-    return (uint32_t)__umul64hi(M * (uint64_t)x, (uint64_t)W);
+// x mod W with m = floor(2^32 / W) (cm_mod_magic; W = 1: 2^32 - 1): the
+// estimate floor(x m / 2^32) is the quotient or one less, so what is left
+// after it is below 2 W.
+__device__ __forceinline__ uint32_t cm_mod(uint32_t x, uint32_t m, uint32_t W) {
+    const uint32_t r = x - __umulhi(x, m) * W;
+    return min(r, r - W);  // r - W wraps above r when r < W
 }
-__host__ __device__ inline uint64_t cm_mod_magic(uint32_t W) { return ~0ull / W + 1ull; }
+__host__ __device__ inline uint32_t cm_mod_magic(uint32_t W) { return W > 1u ? (uint32_t)((1ull << 32) / W) : ~0u; }
 
-__device__ __forceinline__ int cm_cells(uint32_t key, int rows, int W, int aliased, uint64_t M, uint32_t* cell) {
+// The cells (row * W + column) a key touches, one entry per increment, R
+// rows.  ALIASED (R = 3 or 4): row 3's hash lands in row 2, and for R = 4 h3
+// goes into row 2 again.  The hashes and remainders (multiplications at a
+// quarter rate) bound the count-min kernels, so the number of rows is a
+// template parameter, the remainder takes two multiplications, and a
+// thread's cells are kept from the sketch pass to the estimate pass.
+template <int R, bool ALIASED>
+__device__ __forceinline__ void cm_cells(uint32_t key, uint32_t W, uint32_t m, uint32_t* cell) {
+    static_assert(!ALIASED || R == 3 || R == 4, "aliasing touches three or four rows");
 #pragma unroll
-    for (int r = 0; r < 5; ++r) cell[r] = (uint32_t)r * W + cm_mod(cm_hash(r, key), M, (uint32_t)W);
-    if (aliased && (rows == 3 || rows == 4)) {
-        cell[2] -= (uint32_t)W;
-        cell[3] = cell[2];
-    }
-    return rows;
+    for (int r = 0; r < (ALIASED ? 3 : R); ++r) cell[r] = (uint32_t)r * W + cm_mod(cm_hash(r, key), m, W);
+    if constexpr (ALIASED) cell[2] -= W;
+    if constexpr (ALIASED && R == 4) cell[3] = cell[2];
 }
+
+// A key's cells, two to a word (rows * width <= 5 * 4096).
+template <int R>
+struct CmCells {
+    uint32_t w[(R + 1) / 2];
+    __device__ __forceinline__ void set(const uint32_t* c) {
+#pragma unroll
+        for (int i = 0; i < (R + 1) / 2; ++i) w[i] = c[2 * i] | (2 * i + 1 < R ? c[2 * i + 1] << 16 : 0u);
+    }
+    __device__ __forceinline__ uint32_t get(int r) const { return r & 1 ? w[r >> 1] >> 16 : w[r >> 1] & 0xffffu; }
+};
 
 constexpr int32_t kCountminSmallDeg = 16;
 constexpr int kCmSmallClasses = 5;  // lane groups of 1, 2, 4, 8, 16 for degrees 1, 2, 3-4, 5-8, 9-16
@@ -109,9 +122,9 @@ constexpr int32_t kTableLaneMaxDeg = 32;
 // sketch cell an entry c of edge i lands in ends up holding the sum, over
 // the vertex's edges j and their entries, of f_j where the entry is c; the
 // estimate is the minimum of that over edge i's entries.
-template <bool W, int G>
+template <bool W, int G, int R, bool ALIASED>
 __global__ __launch_bounds__(256) void k_countmin_small(StepArgs a, const int32_t* __restrict__ verts, int32_t nv,
-                                                       int32_t rows, int32_t width, int32_t aliased, uint64_t M) {
+                                                       uint32_t width, uint32_t m) {
     constexpr int kShift = G == 1 ? 0 : G == 2 ? 1 : G == 4 ? 2 : G == 8 ? 3 : 4;
     static_assert((1 << kShift) == G && G <= kCountminSmallDeg, "group of 1, 2, 4, 8 or 16 lanes");
     const int lane = lane_id(), ql = lane & (G - 1), g0 = lane & ~(G - 1);
@@ -129,36 +142,33 @@ __global__ __launch_bounds__(256) void k_countmin_small(StepArgs a, const int32_
         key = (uint32_t)a.L[a.nbr[b + ql]] + 1u;
         f = W ? a.w[b + ql] : 1u;
     }
-    uint32_t c[5];
-    const int k = cm_cells(key, rows, width, aliased, M, c);  // k depends on rows and aliased only
+    uint32_t c[R];
+    cm_cells<R, ALIASED>(key, width, m, c);
     // Proper rows occupy disjoint bands [r W, (r+1) W), so entry t of one
     // edge can only meet entry t of another; aliased rows put entries 1..3
-    // in one band, so those are compared crosswise.  (Loops unrolled to the
-    // 5 entries and guarded by k, so the arrays stay in registers.)
-    const bool cross = aliased && (rows == 3 || rows == 4);
+    // in one band, so those are compared crosswise.
     // edges of the wave's groups: the loop runs to the largest degree among them
     const int32_t dmax = __builtin_amdgcn_readfirstlane(
         (int32_t)wave_max_u64(live ? (uint64_t)(e - b) : 0ull));
-    uint32_t sum[5] = {0u, 0u, 0u, 0u, 0u};
+    uint32_t sum[R] = {};
     for (int jj = 0; jj < dmax; ++jj) {
         const uint32_t fj = shfl_u32(f, g0 + jj);
-        uint32_t cj[5];
+        uint32_t cj[R];
 #pragma unroll
-        for (int t = 0; t < 5; ++t) cj[t] = t < k ? shfl_u32(c[t], g0 + jj) : 0xffffffffu;
-        if (!cross) {
+        for (int t = 0; t < R; ++t) cj[t] = shfl_u32(c[t], g0 + jj);
 #pragma unroll
-            for (int t = 0; t < 5; ++t) sum[t] += t < k && cj[t] == c[t] ? fj : 0u;
-        } else {
+        for (int t = 0; t < R; ++t) {
+            if constexpr (!ALIASED) {
+                sum[t] += cj[t] == c[t] ? fj : 0u;
+            } else {
 #pragma unroll
-            for (int t = 0; t < 5; ++t)
-#pragma unroll
-                for (int t2 = 0; t2 < 5; ++t2) sum[t] += t < k && t2 < k && cj[t2] == c[t] ? fj : 0u;
+                for (int t2 = 0; t2 < R; ++t2) sum[t] += cj[t2] == c[t] ? fj : 0u;
+            }
         }
     }
     uint32_t est = 0xffffffffu;
 #pragma unroll
-    for (int t = 0; t < 5; ++t)
-        if (t < k) est = min(est, sum[t]);
+    for (int t = 0; t < R; ++t) est = min(est, sum[t]);
     uint64_t best = live ? pack_score((int32_t)min(est, 0x7fffffffu), key) : 0ull;
 #pragma unroll
     for (int d = G / 2; d >= 1; d >>= 1) best = max_u64(best, shfl_u64(best, lane ^ d));
@@ -172,28 +182,6 @@ __global__ __launch_bounds__(256) void k_countmin_small(StepArgs a, const int32_
     const unsigned long long bal = __ballot(changed);
     if (lane == 0 && bal)
         atomicAdd(&a.changes[blockIdx.x & (kChangeSlots - 1)], (unsigned long long)__popcll(bal));
-}
-
-// One launch of k_countmin_small over n listed vertices of lane-group class
-// gi (groups of 1 << gi lanes).
-template <int G>
-static void launch_countmin_small_g(bool w, const StepArgs& a, const int32_t* verts, int32_t n, int32_t rows,
-                                    int32_t width, int32_t aliased, uint64_t M, hipStream_t s) {
-    const unsigned grid = (unsigned)(((int64_t)n * G + 255) / 256);
-    if (w) hipLaunchKernelGGL((k_countmin_small<true, G>), dim3(grid), dim3(256), 0, s, a, verts, n, rows, width,
-                              aliased, M);
-    else hipLaunchKernelGGL((k_countmin_small<false, G>), dim3(grid), dim3(256), 0, s, a, verts, n, rows, width,
-                            aliased, M);
-}
-static void launch_countmin_small(int gi, bool w, const StepArgs& a, const int32_t* verts, int32_t n, int32_t rows,
-                                  int32_t width, int32_t aliased, uint64_t M, hipStream_t s) {
-    switch (gi) {
-        case 0: launch_countmin_small_g<1>(w, a, verts, n, rows, width, aliased, M, s); break;
-        case 1: launch_countmin_small_g<2>(w, a, verts, n, rows, width, aliased, M, s); break;
-        case 2: launch_countmin_small_g<4>(w, a, verts, n, rows, width, aliased, M, s); break;
-        case 3: launch_countmin_small_g<8>(w, a, verts, n, rows, width, aliased, M, s); break;
-        default: launch_countmin_small_g<16>(w, a, verts, n, rows, width, aliased, M, s); break;
-    }
 }
 
 // Vertices without edges keep their label.
@@ -225,12 +213,12 @@ __device__ __forceinline__ void cm_load_batch(const StepArgs& a, int32_t j, int3
 
 // Vertex verts[blockIdx.x], the sketch in LDS (NT = 64: degrees up to
 // kCountminWaveMaxDeg; NT = 256: up to kCountminMidDeg; NT = 1024: up to
-// kCountminHubDeg).  A thread's keys (at most KB of them) stay in registers
-// from the sketch pass to the estimate pass, so each neighbour label is read
-// once.
-template <bool W, int NT>
-__global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __restrict__ verts, int32_t rows,
-                                                 int32_t width, int32_t aliased, uint64_t M) {
+// kCountminHubDeg).  A thread's keys (at most KB of them) and their cells stay
+// in registers from the sketch pass to the estimate pass, so each neighbour
+// label is read and hashed once.
+template <bool W, int NT, int R, bool ALIASED>
+__global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __restrict__ verts, uint32_t width,
+                                                 uint32_t m) {
     constexpr int KB =
         (NT == 64 ? kCountminWaveMaxDeg : NT == 256 ? kCountminMidDeg : kCountminHubDeg) / NT;
     static_assert(KB % kCmBatch == 0, "whole batches");
@@ -240,10 +228,11 @@ __global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __re
     const int32_t v = verts[blockIdx.x];
     const int32_t b = a.off[v], e = a.off[v + 1];
     const int32_t last = e - 1;
-    const int32_t ncell = rows * width;
+    const int32_t ncell = R * (int32_t)width;
     for (int32_t i = threadIdx.x; i < ncell; i += NT) cells[i] = 0u;
     __syncthreads();
     uint32_t key[KB];
+    CmCells<R> at[KB];
 #pragma unroll
     for (int q = 0; q < KB; q += kCmBatch) {
         if (b + q * NT > last) break;  // uniform: no edges left for any thread
@@ -253,11 +242,11 @@ __global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __re
 #pragma unroll
         for (int u = 0; u < kCmBatch; ++u) {
             if (j + u * NT > last) break;
-            uint32_t c[5];
-            const int k = cm_cells(key[q + u], rows, width, aliased, M, c);
+            uint32_t c[R];
+            cm_cells<R, ALIASED>(key[q + u], width, m, c);
+            at[q + u].set(c);
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (i < k) atomicAdd(&cells[c[i]], f[u]);
+            for (int i = 0; i < R; ++i) atomicAdd(&cells[c[i]], f[u]);
         }
     }
     __syncthreads();
@@ -269,12 +258,9 @@ __global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __re
 #pragma unroll
         for (int u = 0; u < kCmBatch; ++u) {
             if (j + u * NT > last) break;
-            uint32_t c[5];
-            const int k = cm_cells(key[q + u], rows, width, aliased, M, c);
             uint32_t est = 0xffffffffu;
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (i < k) est = min(est, cells[c[i]]);
+            for (int i = 0; i < R; ++i) est = min(est, cells[at[q + u].get(i)]);
             best = max_u64(best, pack_score((int32_t)min(est, 0x7fffffffu), key[q + u]));
         }
     }
@@ -293,6 +279,86 @@ __global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __re
     }
 }
 
+// NV vertices of `verts` (degrees up to 64 EPL) per wavefront, one after
+// another in one sketch: the loads of all of them are issued before any is
+// counted, and a vertex's edges clear the cells they touched.  One vertex per
+// wavefront spent its time in three dependent loads and in clearing the
+// sketch (R-MAT scale 21, 3 x 200, degrees 17-1024: 210 us a step, now 192).
+constexpr int kCmVerts = 4;
+template <bool W, int EPL, int R, bool ALIASED>
+__global__ __launch_bounds__(64) void k_countmin_few(StepArgs a, const int32_t* __restrict__ verts, int32_t nv,
+                                                     uint32_t width, uint32_t m) {
+    extern __shared__ uint32_t cells[];
+    const int lane = lane_id();
+    const int32_t i0 = (int32_t)blockIdx.x * kCmVerts;
+    int32_t v[kCmVerts], b[kCmVerts], e[kCmVerts], old[kCmVerts];
+#pragma unroll
+    for (int k = 0; k < kCmVerts; ++k) v[k] = verts[min(i0 + k, nv - 1)];
+#pragma unroll
+    for (int k = 0; k < kCmVerts; ++k) {
+        b[k] = a.off[v[k]];
+        e[k] = a.off[v[k] + 1];
+        old[k] = a.keep[v[k]];
+    }
+    const int32_t ncell = R * (int32_t)width;
+    for (int32_t i = lane; i < ncell; i += 64) cells[i] = 0u;
+    // (clamped to the last edge; every vertex here has edges)
+    uint32_t key[kCmVerts][EPL], f[kCmVerts][EPL];
+#pragma unroll
+    for (int k = 0; k < kCmVerts; ++k)
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+            const int32_t j = min(b[k] + lane + 64 * i, e[k] - 1);
+            key[k][i] = (uint32_t)a.nbr[j];
+            f[k][i] = W ? a.w[j] : 1u;
+        }
+#pragma unroll
+    for (int k = 0; k < kCmVerts; ++k)
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) key[k][i] = (uint32_t)a.L[key[k][i]] + 1u;
+    uint32_t nch = 0u;
+#pragma unroll
+    for (int k = 0; k < kCmVerts; ++k) {
+        if (i0 + k >= nv) break;  // wave-uniform
+        CmCells<R> at[EPL];
+        wave_lds_sync();  // the cells are clear
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+            if (64 * i >= e[k] - b[k]) break;  // wave-uniform
+            uint32_t c[R];
+            cm_cells<R, ALIASED>(key[k][i], width, m, c);
+            at[i].set(c);
+            if (b[k] + lane + 64 * i < e[k]) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) atomicAdd(&cells[c[r]], f[k][i]);
+            }
+        }
+        wave_lds_sync();
+        uint64_t best = 0ull;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+            if (64 * i >= e[k] - b[k]) break;
+            uint32_t est = 0xffffffffu;
+#pragma unroll
+            for (int r = 0; r < R; ++r) est = min(est, cells[at[i].get(r)]);
+            // (a lane past the last edge repeats that edge's estimate)
+            best = max_u64(best, pack_score((int32_t)min(est, 0x7fffffffu), key[k][i]));
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+            if (64 * i >= e[k] - b[k]) break;
+#pragma unroll
+            for (int r = 0; r < R; ++r) cells[at[i].get(r)] = 0u;
+        }
+        best = wave_max_u64(best);
+        const int32_t nl = packed_label(best);
+        if (lane == 0) a.Lw[v[k]] = nl;
+        nch += nl != old[k] ? 1u : 0u;
+    }
+    if (lane == 0 && nch) atomicAdd(&a.changes[blockIdx.x & (kChangeSlots - 1)], (unsigned long long)nch);
+}
+
 // Count-min hubs (degree above kCountminHubDeg): workgroup i takes chunk
 // chunks[i] = (hub slot h, first edge of the chunk within the hub's edges),
 // kCountminChunk edges.  `sketch` holds rows * width cells per hub and
@@ -302,18 +368,17 @@ __global__ __launch_bounds__(NT) void k_countmin(StepArgs a, const int32_t* __re
 // sketch pass leaves each edge's key in `keys` (kCountminChunk slots per
 // chunk, in edge order), which the estimate pass reads back in order instead
 // of gathering the labels again.
-template <bool W>
+template <bool W, int R, bool ALIASED>
 __global__ __launch_bounds__(1024) void k_countmin_hub_sketch(StepArgs a, const int32_t* __restrict__ hubs,
                                                               const int2* __restrict__ chunks,
                                                               uint32_t* __restrict__ sketch,
-                                                              uint32_t* __restrict__ keys, int32_t rows,
-                                                              int32_t width, int32_t aliased, uint64_t M) {
+                                                              uint32_t* __restrict__ keys, uint32_t width, uint32_t m) {
     extern __shared__ uint32_t cells[];
     const int2 ch = chunks[blockIdx.x];
     const int32_t v = hubs[ch.x];
     const int32_t b = a.off[v] + ch.y, e = min(a.off[v + 1], b + kCountminChunk);
     const int32_t last = e - 1;
-    const int32_t ncell = rows * width;
+    const int32_t ncell = R * (int32_t)width;
     for (int32_t i = threadIdx.x; i < ncell; i += 1024) cells[i] = 0u;
     __syncthreads();
     uint32_t* ck = keys + (size_t)blockIdx.x * kCountminChunk;  // ck[j - b]: edge j's key
@@ -324,11 +389,10 @@ __global__ __launch_bounds__(1024) void k_countmin_hub_sketch(StepArgs a, const 
         for (int u = 0; u < kCmBatch; ++u) {
             if (j + u * 1024 > last) break;
             ck[j - b + u * 1024] = key[u];
-            uint32_t c[5];
-            const int k = cm_cells(key[u], rows, width, aliased, M, c);
+            uint32_t c[R];
+            cm_cells<R, ALIASED>(key[u], width, m, c);
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (i < k) atomicAdd(&cells[c[i]], f[u]);
+            for (int i = 0; i < R; ++i) atomicAdd(&cells[c[i]], f[u]);
         }
     }
     __syncthreads();
@@ -339,12 +403,12 @@ __global__ __launch_bounds__(1024) void k_countmin_hub_sketch(StepArgs a, const 
     }
 }
 
+template <int R, bool ALIASED>
 __global__ __launch_bounds__(1024) void k_countmin_hub_est(StepArgs a, const int32_t* __restrict__ hubs,
                                                            const int2* __restrict__ chunks,
                                                            const uint32_t* __restrict__ sketch,
                                                            const uint32_t* __restrict__ keys,
-                                                           unsigned long long* __restrict__ best_out, int32_t rows,
-                                                           int32_t width, int32_t aliased, uint64_t M) {
+                                                           unsigned long long* __restrict__ best_out, uint32_t width, uint32_t m) {
     extern __shared__ uint32_t cells[];
     __shared__ unsigned long long s_best[16];
     const int lane = lane_id();
@@ -352,7 +416,7 @@ __global__ __launch_bounds__(1024) void k_countmin_hub_est(StepArgs a, const int
     const int32_t v = hubs[ch.x];
     const int32_t b = a.off[v] + ch.y, e = min(a.off[v + 1], b + kCountminChunk);
     const int32_t last = e - 1;
-    const int32_t ncell = rows * width;
+    const int32_t ncell = R * (int32_t)width;
     const uint32_t* hs = sketch + (size_t)ch.x * ncell;
     for (int32_t i = threadIdx.x; i < ncell; i += 1024) cells[i] = hs[i];
     __syncthreads();
@@ -365,12 +429,11 @@ __global__ __launch_bounds__(1024) void k_countmin_hub_est(StepArgs a, const int
 #pragma unroll
         for (int u = 0; u < kCmBatch; ++u) {
             if (j + u * 1024 > last) break;
-            uint32_t c[5];
-            const int k = cm_cells(key[u], rows, width, aliased, M, c);
+            uint32_t c[R];
+            cm_cells<R, ALIASED>(key[u], width, m, c);
             uint32_t est = 0xffffffffu;
 #pragma unroll
-            for (int i = 0; i < 5; ++i)
-                if (i < k) est = min(est, cells[c[i]]);
+            for (int i = 0; i < R; ++i) est = min(est, cells[c[i]]);
             best = max_u64(best, pack_score((int32_t)min(est, 0x7fffffffu), key[u]));
         }
     }
@@ -886,25 +949,36 @@ __global__ __launch_bounds__(64) void k_table(StepArgs a, int32_t cap) {
         atomicAdd(&a.changes[blockIdx.x & (kChangeSlots - 1)], (unsigned long long)__popcll(bal));
 }
 
+template <int R, bool ALIASED>
+static void set_countmin_limits() {
+    auto set = [](const void* f) {
+        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 5 * 4096 * 4);
+    };
+    set((const void*)k_countmin<false, 64, R, ALIASED>);
+    set((const void*)k_countmin<true, 64, R, ALIASED>);
+    set((const void*)k_countmin_few<false, 1, R, ALIASED>);
+    set((const void*)k_countmin_few<true, 1, R, ALIASED>);
+    set((const void*)k_countmin_few<false, 4, R, ALIASED>);
+    set((const void*)k_countmin_few<true, 4, R, ALIASED>);
+    set((const void*)k_countmin<false, 256, R, ALIASED>);
+    set((const void*)k_countmin<true, 256, R, ALIASED>);
+    set((const void*)k_countmin<false, 1024, R, ALIASED>);
+    set((const void*)k_countmin<true, 1024, R, ALIASED>);
+    set((const void*)k_countmin_hub_sketch<false, R, ALIASED>);
+    set((const void*)k_countmin_hub_sketch<true, R, ALIASED>);
+    set((const void*)k_countmin_hub_est<R, ALIASED>);
+}
 // k_countmin takes rows * width * 4 bytes of dynamic LDS, up to 5 * 4096 * 4
 // = 80 KB (the limits check_params enforces), above the 64 KB a launch gets
 // without the attribute; k_table takes at most 64 * 2 * 64 * 4 = 32 KB.
 void init_counting_kernels() {
-    const int lim = 5 * 4096 * 4;
-    (void)hipFuncSetAttribute((const void*)k_countmin<false, 64>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin<true, 64>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin<false, 256>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin<true, 256>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin<false, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin<true, 1024>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin_hub_sketch<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin_hub_sketch<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    (void)hipFuncSetAttribute((const void*)k_countmin_hub_est, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
+    set_countmin_limits<1, false>();
+    set_countmin_limits<2, false>();
+    set_countmin_limits<3, false>();
+    set_countmin_limits<4, false>();
+    set_countmin_limits<5, false>();
+    set_countmin_limits<3, true>();
+    set_countmin_limits<4, true>();
 }
 
 // The counting methods' vertex lists (built once per session), in one
@@ -937,6 +1011,7 @@ int counting_wide_list(glp_session* s) {
     for (int32_t h = 0; h < (int32_t)hubs.size(); ++h)
         for (int32_t c0 = 0; c0 < deg(hubs[h]); c0 += kCountminChunk) chunks.push_back(make_int2(h, c0));
     s->nmid = (int32_t)wide.size();
+    for (int32_t v : wide) ++s->nmid_g[deg(v) > 256 ? 0 : deg(v) > 64 ? 1 : 2];
     s->ncm256 = (int32_t)big.size();
     big.insert(big.end(), big1024.begin(), big1024.end());
     s->nwide = (int32_t)big.size();
@@ -973,6 +1048,71 @@ int counting_wide_list(glp_session* s) {
     return GLP_OK;
 }
 
+// The count-min launches of a step.
+template <bool W, int R, bool ALIASED>
+static void countmin_rows(glp_session* s, const StepArgs& a) {
+    const uint32_t wd = (uint32_t)s->p.cm_width, m = cm_mod_magic(wd);
+    const size_t lds = (size_t)R * wd * 4;
+    const hipStream_t st = s->stream;
+    const int32_t* small = s->wide + s->nmid + s->nwide + s->ncmhub;
+    // lane groups of 1, 2, 4, 8 and 16
+    const int32_t* n = s->nsmall_g;
+    auto blocks = [](int64_t items) { return dim3((unsigned)((items + 255) / 256)); };
+    const int32_t* at = small;
+    if (n[0]) hipLaunchKernelGGL((k_countmin_small<W, 1, R, ALIASED>), blocks(n[0]), dim3(256), 0, st, a, at, n[0], wd, m);
+    at += n[0];
+    if (n[1])
+        hipLaunchKernelGGL((k_countmin_small<W, 2, R, ALIASED>), blocks(2ll * n[1]), dim3(256), 0, st, a, at, n[1], wd, m);
+    at += n[1];
+    if (n[2])
+        hipLaunchKernelGGL((k_countmin_small<W, 4, R, ALIASED>), blocks(4ll * n[2]), dim3(256), 0, st, a, at, n[2], wd, m);
+    at += n[2];
+    if (n[3])
+        hipLaunchKernelGGL((k_countmin_small<W, 8, R, ALIASED>), blocks(8ll * n[3]), dim3(256), 0, st, a, at, n[3], wd, m);
+    at += n[3];
+    if (n[4])
+        hipLaunchKernelGGL((k_countmin_small<W, 16, R, ALIASED>), blocks(16ll * n[4]), dim3(256), 0, st, a, at, n[4], wd, m);
+    if (s->niso > 0) hipLaunchKernelGGL(k_countmin_keep, blocks(s->niso), dim3(256), 0, st, a, small + s->nsmall, s->niso);
+    // the list runs largest degree first
+    const int32_t n1024 = s->nmid_g[0], n256 = s->nmid_g[1], n64 = s->nmid_g[2];
+    auto few = [](int32_t items) { return dim3((unsigned)((items + kCmVerts - 1) / kCmVerts)); };
+    if (n1024) hipLaunchKernelGGL((k_countmin<W, 64, R, ALIASED>), dim3(n1024), dim3(64), lds, st, a, s->wide, wd, m);
+    if (n256)
+        hipLaunchKernelGGL((k_countmin_few<W, 4, R, ALIASED>), few(n256), dim3(64), lds, st, a, s->wide + n1024, n256,
+                           wd, m);
+    if (n64)
+        hipLaunchKernelGGL((k_countmin_few<W, 1, R, ALIASED>), few(n64), dim3(64), lds, st, a, s->wide + n1024 + n256,
+                           n64, wd, m);
+    if (s->ncm256 > 0)
+        hipLaunchKernelGGL((k_countmin<W, 256, R, ALIASED>), dim3(s->ncm256), dim3(256), lds, st, a, s->wide + s->nmid,
+                           wd, m);
+    if (s->nwide > s->ncm256)
+        hipLaunchKernelGGL((k_countmin<W, 1024, R, ALIASED>), dim3((unsigned)(s->nwide - s->ncm256)), dim3(1024), lds, st,
+                           a, s->wide + s->nmid + s->ncm256, wd, m);
+    if (s->ncmhub > 0) {
+        const int32_t* hubs = s->wide + s->nmid + s->nwide;
+        const dim3 grid((unsigned)s->ncmchunk);
+        hipLaunchKernelGGL((k_countmin_hub_sketch<W, R, ALIASED>), grid, dim3(1024), lds, st, a, hubs, s->cm_chunks,
+                           s->cm_sketch, s->cm_keys, wd, m);
+        hipLaunchKernelGGL((k_countmin_hub_est<R, ALIASED>), grid, dim3(1024), lds, st, a, hubs, s->cm_chunks,
+                           s->cm_sketch, s->cm_keys, s->cm_best, wd, m);
+        hipLaunchKernelGGL(k_countmin_hub_final, dim3(s->ncmhub), dim3(256), 0, st, a, hubs, s->cm_sketch, s->cm_best,
+                           (int32_t)(R * wd));
+    }
+}
+template <bool W>
+static void countmin_step(glp_session* s, const StepArgs& a) {
+    // aliasing touches rows 2 and 3 of three or four
+    const bool al = s->p.cm_aliased != 0;
+    switch (s->p.cm_rows) {
+        case 1: return countmin_rows<W, 1, false>(s, a);
+        case 2: return countmin_rows<W, 2, false>(s, a);
+        case 3: return al ? countmin_rows<W, 3, true>(s, a) : countmin_rows<W, 3, false>(s, a);
+        case 4: return al ? countmin_rows<W, 4, true>(s, a) : countmin_rows<W, 4, false>(s, a);
+        default: return countmin_rows<W, 5, false>(s, a);
+    }
+}
+
 int enqueue_counting_step(glp_session* s) {
     const DeviceGraph& dg = *s->g->dev;
     StepArgs a{};
@@ -988,50 +1128,8 @@ int enqueue_counting_step(glp_session* s) {
     const bool w = s->p.weighted != 0;
     if (s->n > 0) {
         if (s->p.method == GLP_COUNTMIN) {
-            const size_t lds = (size_t)s->p.cm_rows * s->p.cm_width * 4;
-            const int32_t r = s->p.cm_rows, wd = s->p.cm_width, al = s->p.cm_aliased;
-            const uint64_t M = cm_mod_magic((uint32_t)wd);
-            const int32_t* small = s->wide + s->nmid + s->nwide + s->ncmhub;
-            for (int gi = 0, at = 0; gi < kCmSmallClasses; at += s->nsmall_g[gi], ++gi)
-                if (s->nsmall_g[gi] > 0)
-                    launch_countmin_small(gi, w, a, small + at, s->nsmall_g[gi], r, wd, al, M, s->stream);
-            if (s->niso > 0)
-                hipLaunchKernelGGL(k_countmin_keep, dim3((unsigned)((s->niso + 255) / 256)), dim3(256), 0, s->stream,
-                                   a, small + s->nsmall, s->niso);
-            if (s->nmid > 0) {
-                if (w) hipLaunchKernelGGL((k_countmin<true, 64>), dim3(s->nmid), dim3(64), lds, s->stream, a,
-                                          s->wide, r, wd, al, M);
-                else hipLaunchKernelGGL((k_countmin<false, 64>), dim3(s->nmid), dim3(64), lds, s->stream, a,
-                                        s->wide, r, wd, al, M);
-            }
-            if (s->ncm256 > 0) {
-                if (w) hipLaunchKernelGGL((k_countmin<true, 256>), dim3(s->ncm256), dim3(256), lds, s->stream,
-                                          a, s->wide + s->nmid, r, wd, al, M);
-                else hipLaunchKernelGGL((k_countmin<false, 256>), dim3(s->ncm256), dim3(256), lds, s->stream,
-                                        a, s->wide + s->nmid, r, wd, al, M);
-            }
-            if (s->nwide > s->ncm256) {
-                const unsigned g1024 = (unsigned)(s->nwide - s->ncm256);
-                const int32_t* v1024 = s->wide + s->nmid + s->ncm256;
-                if (w) hipLaunchKernelGGL((k_countmin<true, 1024>), dim3(g1024), dim3(1024), lds, s->stream,
-                                          a, v1024, r, wd, al, M);
-                else hipLaunchKernelGGL((k_countmin<false, 1024>), dim3(g1024), dim3(1024), lds, s->stream,
-                                        a, v1024, r, wd, al, M);
-            }
-            if (s->ncmhub > 0) {
-                const int32_t* hubs = s->wide + s->nmid + s->nwide;
-                const unsigned cgrid = (unsigned)s->ncmchunk;
-                if (w)
-                    hipLaunchKernelGGL((k_countmin_hub_sketch<true>), dim3(cgrid), dim3(1024), lds, s->stream, a,
-                                       hubs, s->cm_chunks, s->cm_sketch, s->cm_keys, r, wd, al, M);
-                else
-                    hipLaunchKernelGGL((k_countmin_hub_sketch<false>), dim3(cgrid), dim3(1024), lds, s->stream, a,
-                                       hubs, s->cm_chunks, s->cm_sketch, s->cm_keys, r, wd, al, M);
-                hipLaunchKernelGGL(k_countmin_hub_est, dim3(cgrid), dim3(1024), lds, s->stream, a, hubs,
-                                   s->cm_chunks, s->cm_sketch, s->cm_keys, s->cm_best, r, wd, al, M);
-                hipLaunchKernelGGL(k_countmin_hub_final, dim3(s->ncmhub), dim3(256), 0, s->stream, a, hubs,
-                                   s->cm_sketch, s->cm_best, r * wd);
-            }
+            if (w) countmin_step<true>(s, a);
+            else countmin_step<false>(s, a);
         } else {
             const size_t lds = (size_t)64 * 2 * s->p.table_cap * 4;
             const unsigned grid = (unsigned)((s->n + 63) / 64);

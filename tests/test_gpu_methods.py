@@ -702,3 +702,16 @@ def test_label_copies_of_every_size(n):
         s.step(1)
         assert np.array_equal(s.volume(), np.ones(n, dtype=np.int32))
         assert np.array_equal(s.labels(), want)
+
+
+@pytest.mark.parametrize("rows,aliased", [(1, 0), (2, 0), (3, 0), (3, 1), (4, 0), (4, 1), (5, 0), (5, 1)])
+@pytest.mark.parametrize("width", [1, 2, 37, 4095])
+def test_countmin_rows_and_widths(rmat13w, rows, aliased, width):
+    """Each number of rows has kernels of its own: all of them, proper and
+    aliased, with the remainder's smallest and largest widths, weighted."""
+    g, (off, nbr, w) = rmat13w
+    labels, _ = G.run(g, 2, method=G.COUNTMIN, cm_rows=rows, cm_width=width, cm_aliased=aliased, weighted=True)
+    prev = np.arange(len(off) - 1, dtype=np.int32)
+    for _ in range(2):
+        prev = O.countmin_step(off, nbr, prev, rows, width, aliased, w=w)
+    assert np.array_equal(labels, prev)

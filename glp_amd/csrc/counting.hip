@@ -465,24 +465,6 @@ __global__ __launch_bounds__(256) void k_countmin_hub_final(StepArgs a, const in
     }
 }
 
-// Min over the 64 lanes, every lane active, without the LDS pipe: DPP moves
-// within each row of 16 (quad pairs, quad with mirror quad, half-row with
-// half-row), then the four rows' minima by readlane.  A lane whose DPP
-// source is unavailable keeps its own value (old = x).  The full-table
-// case of k_table_wave takes one per edge, in series, so its latency sets
-// the wide tables' speed.
-__device__ __forceinline__ uint32_t wave_min_dpp(uint32_t x) {
-    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
-    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
-    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x141, 0xf, 0xf, false));  // row half-mirror
-    x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x140, 0xf, 0xf, false));  // row mirror
-    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)x, 0);
-    const uint32_t r1 = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
-    const uint32_t r2 = (uint32_t)__builtin_amdgcn_readlane((int)x, 32);
-    const uint32_t r3 = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
-    return min(min(r0, r1), min(r2, r3));
-}
-
 // A wide table: slot i is lane i's (K, A).  A slot's count is A - off, so a
 // drop of every slot is one scalar addition to `off`; `fr` holds the free
 // slots (key 0).  Lanes >= cap hold the key 0xffffffff, which no edge carries
@@ -684,7 +666,7 @@ __device__ __forceinline__ void table_chunk(uint32_t key, uint64_t all, uint64_t
         if ((dead_o | dead_n) == 0ull) {
             const uint32_t lo_o = __builtin_amdgcn_inverse_ballot_w64(live_o) ? co : 0xffffffffu;
             const uint32_t lo_n = __builtin_amdgcn_inverse_ballot_w64(live_n) ? cn : 0xffffffffu;
-            const uint32_t cmin = wave_min_dpp(min(lo_o, lo_n)) - off;  // >= 2
+            const uint32_t cmin = wave_min_u32(min(lo_o, lo_n)) - off;  // >= 2
             const uint32_t skip = min(cmin - 1u, (uint32_t)__popcll(miss));
             for (uint32_t k = 0u; k < skip; ++k) miss &= miss - 1ull;
             off += skip;
@@ -759,7 +741,7 @@ __device__ __forceinline__ void table_edge(uint32_t kk, uint32_t ff, WideTable& 
         t.fr = gone;
         t.K = __builtin_amdgcn_inverse_ballot_w64(gone) ? 0u : t.K;
     } else {
-        const uint32_t least = wave_min_dpp(t.A);  // off + the smallest counter
+        const uint32_t least = wave_min_u32(t.A);  // off + the smallest counter
         const uint32_t left = ff - (least - t.off);
         t.off = least;
         t.fr = __ballot(t.A == least);

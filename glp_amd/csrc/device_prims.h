@@ -1,5 +1,6 @@
-// Wave64 / LDS primitives for gfx950 (CDNA4).  All cross-lane traffic goes
-// through ds_bpermute; a wavefront is 64 lanes.
+// Wave64 / LDS primitives for gfx950 (CDNA4); a wavefront is 64 lanes.
+// Shuffles to any lane go through ds_bpermute, reductions and scans over DPP
+// moves and readlanes.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -33,23 +34,52 @@ __device__ __forceinline__ T ld_stream(const T* p) {
     return __builtin_nontemporal_load(p);
 }
 
-// Max over the 64 lanes; every lane receives the result.
-__device__ __forceinline__ uint64_t wave_max_u64(uint64_t x) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) x = max_u64(x, shfl_u64(x, lane ^ d));
-    return x;
+// Reductions over the 64 lanes, every lane active; every lane receives the
+// result.  DPP moves combine each row of 16 (quad pairs, quad with mirror
+// quad, half-row with half-row), readlanes the four rows: about 15 vector and
+// scalar instructions, where a shuffle tree waits for the LDS pipe six times
+// (twelve for 64 bits).  (A lane whose DPP source is unavailable keeps its
+// own value: old = x.)
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xf, 0xf, false);
+}
+template <class F>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t x, F f) {
+    x = f(x, dpp_u32<0xB1>(x));   // quad_perm [1,0,3,2]
+    x = f(x, dpp_u32<0x4E>(x));   // quad_perm [2,3,0,1]
+    x = f(x, dpp_u32<0x141>(x));  // row half-mirror
+    x = f(x, dpp_u32<0x140>(x));  // row mirror
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)x, 0);
+    const uint32_t r1 = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
+    const uint32_t r2 = (uint32_t)__builtin_amdgcn_readlane((int)x, 32);
+    const uint32_t r3 = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
+    return f(f(r0, r1), f(r2, r3));
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) x = min(x, shfl_u32(x, lane ^ d));
-    return x;
+    return wave_reduce(x, [](uint32_t a, uint32_t b) { return min(a, b); });
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
+    return wave_reduce(x, [](uint32_t a, uint32_t b) { return max(a, b); });
 }
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) x += shfl_u32(x, lane ^ d);
+    return wave_reduce(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint64_t wave_max_u64(uint64_t x) {
+    const uint32_t hi = wave_max_u32((uint32_t)(x >> 32));
+    const uint32_t lo = wave_max_u32((uint32_t)(x >> 32) == hi ? (uint32_t)x : 0u);
+    return ((uint64_t)hi << 32) | lo;
+}
+// Inclusive prefix sum over the 64 lanes, every lane active: within rows by
+// row shifts (a lane without a source adds 0), then each row's last lane into
+// the next row, and lane 31 into the upper half.
+__device__ __forceinline__ int32_t wave_incl_sum(int32_t x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
     return x;
 }
 

@@ -924,16 +924,6 @@ __device__ __forceinline__ void block_body(const StepArgs& a, const int32_t* __r
 // at most 3/4 part_keys distinct labels (its table of 2 part_keys slots takes
 // part_keys before halving) even when every neighbour shows a different
 // label; once labels converge most buckets are empty and exit at once.
-// Inclusive prefix sum over the 64 lanes of a wave.
-__device__ __forceinline__ int32_t wave_incl_sum(int32_t x) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int32_t y = shfl_i32(x, lane >= d ? lane - d : lane);
-        if (lane >= d) x += y;
-    }
-    return x;
-}
 // Exclusive prefix of x over a workgroup of NT threads; *total = the sum.
 template <int NT = 256>
 __device__ __forceinline__ int32_t block_excl_sum(int32_t x, int32_t* total) {

@@ -307,20 +307,29 @@ struct PackedLds {
     unsigned long long best[64];         // per vertex slot: best packed score
 };
 
+// Every lane's first and owner: a vertex's last edge lane takes a mark from
+// it (pushed by ds_permute; lanes nobody pushes to get 0), and an edge lane's
+// owner is the number of marks below it.  With vertices of no edges, that
+// counts the ones with edges, whose slots are looked up by rank.
 __device__ __forceinline__ void packed_segments(PackedGroup& s, int lane) {
-    s.vb = shfl_i32(s.ve, lane > 0 ? lane - 1 : 0);
-    if (lane == 0) s.vb = 0;
-    s.nE = shfl_i32(s.ve, s.vc - 1);
-    // owner: smallest vertex slot i with ve_i > lane
-    int lo = 0, hi = s.vc - 1;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const int mid = (lo + hi) >> 1;
-        const int32_t vm = shfl_i32(s.ve, mid);
-        if (vm <= lane) lo = min(mid + 1, hi);
-        else hi = mid;
+    s.vb = __builtin_amdgcn_update_dpp(0, s.ve, 0x138, 0xf, 0xf, false);  // wave_shr:1
+    s.nE = __builtin_amdgcn_readlane(s.ve, __builtin_amdgcn_readfirstlane(s.vc) - 1);
+    // (a lane without a vertex, and one before the first edge, marks lane 63,
+    // which no lane is above)
+    const unsigned long long ends =
+        __ballot(__builtin_amdgcn_ds_permute(((s.ve - 1) & 63) << 2, 1) != 0);
+    auto below = [](unsigned long long m) {
+        return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    };
+    s.own = below(ends);
+    const bool has = lane < s.vc && s.ve > s.vb;
+    if (__ballot(lane < s.vc && !has) != 0ull) {  // wave-uniform
+        // (fewer than 64 vertices have edges, so lane 63 is free for the rest)
+        const int32_t rank = below(__ballot(has));
+        const int32_t slot = __builtin_amdgcn_ds_permute((has ? rank : 63) << 2, lane);
+        s.own = shfl_i32(slot, s.own);
     }
-    s.own = lo;
+    s.own = min(s.own, s.vc - 1);  // lanes past the group's edges
 }
 
 // Loads of a group with vc >= 1 vertices and nE >= 1 edges: indices past the

@@ -245,13 +245,15 @@ int launch_frontier_gather(const StepArgs& a, int64_t m, int32_t* adj, const Inv
                            void* push, hipStream_t s);
 int launch_fill_i32(int32_t* p, int32_t value, int64_t count, hipStream_t s);
 int launch_iota(int32_t* p, int64_t count, hipStream_t s);
-// LV[u] = {L[u], V[L[u]]} for u < n (layered LP's records for LayeredVol).
-int launch_label_volumes(const int32_t* L, const int32_t* V, int2* LV, int32_t n, hipStream_t s);
-// V[l] += #{v < n : L[v] = l} (layered LP's volume of the written labels;
-// V zeroed first).
-int launch_volume(const int32_t* L, int32_t* V, int32_t n, hipStream_t s);
-// dom_ctl (may be null): chooses the next step's dominant label from the
-// labels dom_L over the m > 0 edges of dom_nbr, {1 when there is none, 0, it}.
+// Layered LP's volume V(l) = #{v < n : L[v] = l} of the labels a step writes:
+// before the step, V is cleared but for the edge-less vertices that show
+// their own id (L: any label buffer); after it, the others are counted.
+int launch_volume_init(const int32_t* off, const int32_t* L, int32_t* V, int32_t n, hipStream_t s);
+int launch_volume(const int32_t* off, const int32_t* L, int32_t* V, int32_t n, hipStream_t s);
+// launch_volume_init of Vw together with LayeredVol's records
+// LV[u] = {L[u], Vr[L[u]]} for u < n.
+int launch_label_volumes(const int32_t* off, const int32_t* L, const int32_t* Vr, int2* LV, int32_t* Vw, int32_t n,
+                         hipStream_t s);
 // Sums `rows` rows of kChangeSlots counters into the ring, one step each, and
 // clears them.
 int launch_end_steps(unsigned long long* acc, int32_t rows, unsigned long long* ring, int32_t* step_ctr,
@@ -273,6 +275,8 @@ struct ResetArgs {
     int32_t* domctl;          // dominant label control words: none
 };
 int launch_reset(const ResetArgs& r, hipStream_t s);
+// dom_ctl (may be null): chooses the next step's dominant label from the
+// labels dom_L over the m > 0 edges of dom_nbr, {1 when there is none, 0, it}.
 int launch_end_step(unsigned long long* acc, unsigned long long* ring, int32_t* step_ctr,
                     int32_t ring_size, hipStream_t s, int32_t* fctl = nullptr, const int32_t* dom_nbr = nullptr,
                     const int32_t* dom_L = nullptr, int64_t dom_m = 0, int32_t* dom_ctl = nullptr);
@@ -295,16 +299,17 @@ inline int launch_zero_bytes(void* p, int64_t count, hipStream_t s) {
 struct VolumeJob {
     const int32_t* L;
     int32_t* V;
+    const int32_t* off;
+    int2* LV;
     int32_t n;
     int32_t pad;
-    int2* LV;
 };
 // Workgroups a job of n vertices needs in the folded zero (and records) and
 // volume launches.
 void volume_job_blocks(int32_t n, int32_t* zero_blocks, int32_t* volume_blocks);
-// kVolumeZero: V = 0 for every job (before the tiers); kVolumeRecords:
-// LV[u] = {L[u], V[L[u]]} (before the tiers); kVolumeFill: V += histogram
-// of L (after them).  cum: nj + 1 prefix sums of the job's workgroups;
+// kVolumeZero: launch_volume_init's V for every job (before the tiers);
+// kVolumeRecords: LV[u] = {L[u], V[L[u]]} (before the tiers); kVolumeFill:
+// launch_volume's counts (after them).  cum: nj + 1 prefix sums of the job's workgroups;
 // grid = cum[nj].
 enum VolumeMode { kVolumeZero, kVolumeRecords, kVolumeFill };
 int launch_multi_volume(VolumeMode mode, const VolumeJob* jobs, const int32_t* cum, int32_t nj, int32_t grid,

@@ -295,23 +295,34 @@ __global__ void k_fill_i32(int32_t* p, int32_t value, int64_t count) {
 // vertices in an LDS table of (label+1, count) slots (each wave first merges
 // its row's first label) and flushes one atomic per distinct label; a label
 // that finds no slot within kVolProbe probes goes to global memory directly.
-constexpr int kVolThreads = 256;
+// Edge-less vertices keep their label for ever, and in a power-law graph they
+// are half of all vertices, each with a label of its own: the pass that
+// clears V gives them their 1, and only the others are counted here.  A
+// chunk of 16,384 keeps the global atomics few (8,192: more of them than the
+// extra workgroups bring); 16 waves share it, which hides the latency of the
+// table's probes.  R-MAT scale 22: 137 us with every vertex counted by
+// 256-thread workgroups, 118 without the edge-less ones, 108 with 1,024
+// threads; tens of jobs of up to 65,536 vertices in one launch: 105, 82, 40.
+constexpr int kVolThreads = 1024;
 constexpr int kVolChunk = 16384;
 constexpr uint32_t kVolSlots = 2048;
 constexpr int kVolProbe = 8;
-__device__ __forceinline__ void volume_body(const int32_t* __restrict__ L, int32_t* __restrict__ V,
-                                            int32_t n, uint32_t blk) {
+constexpr int kVolRows = 4;  // loads in flight per lane
+__device__ __forceinline__ bool counted_alone(const int32_t* __restrict__ off, int64_t v, int32_t label) {
+    return label == (int32_t)v && off[v] == off[v + 1];
+}
+__device__ __forceinline__ void volume_body(const int32_t* __restrict__ off, const int32_t* __restrict__ L,
+                                            int32_t* __restrict__ V, int32_t n, uint32_t blk) {
     __shared__ unsigned long long T[kVolSlots];
     const int lane = lane_id();
     for (uint32_t i = threadIdx.x; i < kVolSlots; i += kVolThreads) T[i] = 0ull;
     __syncthreads();
     const int64_t c0 = (int64_t)blk * kVolChunk;
     const int64_t c1 = min((int64_t)n, c0 + kVolChunk);
-    for (int64_t r = c0 + (threadIdx.x & ~63); r < c1; r += kVolThreads) {  // wave-uniform rows
-        const int64_t v = r + lane;
-        int32_t l = v < c1 ? L[v] : -1;
+    auto count = [&](int32_t l) {  // one row of a wave; -1: nothing to count
         uint32_t c = 1u;
         const unsigned long long act = __ballot(l >= 0);
+        if (act == 0ull) return;
         const int first = (int)__builtin_ctzll(act);
         const int32_t lead = __builtin_amdgcn_readlane(l, first);
         const unsigned long long sm = __ballot(l == lead);
@@ -319,7 +330,7 @@ __device__ __forceinline__ void volume_body(const int32_t* __restrict__ L, int32
             if (lane == first) c = (uint32_t)__popcll(sm);
             else l = -1;  // merged into the first lane
         }
-        if (l < 0) continue;
+        if (l < 0) return;
         const uint32_t key = (uint32_t)l + 1u;
         uint32_t h = fmix32(key) & (kVolSlots - 1u);
         bool done = false;
@@ -336,6 +347,17 @@ __device__ __forceinline__ void volume_body(const int32_t* __restrict__ L, int32
             h = (h + 1u) & (kVolSlots - 1u);
         }
         if (!done) atomicAdd(&V[l], (int32_t)c);
+    };
+    for (int64_t r = c0 + (threadIdx.x & ~63); r < c1; r += kVolThreads * kVolRows) {  // wave-uniform rows
+        int32_t l[kVolRows];
+#pragma unroll
+        for (int i = 0; i < kVolRows; ++i) {
+            const int64_t at = r + i * kVolThreads + lane, v = min(at, c1 - 1);
+            const int32_t x = L[v], d = off[v + 1] - off[v];  // always loaded: no branch between the rows' loads
+            l[i] = (at >= c1) | ((d == 0) & (x == (int32_t)v)) ? -1 : x;
+        }
+#pragma unroll
+        for (int i = 0; i < kVolRows; ++i) count(l[i]);
     }
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < kVolSlots; i += kVolThreads) {
@@ -343,9 +365,10 @@ __device__ __forceinline__ void volume_body(const int32_t* __restrict__ L, int32
         if (x) atomicAdd(&V[(uint32_t)(x >> 32) - 1u], (int32_t)(uint32_t)x);
     }
 }
-__global__ __launch_bounds__(kVolThreads) void k_volume(const int32_t* __restrict__ L,
-                                                        int32_t* __restrict__ V, int32_t n) {
-    volume_body(L, V, n, blockIdx.x);
+__global__ __launch_bounds__(kVolThreads) void k_volume(const int32_t* __restrict__ off,
+                                                        const int32_t* __restrict__ L, int32_t* __restrict__ V,
+                                                        int32_t n) {
+    volume_body(off, L, V, n, blockIdx.x);
 }
 
 // Folded forms for the serving path: one launch zeroes (before the tiers)
@@ -358,12 +381,12 @@ __global__ __launch_bounds__(256) void k_multi_zero(const VolumeJob* __restrict_
     const VolumeJob& jb = jobs[j];
     const int64_t b0 = (int64_t)(blockIdx.x - (uint32_t)cum[j]) * kZeroPerBlock;
     const int64_t b1 = min((int64_t)jb.n, b0 + kZeroPerBlock);
-    for (int64_t i = b0 + threadIdx.x; i < b1; i += 256) jb.V[i] = 0;
+    for (int64_t i = b0 + threadIdx.x; i < b1; i += 256) jb.V[i] = counted_alone(jb.off, i, jb.L[i]) ? 1 : 0;
 }
 __global__ __launch_bounds__(kVolThreads) void k_multi_volume(const VolumeJob* __restrict__ jobs,
                                                               const int32_t* __restrict__ cum, int32_t nj) {
     const int32_t j = job_of(cum, nj, blockIdx.x);
-    volume_body(jobs[j].L, jobs[j].V, jobs[j].n, blockIdx.x - (uint32_t)cum[j]);
+    volume_body(jobs[j].off, jobs[j].L, jobs[j].V, jobs[j].n, blockIdx.x - (uint32_t)cum[j]);
 }
 // The slot-score jobs' records LV[u] = {L[u], V[L[u]]}, kZeroPerBlock rows
 // per workgroup.
@@ -394,12 +417,23 @@ int launch_multi_volume(VolumeMode mode, const VolumeJob* jobs, const int32_t* c
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "folded volume launch: %s", hipGetErrorString(e));
 }
 
-__global__ void k_label_volumes(const int32_t* __restrict__ L, const int32_t* __restrict__ V,
-                                int2* __restrict__ LV, int32_t n) {
+// The write-side volumes before the step's labels are counted (L: any label
+// buffer, edge-less vertices hold their label in both).
+__global__ void k_volume_init(const int32_t* __restrict__ off, const int32_t* __restrict__ L, int32_t* __restrict__ V,
+                              int32_t n) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+        V[i] = counted_alone(off, i, L[i]) ? 1 : 0;
+}
+// The same, and the slot-score records LV from the read-side volumes Vr.
+__global__ void k_label_volumes(const int32_t* __restrict__ off, const int32_t* __restrict__ L,
+                                const int32_t* __restrict__ Vr, int2* __restrict__ LV, int32_t* __restrict__ Vw,
+                                int32_t n) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         const int32_t l = L[i];
-        LV[i] = make_int2(l, V[l]);
+        LV[i] = make_int2(l, Vr[l]);
+        Vw[i] = counted_alone(off, i, l) ? 1 : 0;
     }
 }
 __global__ void k_iota(int32_t* p, int64_t count) {
@@ -854,9 +888,17 @@ int inverse_index_build(const int32_t* nbr, int32_t n, int64_t m, int32_t* curso
     return rc;
 }
 
-int launch_volume(const int32_t* L, int32_t* V, int32_t n, hipStream_t s) {
+int launch_volume_init(const int32_t* off, const int32_t* L, int32_t* V, int32_t n, hipStream_t s) {
     if (n <= 0) return GLP_OK;
-    hipLaunchKernelGGL(k_volume, dim3(grid_for(n, kVolChunk)), dim3(kVolThreads), 0, s, L, V, n);
+    hipLaunchKernelGGL(k_volume_init, dim3((unsigned)std::min<int64_t>(grid_for(n, 256), 256 * 64)), dim3(256), 0, s,
+                       off, L, V, n);
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "volume launch: %s", hipGetErrorString(e));
+}
+
+int launch_volume(const int32_t* off, const int32_t* L, int32_t* V, int32_t n, hipStream_t s) {
+    if (n <= 0) return GLP_OK;
+    hipLaunchKernelGGL(k_volume, dim3(grid_for(n, kVolChunk)), dim3(kVolThreads), 0, s, off, L, V, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "volume launch: %s", hipGetErrorString(e));
 }
@@ -869,10 +911,11 @@ int launch_fill_i32(int32_t* p, int32_t value, int64_t count, hipStream_t s) {
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "fill launch: %s", hipGetErrorString(e));
 }
 
-int launch_label_volumes(const int32_t* L, const int32_t* V, int2* LV, int32_t n, hipStream_t s) {
+int launch_label_volumes(const int32_t* off, const int32_t* L, const int32_t* Vr, int2* LV, int32_t* Vw, int32_t n,
+                         hipStream_t s) {
     if (n <= 0) return GLP_OK;
     const unsigned grid = (unsigned)std::min<int64_t>(grid_for(n, 256), 256 * 64);
-    hipLaunchKernelGGL(k_label_volumes, dim3(grid), dim3(256), 0, s, L, V, LV, n);
+    hipLaunchKernelGGL(k_label_volumes, dim3(grid), dim3(256), 0, s, off, L, Vr, LV, Vw, n);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "label-volume launch: %s", hipGetErrorString(e));
 }

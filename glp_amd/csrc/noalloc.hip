@@ -162,10 +162,10 @@ int run_noalloc(const glp_graph* g, const glp_params* prm, int32_t steps, int32_
             a.Vw = lay.V[cur ^ 1];
             a.score_mul = prm->gamma_den + prm->gamma_num;
             a.score_vmul = prm->gamma_num;
-            if ((rc = launch_fill_i32(a.Vw, 0, n, s))) return rc;
+            if ((rc = launch_volume_init(a.off, a.L, a.Vw, c.n, s))) return rc;
         }
         if ((rc = launch_step(method, prm->weighted != 0, false, dg, lay.hs, a, s, nullptr))) return rc;
-        if (layered && (rc = launch_volume(a.Lw, a.Vw, c.n, s))) return rc;
+        if (layered && (rc = launch_volume(a.off, a.Lw, a.Vw, c.n, s))) return rc;
         cur ^= 1;
         if (step_dump && n)
             GLP_HIP(hipMemcpyAsync(step_dump + (size_t)t * n, lay.L[cur], sizeof(int32_t) * n,

@@ -452,7 +452,7 @@ int glp_server::step_jobs(const std::vector<ServerJob*>& jobs, hipStream_t s, Ti
             a.Vw = j->V[j->cur ^ 1];
             a.score_mul = j->p.gamma_den + j->p.gamma_num;
             a.score_vmul = j->p.gamma_num;
-            h_vol[li] = VolumeJob{a.Lw, a.Vw, dg.n, 0, nullptr};
+            h_vol[li] = VolumeJob{a.Lw, a.Vw, dg.off, nullptr, dg.n, 0};
             int32_t zb = 0, vb = 0;
             volume_job_blocks(dg.n, &zb, &vb);
             h_zc[li + 1] = h_zc[li] + zb;
@@ -460,7 +460,7 @@ int glp_server::step_jobs(const std::vector<ServerJob*>& jobs, hipStream_t s, Ti
             ++li;
             if (j->LV) {
                 a.LV = j->LV;
-                h_rec[ri] = VolumeJob{a.L, j->V[j->cur], dg.n, 0, j->LV};  // read-side volumes
+                h_rec[ri] = VolumeJob{a.L, j->V[j->cur], dg.off, j->LV, dg.n, 0};  // read-side volumes
                 h_rc[ri + 1] = h_rc[ri] + zb;  // the records take the zero launch's rows per workgroup
                 ++ri;
             }

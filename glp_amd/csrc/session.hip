@@ -514,14 +514,13 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
         return set_error(GLP_E_STATE, "SLPA memory holds %d steps", s->p.slpa_T);
     StepArgs a = step_args(s);
     int rc;
-    if (s->method == Method::Layered && (rc = launch_fill_i32(s->V[s->cur ^ 1], 0, s->n, s->stream)))
-        return rc;
     // layered with gamma > 0: each neighbour's label travels with its
     // label's volume, and the tables accumulate scores (LayeredVolHooks)
     Method method = s->method;
     // from L_0 no label is gathered (the frontier gather counts on the adj
     // its steps fill, so gather sessions keep their form)
     const bool first = s->at_l0 && !replayed && !s->p.gather;
+    bool volumes = s->method == Method::Layered;  // still to be cleared
     if (first) {
         method = Method::First;
         a.ascending = s->g->dev->ascending ? 1 : 0;
@@ -529,10 +528,12 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     } else if (s->method == Method::Layered && s->LV && s->p.gamma_num > 0) {
         method = Method::LayeredVol;
         a.LV = s->LV;
-        if ((rc = launch_label_volumes(a.L, a.Vr, s->LV, s->n, s->stream))) return rc;
+        if ((rc = launch_label_volumes(a.off, a.L, a.Vr, s->LV, a.Vw, s->n, s->stream))) return rc;
+        volumes = false;
     } else if (s->method == Method::Layered && s->p.gamma_num == 0) {
         method = Method::Classic;  // the scores are qC: classic's order
     }
+    if (volumes && (rc = launch_volume_init(a.off, a.L, a.Vw, s->n, s->stream))) return rc;
     if (s->domctl && method == Method::Classic) {
         a.act_r = s->dom_act;
         a.fctl = s->domctl;
@@ -557,7 +558,7 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     if (ev) (void)hipEventRecord(ev[2 * GLP_TIER_GATHER + 1], s->stream);
     if ((rc = launch_step(method, s->p.weighted != 0, s->p.gather != 0, *s->g->dev, s->hs, a, s->stream, ev)))
         return rc;
-    if (s->method == Method::Layered && (rc = launch_volume(a.Lw, a.Vw, s->n, s->stream))) return rc;
+    if (s->method == Method::Layered && (rc = launch_volume(a.off, a.Lw, a.Vw, s->n, s->stream))) return rc;
     if ((rc = end_step(s, a.nbr, a.Lw, replayed))) return rc;
     if (s->method != Method::Slpa) s->cur ^= 1;
     s->t += 1;

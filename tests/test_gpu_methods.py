@@ -715,3 +715,24 @@ def test_countmin_rows_and_widths(rmat13w, rows, aliased, width):
     for _ in range(2):
         prev = O.countmin_step(off, nbr, prev, rows, width, aliased, w=w)
     assert np.array_equal(labels, prev)
+
+
+@pytest.mark.parametrize("gamma", [(0, 1), (1, 4)])
+def test_layered_volume_of_restored_edgeless_vertices(gamma):
+    """Edge-less vertices showing their own id are counted apart from the
+    others; restored from a state they may show any label."""
+    n = 5000
+    rng = np.random.default_rng(2)
+    g = G.Graph.from_edges(n, rng.integers(0, n // 2, (9000, 2)))  # the upper half is edge-less
+    lab = rng.integers(0, n, n).astype(np.int32)
+    lab[n // 2::3] = np.arange(n // 2, n, 3)
+    vol = np.bincount(lab, minlength=n).astype(np.int32)
+    with G.Session(g, method=G.LAYERED, gamma=gamma) as s:
+        state = bytearray(s.save())
+        state[-8 * n:] = lab.tobytes() + vol.tobytes()
+        s.load(bytes(state))
+        for _ in range(3):
+            s.step(1)
+            labels = s.labels()
+            assert np.array_equal(labels[n // 2:], lab[n // 2:])
+            assert np.array_equal(s.volume(), np.bincount(labels, minlength=n))

@@ -307,6 +307,11 @@ struct PackedLds {
     unsigned long long best[64];         // per vertex slot: best packed score
 };
 
+// How many of the lanes below this one m holds.
+__device__ __forceinline__ int32_t lanes_below(unsigned long long m) {
+    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // Every lane's first and owner: a vertex's last edge lane takes a mark from
 // it (pushed by ds_permute; lanes nobody pushes to get 0), and an edge lane's
 // owner is the number of marks below it.  With vertices of no edges, that
@@ -318,14 +323,11 @@ __device__ __forceinline__ void packed_segments(PackedGroup& s, int lane) {
     // which no lane is above)
     const unsigned long long ends =
         __ballot(__builtin_amdgcn_ds_permute(((s.ve - 1) & 63) << 2, 1) != 0);
-    auto below = [](unsigned long long m) {
-        return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-    };
-    s.own = below(ends);
+    s.own = lanes_below(ends);
     const bool has = lane < s.vc && s.ve > s.vb;
     if (__ballot(lane < s.vc && !has) != 0ull) {  // wave-uniform
         // (fewer than 64 vertices have edges, so lane 63 is free for the rest)
-        const int32_t rank = below(__ballot(has));
+        const int32_t rank = lanes_below(__ballot(has));
         const int32_t slot = __builtin_amdgcn_ds_permute((has ? rank : 63) << 2, lane);
         s.own = shfl_i32(slot, s.own);
     }
@@ -1046,64 +1048,79 @@ struct PartJob {
 };
 
 // Sums the part's pairs whose fmix32 image lies in [lo, hi) into the LDS
-// table.  The pairs lie in one run per chunk region; the workgroup walks the
-// chunks 64 at a time (every wave holds the 64 runs' lengths and starts, one
-// per lane) and spreads each window's pairs over its lanes, a pair's run
-// found by a binary search over the lanes' inclusive sums.  Stops early (the
-// caller halves the range) once more than `limit` distinct keys arrived;
-// the table has room for limit + kHubThreads.
+// table.  The pairs lie in one run per chunk region; a wave walks the chunks
+// 64 at a time (it holds the 64 runs' lengths and starts, one per lane) and
+// spreads each window's pairs over its lanes, a pair's run found by marks.
+// From kPartSplit chunks on each wave walks a quarter of them, so a large
+// hub's windows are walked side by side; with fewer, lanes would be idle, and
+// every wave walks them all and takes a quarter of the pairs.  `bounded`: the
+// table holds all of the part's pairs, and they all are in range.  Otherwise
+// it stops early (the caller halves the range) once more than `limit`
+// distinct keys arrived; the table has room for limit + kHubThreads.
+// Bound by its instructions (41% of the VALU's cycles, 62% of the LDS's):
+// marks take one permute and one look-up a pair where a binary search took
+// nine, which brought R-MAT scale 25 from 687 to 655 us a step and the
+// scale 22 layered step from 244 to 234; the next part's loads in flight
+// during this one's inserts, or tables of half the size and twice the
+// workgroups, changed nothing.
+constexpr uint32_t kPartSplit = 8;
 __device__ __forceinline__ void part_pass(const HubArgs& h, const PartJob& j, uint64_t lo, uint64_t hi,
-                                          unsigned long long* T, uint32_t shift, uint32_t limit,
-                                          uint32_t* s_distinct, uint32_t* s_over) {
+                                          unsigned long long* T, uint32_t shift, bool bounded,
+                                          uint32_t limit, uint32_t* s_distinct, uint32_t* s_over) {
     const uint32_t mask = (1u << (32 - shift)) - 1u;
     constexpr int kU = 4;  // pairs loaded per thread before any is inserted
     constexpr uint32_t kWaves = kHubThreads / 64;
     const int lane = lane_id();
-    const uint32_t wv = threadIdx.x >> 6;
+    const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t hb = h.hist_base[j.hub] + (int64_t)j.q * j.nch;
     const uint32_t* cnt = h.hs.hist + hb;
     const uint32_t* st = h.hs.lstart + hb;
     const unsigned long long* pr = h.hs.pairs + h.base[j.hub];
-    for (uint32_t c0 = 0; c0 < j.nch; c0 += 64) {  // every wave walks the same windows
+    const bool split = j.nch >= kPartSplit;
+    const uint32_t per = split ? (j.nch + kWaves - 1) / kWaves : j.nch;
+    const uint32_t cb = split ? wv * per : 0u, ce = min(cb + per, j.nch);
+    const uint32_t fb = split ? 0u : wv * 64u, fs = split ? 64u : kWaves * 64u;
+    for (uint32_t c0 = cb; c0 < ce; c0 += 64) {
         const uint32_t c = c0 + (uint32_t)lane;
-        const uint32_t n_c = c < j.nch ? cnt[c] : 0u;
-        const uint32_t s_c = c < j.nch ? c * (uint32_t)h.chunk + st[c] : 0u;
+        const uint32_t n_c = c < ce ? cnt[c] : 0u;
+        const uint32_t s_c = c < ce ? c * (uint32_t)h.chunk + st[c] : 0u;
         const int32_t incl = wave_incl_sum((int32_t)n_c);
-        const uint32_t wtot = (uint32_t)__builtin_amdgcn_readfirstlane(shfl_i32(incl, 63));
-        // the window's runs: lanes [0, nr); the owner search needs
-        // ceil(log2(nr)) halvings (most hubs have a few chunks)
-        const int nr = (int)min(64u, j.nch - c0);
-        const int depth = nr > 1 ? 32 - __builtin_clz((uint32_t)(nr - 1)) : 0;
+        const uint32_t wtot = (uint32_t)__builtin_amdgcn_readlane(incl, 63);
+        // pair f of the window lies at place + f; the runs with pairs are
+        // looked up by rank (when some have none, lane 63 is free for those)
+        const bool has = n_c != 0u;
+        const int32_t rank = lanes_below(__ballot(has));
+        const int32_t place = __builtin_amdgcn_ds_permute((has ? rank : 63) << 2,
+                                                          (int32_t)(s_c + n_c - (uint32_t)incl));
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readlane(place, 0);  // the window's first pair
         // the trip count is wave-uniform, so the wave reductions below run
-        // with every lane; lanes past the window's pairs load a clamped pair
+        // with every lane; lanes past the window's pairs load its first one
         // and skip it
-        for (uint32_t f0 = wv * 64u; f0 < wtot; f0 += kWaves * 64u * kU) {
-            if (lds_load(s_over)) return;  // one LDS read for the wave: uniform
+        for (uint32_t f0 = fb; f0 < wtot; f0 += fs * kU) {
+            if (!bounded && lds_load(s_over)) return;  // one LDS read for the wave: uniform
             unsigned long long xs[kU];
             bool in[kU];
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
-                const uint32_t f = f0 + (uint32_t)u * kWaves * 64u + (uint32_t)lane;
+                const uint32_t fu = f0 + (uint32_t)u * fs, f = fu + (uint32_t)lane;
                 in[u] = f < wtot;
-                const int32_t fc = (int32_t)min(f, wtot - 1u);
-                // owner: the first lane whose inclusive sum exceeds fc
-                // (lanes >= nr hold no pairs, so it lies in [0, nr))
-                int o = 0, top = nr - 1;
-                for (int k = 0; k < depth; ++k) {  // wave-uniform trip count
-                    const int mid = (o + top) >> 1;
-                    if (shfl_i32(incl, mid) <= fc) o = mid + 1;
-                    else top = mid;
-                }
-                const int32_t oi = shfl_i32(incl, o);
-                const uint32_t on = shfl_u32(n_c, o), os = shfl_u32(s_c, o);
-                xs[u] = pr[os + (uint32_t)(fc - (oi - (int32_t)on))];
+                if (fu >= wtot) continue;  // wave-uniform
+                // rank of a pair's run: the runs that end before fu, and the
+                // marks below its lane of those that end at fu + 0..62 (a run
+                // that ends elsewhere marks lane 63, which no lane is above)
+                const uint32_t end = (uint32_t)incl - 1u - fu;
+                const int before = __popcll(__ballot(has && incl <= (int32_t)fu));
+                const unsigned long long ends =
+                    __ballot(__builtin_amdgcn_ds_permute((int)min(end, 63u) << 2, 1) != 0);
+                const int32_t at = shfl_i32(place, min(before + lanes_below(ends), 63));
+                xs[u] = pr[in[u] ? (uint32_t)at + f : first];
             }
             uint32_t claimed = 0u;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
                 const uint32_t key = (uint32_t)(xs[u] >> 32);
                 const uint32_t hk = fmix32(key);
-                if (!in[u] || hk < lo || hk >= hi) continue;
+                if (!in[u] || (!bounded && (hk < lo || hk >= hi))) continue;
                 // a pair is already a (key << 32 | count) slot value; most pairs
                 // of a bucket bring a new label while labels are diverse, so the
                 // claim is tried first
@@ -1127,6 +1144,7 @@ __device__ __forceinline__ void part_pass(const HubArgs& h, const PartJob& j, ui
                     s = (s + 1u) & mask;
                 }
             }
+            if (bounded) continue;
             // one atomic per wave on the distinct-label counter
             const int32_t wave_claimed = __builtin_amdgcn_readfirstlane(
                 shfl_i32(wave_incl_sum((int32_t)claimed), 63));
@@ -1150,7 +1168,8 @@ __device__ __forceinline__ void hub_part_count(const StepArgs& a, const HubArgs&
     // at most n distinct labels, so it cannot overflow, and converged buckets
     // (a few pairs) scan a few slots instead of the whole table
     uint32_t cap = cap_max;
-    if (h.part_limit == 0 && n <= cap_max / 2u) cap = max(next_pow2(2u * n), 64u);
+    const bool bounded = h.part_limit == 0 && n <= cap_max / 2u;
+    if (bounded) cap = max(next_pow2(2u * n), 64u);
     const uint32_t shift = 32u - (31u - __builtin_clz(cap));
     unsigned long long* T = reinterpret_cast<unsigned long long*>(s_dyn);  // cap slots
     const uint64_t end = bucket_lo(j.q + 1, j.P);
@@ -1163,7 +1182,7 @@ __device__ __forceinline__ void hub_part_count(const StepArgs& a, const HubArgs&
             *s_over = 0u;
         }
         __syncthreads();
-        part_pass(h, j, lo, hi, T, shift, limit, s_distinct, s_over);
+        part_pass(h, j, lo, hi, T, shift, bounded, limit, s_distinct, s_over);
         __syncthreads();
         if (*s_over != 0u) {
             // the pass stopped part-way: clear the table and retry the lower

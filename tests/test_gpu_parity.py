@@ -138,6 +138,22 @@ def test_hub_part_batches(n):
     assert_steps_equal(dump, O.classic(off, nbr, 3))
 
 
+@pytest.mark.parametrize("part_keys", [256, 4096])
+@pytest.mark.parametrize("chunks", [7, 8, 9, 63, 256, 257, 520])
+def test_hub_part_runs(chunks, part_keys):
+    """One hub of `chunks` runs per part, short or long ones, walked by all
+    waves together or a quarter by each, in one window of 64 runs or more."""
+    n = chunks * 256 - 3
+    rng = np.random.default_rng(chunks)
+    e = np.stack([np.zeros(n, np.int64), np.arange(1, n + 1)], 1)
+    e = np.concatenate([e, rng.integers(1, n + 1, (n // 2, 2))])
+    with G.tuning(hub_chunk=256, part_keys=part_keys, wave_max_deg=64, block_max_deg=128):
+        g, off, nbr, _ = hand_graph([tuple(x) for x in e], n + 1)
+        _, dump, timing = G.run(g, 4, dump=True)
+    assert timing["tier_vertices"]["hub"] == 1
+    assert_steps_equal(dump, O.classic(off, nbr, 4))
+
+
 def test_hub_weighted_small_tiers():
     with G.tuning(pack_max_deg=4, wave_max_deg=8, block_max_deg=16, hub_chunk=256, part_keys=256):
         g = G.Graph.rmat(13, 16, seed=22, wmax=8)

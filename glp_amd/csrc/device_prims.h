@@ -45,11 +45,15 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, CTRL, 0xf, 0xf, false);
 }
 template <class F>
-__device__ __forceinline__ uint32_t wave_reduce(uint32_t x, F f) {
+__device__ __forceinline__ uint32_t row_reduce(uint32_t x, F f) {  // over each row of 16 lanes
     x = f(x, dpp_u32<0xB1>(x));   // quad_perm [1,0,3,2]
     x = f(x, dpp_u32<0x4E>(x));   // quad_perm [2,3,0,1]
     x = f(x, dpp_u32<0x141>(x));  // row half-mirror
-    x = f(x, dpp_u32<0x140>(x));  // row mirror
+    return f(x, dpp_u32<0x140>(x));  // row mirror
+}
+template <class F>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t x, F f) {
+    x = row_reduce(x, f);
     const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)x, 0);
     const uint32_t r1 = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
     const uint32_t r2 = (uint32_t)__builtin_amdgcn_readlane((int)x, 32);
@@ -69,6 +73,32 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t x) {
     const uint32_t hi = wave_max_u32((uint32_t)(x >> 32));
     const uint32_t lo = wave_max_u32((uint32_t)(x >> 32) == hi ? (uint32_t)x : 0u);
     return ((uint64_t)hi << 32) | lo;
+}
+// The same over each group of S = 16 or 32 consecutive lanes (two rows meet
+// through one shuffle).
+template <int S, class F>
+__device__ __forceinline__ uint32_t group_reduce(uint32_t x, F f) {
+    static_assert(S == 16 || S == 32, "one row or two");
+    x = row_reduce(x, f);
+    if (S == 32) x = f(x, shfl_u32(x, lane_id() ^ 16));
+    return x;
+}
+template <int S>
+__device__ __forceinline__ uint32_t group_sum_u32(uint32_t x) {
+    return group_reduce<S>(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+template <int S>
+__device__ __forceinline__ uint64_t group_max_u64(uint64_t x) {
+    auto mx = [](uint32_t a, uint32_t b) { return max(a, b); };
+    const uint32_t hi = group_reduce<S>((uint32_t)(x >> 32), mx);
+    const uint32_t lo = group_reduce<S>((uint32_t)(x >> 32) == hi ? (uint32_t)x : 0u, mx);
+    return ((uint64_t)hi << 32) | lo;
+}
+// The group's lane I to all of its lanes.
+template <int S, int I>
+__device__ __forceinline__ uint32_t group_lane(uint32_t x) {
+    if constexpr (S == 16) return dpp_u32<0x150 + I>(x);  // row_newbcast:I
+    else return shfl_u32(x, (lane_id() & ~(S - 1)) + I);
 }
 // Inclusive prefix sum over the 64 lanes, every lane active: within rows by
 // row shifts (a lane without a source adds 0), then each row's last lane into

@@ -523,7 +523,10 @@ __device__ __forceinline__ void packed_body(const StepArgs& a, const int2* __res
 // edges per lane; S = 16: quarters, four edges per lane), each lane group in
 // its own LDS table of kHalfCap slots.  A wave takes NP such units (chosen
 // per launch like the packed tier's NG), their loads issued before any is
-// counted.
+// counted.  Group sums and maxima run over DPP rows (one shuffle more with 32
+// lanes) and both majority candidates share one sum: 244 -> 233 us a step
+// over 96 graphs' 1.6 M vertices of 33 to 64 edges, of which bringing the
+// label lines into L1 (about 300 G lines/s) takes 200.
 constexpr uint32_t kHalfCap = 2 * kHalfMaxDeg;
 
 // Per-wave LDS of the half tier: one (key << 32 | sum) table per lane group.
@@ -585,12 +588,6 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
     bool cleared = false;  // wave-uniform
     // lanes of this group where x holds
     auto group_count = [&](bool x) { return (uint32_t)__popcll(__ballot(x) & gm); };
-    // sum over this group's lanes (xor distances below S stay in the group)
-    auto group_sum = [&](uint32_t x) {
-#pragma unroll
-        for (int d = S / 2; d >= 1; d >>= 1) x += shfl_u32(x, lane ^ d);
-        return x;
-    };
     uint32_t nch = 0u;
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
@@ -606,11 +603,10 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
 #pragma unroll
             for (int i = 0; i < EPL; ++i)
                 if (key[p][i]) fast = max_u64(fast, H::label_score(a, v[p], key[p][i], W ? fr[p][i] : 1u));
-#pragma unroll
-            for (int d = S / 2; d >= 1; d >>= 1) fast = max_u64(fast, shfl_u64(fast, lane ^ d));
+            fast = group_max_u64<S>(fast);
         } else if constexpr (count_score_of<H>::value) {
-            const uint32_t lead = shfl_u32(key[p][0], g0);
-            const uint32_t lead2 = shfl_u32(key[p][0], g0 + S / 2);
+            const uint32_t lead = group_lane<S, 0>(key[p][0]);
+            const uint32_t lead2 = group_lane<S, S / 2>(key[p][0]);
             uint32_t c = 0u, c2 = 0u, tot = 0u;
             if (W) {
 #pragma unroll
@@ -620,9 +616,9 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
                     c2 += k && k == lead2 ? fr[p][i] : 0u;
                     tot += k ? fr[p][i] : 0u;
                 }
-                c = group_sum(c);
-                c2 = group_sum(c2);
-                tot = group_sum(tot);
+                c = group_sum_u32<S>(c);
+                c2 = group_sum_u32<S>(c2);
+                tot = group_sum_u32<S>(tot);
             } else {
                 // only seeded LP has unlabeled neighbours (key 0); otherwise
                 // every edge of the vertex counts once
@@ -632,14 +628,13 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
                 } else {
                     tot = run[p] ? (uint32_t)(e[p] - b[p]) : 0u;
                 }
+                // both candidates in one sum of half words (at most 64 edges)
 #pragma unroll
-                for (int i = 0; i < EPL; ++i) c += group_count(key[p][i] != 0u && key[p][i] == lead);
-                // the second candidate only when some group still needs one
-                if (__ballot(run[p] && !(lead != 0u && 2ull * c > (unsigned long long)tot)) != 0ull) {
-#pragma unroll
-                    for (int i = 0; i < EPL; ++i)
-                        c2 += group_count(key[p][i] != 0u && key[p][i] == lead2);
-                }
+                for (int i = 0; i < EPL; ++i)
+                    c += (key[p][i] == lead ? 1u : 0u) + (key[p][i] == lead2 ? 0x10000u : 0u);
+                c = group_sum_u32<S>(c);
+                c2 = c >> 16;
+                c &= 0xffffu;
             }
             if (run[p] && lead != 0u && 2ull * c > (unsigned long long)tot)
                 fast = H::label_score(a, v[p], lead, c);
@@ -675,7 +670,7 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
                     const uint32_t cnt = group_count(same);
                     if (W) {
                         // weighted: the group's sum of the merged lanes' frequencies
-                        const uint32_t x = group_sum(same ? f : 0u);
+                        const uint32_t x = group_sum_u32<S>(same ? f : 0u);
                         if (same && cnt >= 2u) f = x;
                     } else if (same && cnt >= 2u) {
                         f = cnt;
@@ -698,9 +693,7 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
                     pm = max_u64(pm, slot_value_score<H, S_>(a, v[p], sk[i], (uint32_t)*slot));
                     *slot = 0ull;
                 }
-            // max over the group (xor distances below S stay in the group)
-#pragma unroll
-            for (int d = S / 2; d >= 1; d >>= 1) pm = max_u64(pm, shfl_u64(pm, lane ^ d));
+            pm = group_max_u64<S>(pm);
             if (!fast) best = pm;
         }
         bool changed = false;

@@ -45,9 +45,10 @@ TRAFFIC_SOURCE = ("profiles/pmc_traffic_rmat_s25_classic.txt: rocprofv3 FETCH_SI
 TRAFFIC_FILE_LAYERED = os.path.join(ROOT, "profiles", "pmc_traffic_rmat_s25_layered_g1_4.txt")
 METRIC = "GTEPS per LP iteration (RMAT-25, 1 GPU); batched graphs/s vs plain; p50/p99"
 TIER_FAMILIES = {"packed": ["k_packed"], "wave": ["k_wave", "k_half"], "block": ["k_block"],
-                 "hub": ["k_hub_agg"]}
+                 "hub": ["k_hub_agg"], "gather": ["k_dominant_bits", "k_dominant_edges", "k_dominant_decide"]}
 KERNEL_NAMES = {"packed": "k_packed", "wave": "k_wave + k_half", "block": "k_block (all degree classes)",
-                "hub": "k_hub_agg", "aux": "k_hub_part+k_hub_final"}
+                "hub": "k_hub_agg", "aux": "k_hub_part+k_hub_final",
+                "gather": "k_dominant_bits + k_dominant_edges + k_dominant_decide"}
 
 
 def log(*a):
@@ -83,11 +84,18 @@ def tiers_over(base, tim, steps):
     return tiers
 
 
-def dominant_roofline(tiers, per_edge, per_vertex):
+def dominant_roofline(tiers, per_edge, per_vertex, m, n):
+    """The roofline of the tier that takes longest.  In a fused session the
+    gather slot times the dominant label's passes: 4 B per edge (neighbour
+    ids, whose labels are bits of a bitmap) and 12 B per vertex of the whole
+    graph; the tiers then skip the vertices it settled."""
     dom = max((k for k in tiers if k in TIER_FAMILIES), key=lambda k: tiers[k]["ms"], default=None)
     if dom is None:
         return None, None
-    b = tier_bytes(tiers[dom]["edges"], tiers[dom]["vertices"], per_edge, per_vertex)
+    edges, vertices = tiers[dom]["edges"], tiers[dom]["vertices"]
+    if dom == "gather":
+        edges, vertices, per_edge, per_vertex = m, n, 4, 12
+    b = tier_bytes(edges, vertices, per_edge, per_vertex)
     achieved = b / (tiers[dom]["ms"] / 1e3) / 1e9
     return dom, {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                  "frac": round(achieved / HBM_PEAK_GBS, 4), "kernel": KERNEL_NAMES[dom],
@@ -256,7 +264,7 @@ def layered_legs(args, G, g, n, m):
         ls.sync()
         lms = (time.perf_counter() - t0) * 1e3 / args.steps
         tiers = tiers_over(base, ls.timing(), args.steps)
-        dom, roof = dominant_roofline(tiers, 12, 16)
+        dom, roof = dominant_roofline(tiers, 12, 16, m, n)
         if roof is not None and (gn, gd) == (1, 4):
             # rocprof FETCH_SIZE + WRITE_SIZE of the same kernels at gamma 1/4
             t = RS.traffic_for(TRAFFIC_FILE_LAYERED, "rmat-s%d-ef%d-seed%d-layered-1/4" % (
@@ -760,7 +768,7 @@ def main():
         ls.sync()
         lms = (time.perf_counter() - t0) * 1e3 / args.steps
         tiers = tiers_over(base, ls.timing(), args.steps)
-        _, roof = dominant_roofline(tiers, 12, 16)
+        _, roof = dominant_roofline(tiers, 12, 16, m, n)
         ls.free()
         print(json.dumps({"metric": "GTEPS per layered LP iteration (RMAT-%d, gamma %d/%d)" % (args.scale, gp, gq),
                           "value": round(m / (lms / 1e3) / 1e9, 3), "unit": "GTEPS", "ms_per_step": round(lms, 4),
@@ -770,7 +778,7 @@ def main():
 
     ms_per_step, tiers, changes, dense_labels = rmat_main(args, G, g, n, m)
     gteps = m / (ms_per_step / 1e3) / 1e9
-    dom, roofline = dominant_roofline(tiers, 8, 12)
+    dom, roofline = dominant_roofline(tiers, 8, 12, m, n)
     if roofline is not None:
         traffic = RS.traffic_for(TRAFFIC_FILE, wl_key, "main", TIER_FAMILIES[dom])
         roofline["traffic"] = None if traffic is None else int(traffic)

@@ -534,11 +534,6 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
         method = Method::Classic;  // the scores are qC: classic's order
     }
     if (volumes && (rc = launch_volume_init(a.off, a.L, a.Vw, s->n, s->stream))) return rc;
-    if (s->domctl && method == Method::Classic) {
-        a.act_r = s->dom_act;
-        a.fctl = s->domctl;
-        if ((rc = launch_dominant(*s->g->dev, a, s->dom_bits, s->dom_ebits, s->dom_act, s->stream))) return rc;
-    }
     // frontier flags for the next step start clear (they held the last step's)
     if (s->fctl && (rc = launch_zero_bytes(s->act[s->cur ^ 1], s->act_bytes, s->stream))) return rc;
     // this step's changed-vertex bits start clear (they held two steps back)
@@ -549,6 +544,11 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     }
     if (ev) (void)hipEventRecord(ev[2 * GLP_TIER_PICK + 1], s->stream);
     if (ev) (void)hipEventRecord(ev[2 * GLP_TIER_GATHER], s->stream);
+    if (s->domctl && method == Method::Classic) {
+        a.act_r = s->dom_act;
+        a.fctl = s->domctl;
+        if ((rc = launch_dominant(*s->g->dev, a, s->dom_bits, s->dom_ebits, s->dom_act, s->stream))) return rc;
+    }
     if (s->p.gather) {
         int32_t* adj = const_cast<int32_t*>(a.adj);
         if (s->chg[0]) rc = launch_frontier_gather(a, s->g->csr.m, adj, s->g->dev->inv, s->push, s->stream);

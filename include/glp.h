@@ -80,7 +80,9 @@ typedef struct glp_params {
 } glp_params;
 
 /* Per-tier timing and shape record.  Replaces header/test_result.h:5-23
- * (Test_result): times are milliseconds from HIP events, not host clocks. */
+ * (Test_result): times are milliseconds from HIP events, not host clocks.
+ * The gather slot times the separate gather, or in a fused session the passes
+ * that settle vertices by a dominant label. */
 enum { GLP_TIER_PACKED = 0, GLP_TIER_WAVE = 1, GLP_TIER_BLOCK = 2, GLP_TIER_HUB = 3,
        GLP_TIER_GATHER = 4, GLP_TIER_PICK = 5, GLP_TIER_AUX = 6, GLP_NTIERS = 8 };
 typedef struct glp_timing {

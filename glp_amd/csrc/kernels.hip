@@ -706,22 +706,37 @@ __global__ __launch_bounds__(kDomThreads) void k_dominant_edges(const int32_t* _
     }
 }
 
-// Set bits among bits [b, e) of ebits, `stride` threads cooperating.
+// Set bits among bits [b, e) of ebits, `stride` threads cooperating, U words
+// of each in flight (a word past the end is the last one again, not counted).
+template <int U>
 __device__ __forceinline__ uint32_t count_bits(const uint32_t* __restrict__ ebits, int32_t b, int32_t e, int tid,
                                                int stride) {
     uint32_t c = 0u;
     const int32_t w1 = (int32_t)(((uint32_t)e + 31u) >> 5);
-    for (int32_t w = (b >> 5) + tid; w < w1; w += stride) {
-        uint32_t x = ebits[w];
-        if (w == (b >> 5)) x &= 0xffffffffu << (b & 31);
-        if (w == (e >> 5)) x &= (1u << (e & 31)) - 1u;  // (not met when e is a multiple of 32)
-        c += (uint32_t)__popc(x);
+    for (int32_t w0 = (b >> 5) + tid; w0 < w1; w0 += stride * U) {
+        uint32_t x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = ebits[min(w0 + u * stride, w1 - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int32_t w = w0 + u * stride;
+            if (w == (b >> 5)) x[u] &= 0xffffffffu << (b & 31);
+            if (w == (e >> 5)) x[u] &= (1u << (e & 31)) - 1u;  // (not met when e is a multiple of 32)
+            c += w < w1 ? (uint32_t)__popc(x[u]) : 0u;
+        }
     }
     return c;
 }
-// Workgroups [0, nhubs) take a hub each; the others 256 vertices each, one
-// lane per vertex up to kDomLaneDeg edges, a wave above (hubs left out).
+// Workgroups [0, nhubs) take a hub each; the others 1,024 vertices each, one
+// lane per vertex up to kDomLaneDeg edges, 16 lanes above (hubs left out).
+// Ids in degree order put 64 of the larger ones in one wave, which then is a
+// chain of dependent reads: four of them at a time, several words of each in
+// flight, instead of one after another by the whole wave.  R-MAT scale 25,
+// converged: 217 us a step with a whole wave per larger vertex, 172 with rows
+// of 16 lanes, 140 with four vertices per lane, 470 MB; an undecided step's
+// launch, which only ends, 31 -> 11 us.
 constexpr int32_t kDomLaneDeg = 256;
+constexpr int kDomVerts = 4;  // vertices per lane, their offsets loaded together
 __global__ __launch_bounds__(256) void k_dominant_decide(StepArgs a, const uint32_t* __restrict__ ebits,
                                                          const int32_t* __restrict__ hubs, int32_t nhubs,
                                                          int32_t hub_deg, uint8_t* __restrict__ act) {
@@ -737,33 +752,53 @@ __global__ __launch_bounds__(256) void k_dominant_decide(StepArgs a, const uint3
         a.Lw[v] = label;
         return a.keep[v] != label;
     };
-    bool changed = false;
     if ((int32_t)blockIdx.x < nhubs) {
         __shared__ uint32_t s_c[4];
+        bool changed = false;
         const int32_t v = hubs[blockIdx.x];
         const int32_t b = a.off[v], e = a.off[v + 1];
-        const uint32_t c = wave_sum_u32(count_bits(ebits, b, e, threadIdx.x, 256));
+        const uint32_t c = wave_sum_u32(count_bits<2>(ebits, b, e, threadIdx.x, 256));
         if (lane == 0) s_c[threadIdx.x >> 6] = c;
         __syncthreads();
         if (threadIdx.x == 0) changed = settle(v, e - b, s_c[0] + s_c[1] + s_c[2] + s_c[3]);
         if (threadIdx.x < 64) count_changes(a, changed);
         return;
     }
-    const int64_t v0 = (int64_t)(blockIdx.x - (uint32_t)nhubs) * 256 + (threadIdx.x & ~63);
-    const int64_t v = v0 + lane;
-    int32_t b = 0, e = 0;
-    if (v < a.n) {
-        b = a.off[v];
-        e = a.off[v + 1];
+    const int64_t vw = (int64_t)(blockIdx.x - (uint32_t)nhubs) * (256 * kDomVerts) + (threadIdx.x & ~63);
+    int32_t vb[kDomVerts], ve[kDomVerts];
+#pragma unroll
+    for (int k = 0; k < kDomVerts; ++k) {
+        const int64_t v = min(vw + k * 256 + lane, (int64_t)a.n - 1);
+        vb[k] = a.off[v];
+        ve[k] = a.off[v + 1];
     }
-    if (v < a.n && e - b <= kDomLaneDeg) changed = settle((int32_t)v, e - b, count_bits(ebits, b, e, 0, 1));
-    for (unsigned long long q = __ballot(e - b > kDomLaneDeg && e - b <= hub_deg); q; q &= q - 1ull) {
-        const int src = (int)__builtin_ctzll(q);
-        const int32_t vb = shfl_i32(b, src), ve = shfl_i32(e, src);
-        const uint32_t c = wave_sum_u32(count_bits(ebits, vb, ve, lane, 64));
-        if (lane == src) changed = settle((int32_t)v, ve - vb, c);
+    uint32_t nch = 0u;
+#pragma unroll
+    for (int k = 0; k < kDomVerts; ++k) {
+        const int64_t v0 = vw + k * 256, v = v0 + lane;
+        const int32_t b = vb[k], e = ve[k];
+        const bool small = v < a.n && e - b <= kDomLaneDeg;
+        uint32_t c = 0u;
+        if (__ballot(small && e - b > 64) != 0ull) c = small ? count_bits<4>(ebits, b, e, 0, 1) : 0u;
+        else if (small) c = count_bits<1>(ebits, b, e, 0, 1);
+        bool changed = small && settle((int32_t)v, e - b, c);
+        nch += (uint32_t)__popcll(__ballot(changed));
+        unsigned long long q = __ballot(v < a.n && e - b > kDomLaneDeg && e - b <= hub_deg);
+        while (q) {  // wave-uniform: the next four, a row of 16 lanes each
+            int src = -1;
+#pragma unroll
+            for (int row = 0; row < 4; ++row) {
+                if (lane >> 4 == row && q) src = (int)__builtin_ctzll(q);
+                q &= q - 1ull;  // (0 stays 0)
+            }
+            const int32_t sb = shfl_i32(b, max(src, 0)), se = shfl_i32(e, max(src, 0));
+            const int32_t rb = src < 0 ? 0 : sb, re = src < 0 ? 0 : se;  // no vertex: no words
+            c = group_sum_u32<16>(count_bits<4>(ebits, rb, re, lane & 15, 16));
+            changed = src >= 0 && (lane & 15) == 0 && settle((int32_t)(v0 + src), re - rb, c);
+            nch += (uint32_t)__popcll(__ballot(changed));
+        }
     }
-    count_changes(a, changed);
+    add_changes(a, nch);
 }
 
 void init_kernels() {
@@ -1020,7 +1055,7 @@ int launch_dominant(const DeviceGraph& g, const StepArgs& a, uint32_t* bits, uin
                            bits, blocks, fine, nblocks, a.fctl, ebits);
     }
     const int32_t nh = (int32_t)g.plan.hubs.size();
-    hipLaunchKernelGGL(k_dominant_decide, dim3((unsigned)nh + grid_for(g.n, 256)), dim3(256), 0, s, a, ebits, g.d_hubs,
+    hipLaunchKernelGGL(k_dominant_decide, dim3((unsigned)nh + grid_for(g.n, 256 * kDomVerts)), dim3(256), 0, s, a, ebits, g.d_hubs,
                        nh, nh ? g.plan.tune.block_max_deg : INT32_MAX, act);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "dominant label launch: %s", hipGetErrorString(e));

@@ -396,6 +396,27 @@ def test_first_step_of_a_loaded_file(tmp_path):
         assert_steps_equal(gpu_steps(g, 3), O.classic(off, nbr, 3))
 
 
+@pytest.mark.parametrize("more", [5, 1021])
+def test_dominant_label_of_ragged_vertex_counts(more):
+    """Vertices past a full workgroup's share, with degrees on both sides of
+    each split of the deciding pass (64, 256 and the hubs' 4,096 edges)."""
+    base = G.Graph.rmat(20, 20, seed=12)
+    off, nbr, _ = base.csr()
+    u = np.repeat(np.arange(base.n, dtype=np.int64), np.diff(off))
+    keep = u < nbr
+    degs = np.resize([64, 256, 65, 257, 4096, 4097, 3, 0], more)
+    rng = np.random.default_rng(more)
+    u2 = np.repeat(base.n + np.arange(more), degs)
+    v2 = np.concatenate([rng.choice(base.n, d, replace=False) for d in degs])
+    e = np.concatenate([np.stack([u[keep], nbr[keep].astype(np.int64)], 1), np.stack([u2, v2], 1)])
+    g = G.Graph.from_edges(base.n + more, e)
+    assert g.m >= 1 << 24 and np.array_equal(np.diff(g.csr()[0])[base.n:], degs)
+    steps = 8
+    want = gpu_steps(g, steps, gather=True)
+    assert np.bincount(want[steps - 2][g.csr()[1]]).max() > 0.55 * g.m  # the last step has a dominant label
+    assert_steps_equal(gpu_steps(g, steps), want)
+
+
 @pytest.mark.parametrize("sort", [False, True])
 def test_dominant_label_settles_the_same_labels(sort):
     """A graph large enough for the dominant label's passes (2^24 edges,

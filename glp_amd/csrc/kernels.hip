@@ -727,8 +727,9 @@ __device__ __forceinline__ uint32_t count_bits(const uint32_t* __restrict__ ebit
     }
     return c;
 }
-// Workgroups [0, nhubs) take a hub each; the others 1,024 vertices each, one
-// lane per vertex up to kDomLaneDeg edges, 16 lanes above (hubs left out).
+// Workgroups [0, nhubs) take a hub each (degrees above hub_deg, which may be
+// less than kDomLaneDeg); the others 1,024 vertices each, hubs left out, one
+// lane per vertex up to kDomLaneDeg edges, 16 lanes above.
 // Ids in degree order put 64 of the larger ones in one wave, which then is a
 // chain of dependent reads: four of them at a time, several words of each in
 // flight, instead of one after another by the whole wave.  R-MAT scale 25,
@@ -777,7 +778,7 @@ __global__ __launch_bounds__(256) void k_dominant_decide(StepArgs a, const uint3
     for (int k = 0; k < kDomVerts; ++k) {
         const int64_t v0 = vw + k * 256, v = v0 + lane;
         const int32_t b = vb[k], e = ve[k];
-        const bool small = v < a.n && e - b <= kDomLaneDeg;
+        const bool small = v < a.n && e - b <= min(kDomLaneDeg, hub_deg);
         uint32_t c = 0u;
         if (__ballot(small && e - b > 64) != 0ull) c = small ? count_bits<4>(ebits, b, e, 0, 1) : 0u;
         else if (small) c = count_bits<1>(ebits, b, e, 0, 1);

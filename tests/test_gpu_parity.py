@@ -455,6 +455,31 @@ def test_dominant_label_settles_the_same_labels(sort):
     assert np.array_equal(dumps[0], dumps[1])
 
 
+def test_dominant_label_counts_small_hubs_once():
+    """With hubs from 129 edges on, the deciding pass leaves each of them to
+    its own workgroup: the change counts are those of the labels."""
+    steps = 8
+    with G.tuning(pack_max_deg=16, wave_max_deg=64, block_max_deg=128):
+        g = G.Graph.rmat(20, 20, seed=13)
+        off, nbr, _ = g.csr()
+        deg = np.diff(off)
+        src = np.repeat(np.arange(g.n), deg)
+        want = gpu_steps(g, steps, gather=True)
+        hit = 0  # hubs of at most 256 edges that a step's dominant label, on most of their edges, moves to it
+        for t in range(1, steps):
+            top = np.bincount(want[t - 1][nbr])
+            if top.max() > 0.55 * g.m:
+                label = top.argmax()
+                most = 2 * np.bincount(src[want[t - 1][nbr] == label], minlength=g.n) > deg
+                hit += int((most & (want[t - 1] != label) & (deg > 128) & (deg <= 256)).sum())
+        assert hit > 0
+        with G.Session(g) as s:
+            s.step(steps)
+            prev = np.vstack([np.arange(g.n, dtype=np.int32)[None], want[:-1]])
+            assert s.changes().tolist() == (want != prev).sum(axis=1).tolist()
+            assert np.array_equal(s.labels(), want[-1])
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(weighted=True), dict(method=G.LAYERED, gamma=(1, 4)),
                                 dict(method=G.LAYERED, gamma=(1, 2), weighted=True), dict(method=G.USER),
                                 dict(method=G.SLPA, slpa_T=4), dict(frontier=1)])

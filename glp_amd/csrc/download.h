@@ -11,7 +11,7 @@ struct CopySlots {
     char* slot[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};
     size_t chunk = 0;
-    int create(size_t chunk);
+    bool create(size_t chunk);  // false: no memory or events to be had
     ~CopySlots();
 };
 
@@ -24,7 +24,8 @@ struct Staging {
 };
 
 // Copies `bytes` from the device to pageable host memory after the work
-// queued on s; returns when they are there.
+// queued on s; returns when they are there.  Where the buffers cannot be had
+// the copy is a plain one.
 int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s);
 
 }  // namespace glp

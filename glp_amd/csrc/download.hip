@@ -32,18 +32,25 @@ CopySlots::~CopySlots() {
     if (slot[0]) (void)hipHostFree(slot[0]);
 }
 
-int CopySlots::create(size_t bytes) {
-    if (chunk) return GLP_OK;
+bool CopySlots::create(size_t bytes) {
+    if (chunk) return true;
+    hipError_t err = hipSuccess;
     if (!slot[0]) {
         void* p = nullptr;
-        GLP_HIP(hipHostMalloc(&p, 2 * bytes, hipHostMallocDefault));
-        slot[0] = static_cast<char*>(p);
-        slot[1] = slot[0] + bytes;
+        err = hipHostMalloc(&p, 2 * bytes, hipHostMallocDefault);
+        if (err == hipSuccess) {
+            slot[0] = static_cast<char*>(p);
+            slot[1] = slot[0] + bytes;
+        }
     }
     for (auto& e : done)
-        if (!e) GLP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        if (err == hipSuccess && !e) err = hipEventCreateWithFlags(&e, hipEventDisableTiming);
+    if (err != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
     chunk = bytes;
-    return GLP_OK;
+    return true;
 }
 
 // Chunk i + 1 crosses the link while chunk i goes from its slot to its place.
@@ -71,7 +78,11 @@ int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStrea
     if (bytes == 0) return GLP_OK;
     const bool repeat = st.used;
     st.used = true;
-    if (bytes < kCopyDirect || (!repeat && bytes < kCopyLarge)) {
+    bool staged = bytes >= kCopyLarge || (repeat && bytes >= kCopyDirect);
+    if (staged && bytes < kCopyLarge) staged = st.small.create(kSmallChunk);
+    else if (staged)
+        for (auto& w : st.large) staged = staged && w.create(kLargeChunk);
+    if (!staged) {
         GLP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         GLP_HIP(hipStreamSynchronize(s));
         return GLP_OK;
@@ -79,14 +90,8 @@ int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStrea
     char* to = static_cast<char*>(dst);
     const char* from = static_cast<const char*>(src);
     if (bytes < kCopyLarge) {
-        const int rc = st.small.create(kSmallChunk);
-        if (rc != GLP_OK) return rc;
         const hipError_t e = copy_range(st.small, to, from, bytes, s);
         return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(e));
-    }
-    for (auto& w : st.large) {
-        const int rc = w.create(kLargeChunk);
-        if (rc != GLP_OK) return rc;
     }
     int dev = 0;
     GLP_HIP(hipGetDevice(&dev));

@@ -1,0 +1,73 @@
+"""Host paths of the library on a stand-in for the HIP runtime
+(fake_hip.cpp): what it allocates, launches and copies, and what it does when
+an allocation is refused.  Each test body runs in a process of its own, since
+the stand-in has to be loaded before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+TESTS = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(TESTS)
+
+PRELUDE = """
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+fake.fake_log.restype = ctypes.c_char_p
+fake.fake_device_bytes.restype = ctypes.c_size_t
+fake.fake_limit_device.argtypes = [ctypes.c_size_t]
+for f in (fake.fake_fail_host_alloc, fake.fake_fail_events, fake.fake_fail_new):
+    f.argtypes = [ctypes.c_long]
+import numpy as np
+import glp_amd as G
+
+def log():
+    return fake.fake_log().decode().split()
+
+def edgeless(n):
+    return G.Graph.from_csr(np.zeros(n + 1, dtype=np.int32), np.zeros(0, dtype=np.int32))
+
+def with_labels(s, n, seed=0):
+    # a session showing labels of its own, and those labels
+    state = bytearray(s.save())
+    lab = np.random.default_rng(seed).integers(0, n, n).astype(np.int32)
+    state[-4 * n:] = lab.tobytes()
+    s.load(bytes(state))
+    return lab
+"""
+
+
+@pytest.fixture(scope="session")
+def fake_hip(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-I" + os.path.join(rocm, "include"),
+                    os.path.join(TESTS, "fake_hip.cpp"), "-o", out], check=True)
+
+    def run(body):
+        env = dict(os.environ, PYTHONPATH=ROOT + os.pathsep + os.environ.get("PYTHONPATH", ""))
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, out], capture_output=True, text=True, env=env,
+                           timeout=300)
+        assert r.returncode == 0, (r.returncode, r.stdout[-2000:], r.stderr[-4000:])
+        return r.stdout
+
+    return run
+
+
+def test_result_copies_without_pinned_memory(fake_hip):
+    """Results are copied whether or not pinned slots and their events can be
+    had, for sizes with one and with several copying threads."""
+    fake_hip("""
+for n in (1 << 19, 3 << 19, 1 << 22, (1 << 22) + 5):
+    for fail, least in ((fake.fake_fail_host_alloc, 0), (fake.fake_fail_events, 0), (fake.fake_fail_events, 1),
+                        (fake.fake_fail_events, 5), (fake.fake_fail_host_alloc, -1)):
+        s = G.Session(edgeless(n))
+        lab = with_labels(s, n)
+        fail(least)
+        for _ in range(3):
+            assert np.array_equal(s.labels(), lab), (n, least)
+        fail(-1)
+        assert np.array_equal(s.labels(), lab), (n, least)  # and once there is memory again
+        s.free()
+""")

@@ -5,8 +5,7 @@
 
 #include <algorithm>
 #include <cstring>
-#include <system_error>
-#include <thread>
+#include <pthread.h>
 
 namespace glp {
 
@@ -74,6 +73,24 @@ static hipError_t copy_range(CopySlots& w, char* dst, const char* src, size_t by
     return e;
 }
 
+// A worker's share of a large copy.  (Threads are made by pthread_create,
+// which reports what it cannot do; std::thread allocates and throws.)
+struct CopyShare {
+    CopySlots* slots;
+    char* dst;
+    const char* src;
+    size_t bytes;
+    hipStream_t s;
+    int dev;
+    hipError_t err;
+};
+static void* copy_share(void* arg) {
+    CopyShare& c = *static_cast<CopyShare*>(arg);
+    c.err = hipSetDevice(c.dev);
+    if (c.err == hipSuccess) c.err = copy_range(*c.slots, c.dst, c.src, c.bytes, c.s);
+    return nullptr;
+}
+
 int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes == 0) return GLP_OK;
     const bool repeat = st.used;
@@ -96,28 +113,21 @@ int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStrea
     int dev = 0;
     GLP_HIP(hipGetDevice(&dev));
     const size_t share = ((bytes + kLargeChunk - 1) / kLargeChunk + kCopyWorkers - 1) / kCopyWorkers * kLargeChunk;
-    hipError_t err[kCopyWorkers] = {};
-    auto work = [&](int i) {
+    CopyShare part[kCopyWorkers];
+    pthread_t helper[kCopyWorkers];
+    bool runs[kCopyWorkers] = {};
+    for (int i = 0; i < kCopyWorkers; ++i) {
         const size_t b = std::min(bytes, (size_t)i * share), e = std::min(bytes, b + share);
-        err[i] = copy_range(st.large[i], to + b, from + b, e - b, s);
-    };
-    std::thread helper[kCopyWorkers];
-    for (int i = 1; i < kCopyWorkers; ++i) {
-        try {
-            helper[i] = std::thread([&, i] {
-                err[i] = hipSetDevice(dev);
-                if (err[i] == hipSuccess) work(i);
-            });
-        } catch (const std::system_error&) {
-            // no thread to be had: this one takes the share below
-        }
+        part[i] = CopyShare{&st.large[i], to + b, from + b, e - b, s, dev, hipSuccess};
+        if (i) runs[i] = pthread_create(&helper[i], nullptr, copy_share, &part[i]) == 0;
     }
+    // this thread takes the first share, and those for which no thread was to be had
     for (int i = 0; i < kCopyWorkers; ++i)
-        if (!helper[i].joinable()) work(i);
-    for (auto& h : helper)
-        if (h.joinable()) h.join();
-    for (hipError_t e : err)
-        if (e != hipSuccess) return set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(e));
+        if (!runs[i]) (void)copy_share(&part[i]);
+    for (int i = 0; i < kCopyWorkers; ++i)
+        if (runs[i]) (void)pthread_join(helper[i], nullptr);
+    for (const CopyShare& p : part)
+        if (p.err != hipSuccess) return set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(p.err));
     return GLP_OK;
 }
 

@@ -71,3 +71,21 @@ for n in (1 << 19, 3 << 19, 1 << 22, (1 << 22) + 5):
         assert np.array_equal(s.labels(), lab), (n, least)  # and once there is memory again
         s.free()
 """)
+
+
+def test_result_copies_when_no_thread_state_can_be_allocated(fake_hip):
+    """A copy by several threads neither throws nor ends the process when an
+    allocation fails inside it, whichever one: it gives the labels."""
+    fake_hip("""
+n = (1 << 22) + 5
+s = G.Session(edgeless(n))
+lab = with_labels(s, n)
+out = np.empty(n, dtype=np.int32)
+copy = G.lib().glp_session_labels
+for after in (-1, 0, 1, 2, 3, 4, 5, 6):
+    out[:] = -1
+    fake.fake_fail_new(after)
+    rc = copy(s._h, out.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)))
+    fake.fake_fail_new(-1)
+    assert rc == 0 and np.array_equal(out, lab), after
+""")

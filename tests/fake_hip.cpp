@@ -24,7 +24,15 @@ std::string& log_text() {
     static auto* s = new std::string;
     return *s;
 }
+// operator new of the arming thread throws once this many more were made
+thread_local long news_left = -1;
+struct Spared {  // what the stand-in itself allocates does not count
+    long saved = news_left;
+    Spared() { news_left = -1; }
+    ~Spared() { news_left = saved; }
+};
 void note(const char* what) {
+    Spared own;
     std::lock_guard<std::mutex> lk(mu);
     log_text() += what;
     log_text() += '\n';
@@ -42,8 +50,6 @@ thread_local struct {
     size_t lds;
     hipStream_t s;
 } config;
-// operator new of the arming thread throws once this many more were made
-thread_local long news_left = -1;
 
 hipError_t give(void** p, size_t n) {
     *p = std::calloc(1, n ? n : 1);
@@ -76,6 +82,7 @@ void fake_fail_new(long after) { news_left = after; }
 
 // ---- the runtime ----
 hipError_t hipMalloc(void** p, size_t n) {
+    Spared own;
     std::lock_guard<std::mutex> lk(mu);
     if (n > device_limit || device_bytes > device_limit - n) return hipErrorOutOfMemory;
     const hipError_t e = give(p, n);
@@ -95,7 +102,10 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
-    note(("hipHostMalloc " + std::to_string(n)).c_str());
+    {
+        Spared own;
+        note(("hipHostMalloc:" + std::to_string(n)).c_str());
+    }
     if (host_allocs_left >= 0 && host_allocs_left-- <= 0) {
         host_allocs_left = 0;
         return hipErrorOutOfMemory;

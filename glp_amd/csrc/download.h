@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstddef>
+#include <mutex>
 
 namespace glp {
 
@@ -19,13 +20,14 @@ constexpr int kCopyWorkers = 4;
 // A session's buffers, made when copies repeat and kept while it lives (1 MB,
 // and 16 MB once its copies are large).
 struct Staging {
+    std::mutex mu;  // held by the copy that uses them
     CopySlots small, large[kCopyWorkers];
     bool used = false;  // a copy that could have used them was made
 };
 
 // Copies `bytes` from the device to pageable host memory after the work
-// queued on s; returns when they are there.  Where the buffers cannot be had
-// the copy is a plain one.
+// queued on s; returns when they are there.  Where the buffers cannot be had,
+// or are in use by a copy of another thread, the copy is a plain one.
 int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s);
 
 }  // namespace glp

@@ -93,13 +93,17 @@ static void* copy_share(void* arg) {
 
 int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes == 0) return GLP_OK;
-    const bool repeat = st.used;
-    st.used = true;
-    bool staged = bytes >= kCopyLarge || (repeat && bytes >= kCopyDirect);
-    if (staged && bytes < kCopyLarge) staged = st.small.create(kSmallChunk);
-    else if (staged)
-        for (auto& w : st.large) staged = staged && w.create(kLargeChunk);
+    std::unique_lock<std::mutex> slots(st.mu, std::try_to_lock);
+    bool staged = false;
+    if (slots.owns_lock()) {
+        staged = bytes >= kCopyLarge || (st.used && bytes >= kCopyDirect);
+        st.used = true;
+        if (staged && bytes < kCopyLarge) staged = st.small.create(kSmallChunk);
+        else if (staged)
+            for (auto& w : st.large) staged = staged && w.create(kLargeChunk);
+    }
     if (!staged) {
+        if (slots.owns_lock()) slots.unlock();
         GLP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
         GLP_HIP(hipStreamSynchronize(s));
         return GLP_OK;

@@ -89,3 +89,32 @@ for after in (-1, 0, 1, 2, 3, 4, 5, 6):
     fake.fake_fail_new(-1)
     assert rc == 0 and np.array_equal(out, lab), after
 """)
+
+
+def test_result_copies_by_several_threads(fake_hip):
+    """Threads that read one session's results at a time, with sizes for one
+    and for several copying threads, each get their own."""
+    fake_hip("""
+import threading
+for n in (3 << 19, (1 << 22) + 5):
+    s = G.Session(edgeless(n), method=G.LAYERED, gamma=(1, 2))
+    rng = np.random.default_rng(n)
+    want = {"labels": rng.integers(0, n, n).astype(np.int32), "volume": rng.integers(0, n, n).astype(np.int32)}
+    state = bytearray(s.save())
+    state[-8 * n:] = want["labels"].tobytes() + want["volume"].tobytes()
+    s.load(bytes(state))
+    s.labels()
+    wrong = []
+
+    def read(what):
+        for _ in range(20):
+            if not np.array_equal(getattr(s, what)(), want[what]):
+                wrong.append(what)
+
+    threads = [threading.Thread(target=read, args=(w,)) for w in ("labels", "volume", "labels", "volume")]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, (n, len(wrong))
+""")

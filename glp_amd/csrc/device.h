@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "download.h"
 #include "hooks.h"
 
 namespace glp {
@@ -101,6 +102,7 @@ struct DeviceGraph {
     bool ascending = false;  // every neighbour list is strictly ascending (no repeats)
     bool owns_csr = true;   // false: off/nbr/w borrowed from another DeviceGraph
     bool owns_plan = true;  // false: the d_* plan arrays live in memory the graph does not own
+    Staging staging;        // of its sessions' copies to the caller
     ~DeviceGraph();
 };
 int device_graph_create(const HostCSR& g, const Tuning& t, hipStream_t s, DeviceGraph** out);

@@ -17,17 +17,21 @@ struct CopySlots {
 };
 
 constexpr int kCopyWorkers = 4;
-// A session's buffers, made when copies repeat and kept while it lives (1 MB,
-// and 16 MB once its copies are large).
+// The pinned buffers and the stream of copies, made when copies repeat and
+// kept: a graph's, for all sessions on it, as long as its device copy, or a
+// server's (1 MB, and 16 MB once its copies are large).
 struct Staging {
     std::mutex mu;  // held by the copy that uses them
+    hipStream_t stream = nullptr;
     CopySlots small, large[kCopyWorkers];
     bool used = false;  // a copy that could have used them was made
+    bool ready(size_t bytes);  // makes what a copy of `bytes` needs; false: not to be had
+    ~Staging();
 };
 
 // Copies `bytes` from the device to pageable host memory after the work
-// queued on s; returns when they are there.  Where the buffers cannot be had,
-// or are in use by a copy of another thread, the copy is a plain one.
+// queued on s; returns when they are there.  Where the buffers cannot be had
+// the copy is a plain one.
 int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s);
 
 }  // namespace glp

@@ -18,8 +18,12 @@ namespace glp {
 // 512 KB chunks 6.1 ms), threads do not pay below (16 MB 0.77-1.0 ms with any
 // number), and under 2 MB a plain copy into memory the program has used
 // before is faster (a pass with 1 MB of labels 821 / 909 us, 96 arrays of 0.2
-// MB 12.9 / 13.4 ms).  Making the slots takes about 0.1 ms, so a session's
-// first copy is plain unless it is large.
+// MB 12.9 / 13.4 ms).  Making the slots takes 0.1 ms (1 MB), so the first copy
+// is plain unless it is large; the large form's 16 MB take up to 5 ms to make,
+// use first and give back, so they stay with the graph and not with each
+// session (one-shot runs with a 32 MB result: plain 4.0 ms, slots made and
+// freed by each session 4.6-5.2, the graph's 2.4; 16 MB 1.38 / 1.20 / 1.05, 64
+// MB 8.7 / 5.5-6.6 / 6.1).
 constexpr size_t kCopyDirect = 2 << 20;
 constexpr size_t kCopyLarge = 16 << 20;
 constexpr size_t kSmallChunk = 512 << 10;
@@ -49,6 +53,22 @@ bool CopySlots::create(size_t bytes) {
         return false;
     }
     chunk = bytes;
+    return true;
+}
+
+Staging::~Staging() {
+    if (stream) (void)hipStreamDestroy(stream);
+}
+
+bool Staging::ready(size_t bytes) {
+    if (!stream && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) {
+        stream = nullptr;
+        (void)hipGetLastError();
+        return false;
+    }
+    if (bytes < kCopyLarge) return small.create(kSmallChunk);
+    for (auto& w : large)
+        if (!w.create(kLargeChunk)) return false;
     return true;
 }
 
@@ -91,38 +111,19 @@ static void* copy_share(void* arg) {
     return nullptr;
 }
 
-int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes == 0) return GLP_OK;
-    std::unique_lock<std::mutex> slots(st.mu, std::try_to_lock);
-    bool staged = false;
-    if (slots.owns_lock()) {
-        staged = bytes >= kCopyLarge || (st.used && bytes >= kCopyDirect);
-        st.used = true;
-        if (staged && bytes < kCopyLarge) staged = st.small.create(kSmallChunk);
-        else if (staged)
-            for (auto& w : st.large) staged = staged && w.create(kLargeChunk);
-    }
-    if (!staged) {
-        if (slots.owns_lock()) slots.unlock();
-        GLP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
-        GLP_HIP(hipStreamSynchronize(s));
-        return GLP_OK;
-    }
-    char* to = static_cast<char*>(dst);
-    const char* from = static_cast<const char*>(src);
-    if (bytes < kCopyLarge) {
-        const hipError_t e = copy_range(st.small, to, from, bytes, s);
-        return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(e));
-    }
+// The copy through st's slots (its lock held), st.ready for it.
+static hipError_t copy_staged(Staging& st, char* to, const char* from, size_t bytes) {
+    if (bytes < kCopyLarge) return copy_range(st.small, to, from, bytes, st.stream);
     int dev = 0;
-    GLP_HIP(hipGetDevice(&dev));
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
     const size_t share = ((bytes + kLargeChunk - 1) / kLargeChunk + kCopyWorkers - 1) / kCopyWorkers * kLargeChunk;
     CopyShare part[kCopyWorkers];
     pthread_t helper[kCopyWorkers];
     bool runs[kCopyWorkers] = {};
     for (int i = 0; i < kCopyWorkers; ++i) {
-        const size_t b = std::min(bytes, (size_t)i * share), e = std::min(bytes, b + share);
-        part[i] = CopyShare{&st.large[i], to + b, from + b, e - b, s, dev, hipSuccess};
+        const size_t b = std::min(bytes, (size_t)i * share), end = std::min(bytes, b + share);
+        part[i] = CopyShare{&st.large[i], to + b, from + b, end - b, st.stream, dev, hipSuccess};
         if (i) runs[i] = pthread_create(&helper[i], nullptr, copy_share, &part[i]) == 0;
     }
     // this thread takes the first share, and those for which no thread was to be had
@@ -131,7 +132,24 @@ int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStrea
     for (int i = 0; i < kCopyWorkers; ++i)
         if (runs[i]) (void)pthread_join(helper[i], nullptr);
     for (const CopyShare& p : part)
-        if (p.err != hipSuccess) return set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(p.err));
+        if (p.err != hipSuccess) return p.err;
+    return hipSuccess;
+}
+
+int copy_to_host(Staging& st, void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes >= kCopyDirect) {
+        GLP_HIP(hipStreamSynchronize(s));  // (the copies are not on s)
+        std::lock_guard<std::mutex> lock(st.mu);
+        const bool staged = (st.used || bytes >= kCopyLarge) && st.ready(bytes);
+        st.used = true;
+        if (staged) {
+            const hipError_t e = copy_staged(st, static_cast<char*>(dst), static_cast<const char*>(src), bytes);
+            return e == hipSuccess ? GLP_OK : set_error(GLP_E_HIP, "copying results: %s", hipGetErrorString(e));
+        }
+    }
+    if (bytes == 0) return GLP_OK;
+    GLP_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+    GLP_HIP(hipStreamSynchronize(s));
     return GLP_OK;
 }
 

@@ -2,7 +2,6 @@
 #pragma once
 
 #include "device.h"
-#include "download.h"
 
 #include <array>
 #include <vector>
@@ -63,7 +62,6 @@ struct glp_session {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     glp_timing timing{};
-    glp::Staging staging;                  // of copies to the caller
     std::vector<int64_t> host_changes;
     ~glp_session();
 };

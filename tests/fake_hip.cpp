@@ -113,6 +113,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     return give(p, n);
 }
 hipError_t hipHostFree(void* p) {
+    if (p) note("hipHostFree");
     std::free(p);
     return hipSuccess;
 }

@@ -118,3 +118,24 @@ for n in (3 << 19, (1 << 22) + 5):
         t.join()
     assert not wrong, (n, len(wrong))
 """)
+
+
+def test_copy_slots_stay_with_the_graph(fake_hip):
+    """The pinned slots of result copies are made once for all sessions on a
+    graph, one after another or alive together, and freed with it."""
+    fake_hip("""
+for n, slots in (((1 << 22) + 5, 4), (1 << 20, 1)):
+    g = edgeless(n)
+    log()
+    for _ in range(5):
+        G.run(g, 1)
+    a, b = G.Session(g), G.Session(g, method=G.LAYERED)
+    for s in (a, b, a):
+        s.labels()
+    a.free()
+    b.free()
+    seen = log()
+    assert sum(x.startswith("hipHostMalloc") for x in seen) == slots and "hipHostFree" not in seen
+    g.free()
+    assert log().count("hipHostFree") == slots
+""")

@@ -255,8 +255,28 @@ namespace glp {
 // 2.92, 21 4.12 / 4.44 against 5.10 / 5.53.
 constexpr int64_t kDomMinEdges = 1 << 24;
 static bool dominant_session(const HostCSR& g, const Plan& p, const glp_params& prm) {
-    return (prm.method == GLP_CLASSIC || prm.method == GLP_LAYERED) && !prm.weighted && !prm.gather &&
-           !prm.frontier && g.m >= kDomMinEdges && !p.hubs.empty();
+    return (prm.method == GLP_CLASSIC || (prm.method == GLP_LAYERED && prm.gamma_num == 0)) && !prm.weighted &&
+           !prm.gather && !prm.frontier && g.m >= kDomMinEdges && !p.hubs.empty();
+}
+// The memory that takes (a layered session's, once its gamma is 0); where it
+// cannot be had the session does without.
+static void make_dominant(glp_session* s) {
+    const HostCSR& g = s->g->csr;
+    if (s->domctl || !dominant_session(g, s->g->dev->plan, s->p)) return;
+    const size_t bits = dominant_bytes(g.n) + dominant_bytes(g.n / 64 + 1), ebits = dominant_bytes(g.m),
+                 act = (size_t)g.n;
+    if (hipMalloc(&s->dom_bits, bits) == hipSuccess && hipMalloc(&s->dom_ebits, ebits) == hipSuccess &&
+        hipMalloc(&s->dom_act, act) == hipSuccess && hipMalloc(&s->domctl, 16) == hipSuccess) {
+        s->bytes += bits + ebits + act + 16;
+        return;
+    }
+    (void)hipGetLastError();
+    (void)hipFree(s->dom_bits);
+    (void)hipFree(s->dom_ebits);
+    (void)hipFree(s->dom_act);
+    s->dom_bits = s->dom_ebits = nullptr;
+    s->dom_act = nullptr;
+    s->domctl = nullptr;
 }
 
 size_t session_bytes(const HostCSR& g, const Plan& p, const glp_params& prm) {
@@ -270,7 +290,6 @@ size_t session_bytes(const HostCSR& g, const Plan& p, const glp_params& prm) {
     if (prm.frontier) b += 2 * (n + 4);
     if (prm.frontier && prm.gather) b += 2 * ((n + 31) / 32) * 4 + push_entry_bytes(g.n, g.m);
     if (prm.frontier == 2 && prm.gather) b += (size_t)g.m * 4;  // the lookahead's second adj
-    if (dominant_session(g, p, prm)) b += dominant_bytes(g.n) + dominant_bytes(g.n / 64 + 1) + dominant_bytes(g.m) + n + 16;
     b += hub_scratch_bytes(p, prm.frontier != 0);
     b += 8 * kChangeSlots * kAccRows + 8 * kChangeRing + 4 + 4;  // change counters and ring, step and unit counters
     return b;
@@ -346,12 +365,6 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
             }
         }
     }
-    if (dominant_session(g->csr, p, *prm)) {
-        GLP_HIP(hipMalloc(&s->dom_bits, dominant_bytes(s->n) + dominant_bytes(s->n / 64 + 1)));
-        GLP_HIP(hipMalloc(&s->dom_ebits, dominant_bytes(g->csr.m)));
-        GLP_HIP(hipMalloc(&s->dom_act, nn));
-        GLP_HIP(hipMalloc(&s->domctl, 16));
-    }
     GLP_HIP(hipMalloc(&s->hs.work, 4));  // the persistent small-tier launch's counter
     GLP_HIP(hipMalloc(&s->d_acc, 8 * kChangeSlots * kAccRows));
     GLP_HIP(hipMalloc(&s->d_ring, 8 * kChangeRing));
@@ -360,6 +373,7 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
     GLP_HIP(hipEventCreate(&s->ev_stop));
     s->bytes = session_bytes(g->csr, p, *prm);
     if (counting_method(prm->method) && (rc = counting_wide_list(s.get())) != GLP_OK) return rc;
+    make_dominant(s.get());
     for (int t = 0; t < 4; ++t) {
         s->timing.tier_vertices[t] = p.verts[t];
         s->timing.tier_edges[t] = p.edges[t];
@@ -436,10 +450,11 @@ int end_steps(glp_session* s) {
 }
 
 int end_step(glp_session* s, const int32_t* nbr, const int32_t* Lw, bool replayed) {
-    if (replayed || s->fctl || s->domctl)
-        // (steps with gamma > 0 use no dominant label and choose none)
+    // (steps with gamma > 0 use no dominant label and choose none)
+    int32_t* domctl = s->method == Method::Layered && s->p.gamma_num > 0 ? nullptr : s->domctl;
+    if (replayed || s->fctl || domctl)
         return launch_end_step(step_counters(s), s->d_ring, s->d_ctr, kChangeRing, s->stream, s->fctl, nbr, Lw,
-                               s->g->csr.m, s->p.gamma_num == 0 ? s->domctl : nullptr);
+                               s->g->csr.m, domctl);
     return ++s->acc_rows == kAccRows ? end_steps(s) : GLP_OK;
 }
 
@@ -791,6 +806,7 @@ extern "C" int glp_session_set_gamma(glp_session* s, int32_t gamma_num, int32_t 
     int rc = check_params(s->g->csr, &q);
     if (rc != GLP_OK) return rc;
     s->p = q;
+    make_dominant(s);
     // gamma > 0 steps leave the choice of the last gamma = 0 step behind
     if (s->domctl && (rc = clear_dominant(s))) return rc;
     // captured step graphs baked the old scores in

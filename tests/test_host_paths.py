@@ -139,3 +139,59 @@ for n, slots in (((1 << 22) + 5, 4), (1 << 20, 1)):
     g.free()
     assert log().count("hipHostFree") == slots
 """)
+
+
+def test_dominant_label_scratch_only_where_it_is_used(fake_hip):
+    """Sessions on a large graph hold the dominant label's scratch, and end
+    their steps one by one, while gamma is 0; where that memory cannot be had
+    they run without it."""
+    fake_hip("""
+n = 1 << 22
+deg = np.full(n, 4, dtype=np.int64)
+deg[0] = 5000
+off = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+nbr = (np.arange(off[-1], dtype=np.int64) * 7919 % n).astype(np.int32)
+g = G.Graph.from_csr(off, nbr)
+scratch = n + g.m // 8  # at least
+
+def count(s, steps=3):
+    log()
+    s.step(steps)
+    seen = log()
+    return [sum(k in x for x in seen) for k in ("k_dominant_decide", "k_end_stepE", "k_end_stepsE")]
+
+G.Session(g).free()  # the graph's device copy
+held = []
+for gamma in ((1, 4), (0, 1)):
+    before = fake.fake_device_bytes()
+    s = G.Session(g, method=G.LAYERED, gamma=gamma)
+    held.append(fake.fake_device_bytes() - before)
+    if gamma[0]:
+        assert count(s) == [0, 0, 1]
+        before = fake.fake_device_bytes()
+        s.set_gamma(0, 1)
+        assert fake.fake_device_bytes() - before >= scratch
+        assert count(s) == [3, 3, 0]
+        s.set_gamma(1, 4)
+        assert count(s) == [0, 0, 1]
+        s.set_gamma(1, 2)
+        s.set_gamma(0, 1)
+        assert fake.fake_device_bytes() - before < 2 * scratch
+        s.reset()
+        assert count(s) == [2, 3, 0]  # none in the first step
+    s.free()
+assert held[1] - held[0] >= scratch
+for method in (G.CLASSIC, G.LAYERED):
+    s = G.Session(g, method=method)
+    whole = fake.fake_device_bytes()
+    s.free()
+    fake.fake_limit_device(whole - fake.fake_device_bytes() - 1)
+    s = G.Session(g, method=method)
+    assert count(s) == [0, 0, 1]
+    s.free()
+    fake.fake_limit_device(ctypes.c_size_t(-1).value)
+s = G.Session(g, method=G.LAYERED, gamma=(1, 4))
+fake.fake_limit_device(0)
+s.set_gamma(0, 1)
+assert count(s) == [0, 0, 1]
+""")

@@ -3,7 +3,8 @@
 //
 // Coordinate descent: starting from the current defaults, each key in turn
 // tries its candidate values with the others fixed and keeps a value that is
-// at least 2% faster; two sweeps.  A candidate reuses the graph's uploaded
+// at least 2% faster; two sweeps.  Values that make the same launches as the
+// key's default are left out.  A candidate reuses the graph's uploaded
 // CSR and only re-plans and re-uploads the tier lists.  Every tuning computes
 // the same labels (tiers differ only in how a vertex's count is organised),
 // so tuning never changes results.
@@ -12,6 +13,7 @@
 #include "session.h"
 
 #include <cstdio>
+#include <cstring>
 #include <fstream>
 #include <memory>
 
@@ -58,14 +60,24 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
     }
     DeviceGraph* base = g->dev;
 
-    // Times `steps` steps from L_0 with tuning t; ms < 0 when t is invalid.
-    auto time_tuning = [&](const Tuning& t, double* ms) -> int {
+    // Whether a plan's steps have the shapes of half_lanes 0 and block_threads
+    // 256 also with 32 and 512: the launch of all tiers has one shape.
+    auto fixed_shapes = [&](const Plan& plan) {
+        return !p->gather && !p->profile && tiers_in_one_launch(plan, plan.groups_with_edges);
+    };
+    // Times `steps` steps from L_0 with tuning t; ms < 0 when t is invalid or
+    // changes nothing.
+    auto time_tuning = [&](const Tuning& t, const char* key, double* ms) -> int {
         *ms = -1.0;
         auto dg = std::make_unique<DeviceGraph>();
         if (build_plan(g->csr, t, dg->plan) != GLP_OK) {
             clear_error();
             return GLP_OK;
         }
+        if (key && fixed_shapes(dg->plan) &&
+            ((!std::strcmp(key, "half_lanes") && t.half_lanes == 32) ||
+             (!std::strcmp(key, "block_threads") && t.block_threads == kTiersThreads)))
+            return GLP_OK;
         dg->n = base->n;
         dg->m = base->m;
         dg->off = base->off;
@@ -91,7 +103,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
     // from the graph's current tuning
     Tuning cur = base->plan.tune;
     double best = 0;
-    if ((rc = time_tuning(cur, &best)) != GLP_OK) return rc;
+    if ((rc = time_tuning(cur, nullptr, &best)) != GLP_OK) return rc;
     if (best < 0) return set_error(GLP_E_ARG, "current tuning is invalid for this graph");
     for (int sweep = 0; sweep < 2; ++sweep) {
         bool improved = false;
@@ -103,7 +115,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
                 Tuning t = cur;
                 tuning_set(t, c.key, v);
                 double ms = 0;
-                if ((rc = time_tuning(t, &ms)) != GLP_OK) return rc;
+                if ((rc = time_tuning(t, c.key, &ms)) != GLP_OK) return rc;
                 if (ms >= 0 && ms < best * 0.98) {
                     best = ms;
                     cur = t;

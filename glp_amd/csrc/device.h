@@ -70,6 +70,12 @@ struct Plan {
     int64_t edges[4] = {}, verts[4] = {};     // per tier: packed, wave, block, hub
 };
 int build_plan(const HostCSR& g, const Tuning& t, Plan& p);
+constexpr int kWaveNV = 4;          // wave-tier vertices per wave
+constexpr int kTiersThreads = 512;  // workgroup of the launch of all tiers (k_tiers)
+constexpr int kTiersWaves = kTiersThreads / 64;
+// Whether the plan's tiers, `groups` packed groups of them, are counted in
+// one launch (a step without a separate gather or tier timing).
+bool tiers_in_one_launch(const Plan& p, int64_t groups);
 
 // HBM copy of a graph plus its plan (shared by all sessions on the graph).
 // For each vertex u, the CSR positions j with nbr[j] = u: off[n+1], pos[m]

@@ -210,6 +210,31 @@ int build_plan(const HostCSR& g, const Tuning& t, Plan& p) {
     return GLP_OK;
 }
 
+// Each launch saved is worth about 5 us, and each workgroup runs with the
+// largest tier's registers and LDS.  12 steps, separate / together (thousands
+// of workgroups, launches): R-MAT scale 12 510 / 177 us, 16 873 / 437 us, 18
+// 1,123 / 907 us (10, 10), 19 1,737 / 2,362 us (20, 10); LFR 300,000 vertices
+// 1,098 / 953 us (9, 5); planted 65,536 525 / 494 us (2.3, 2), 100,000 of
+// degree 38 463 / 484 us (6, 2).
+// k_tiers has one shape: 32 lanes per half-tier vertex and 512 threads per
+// block-tier vertex.  A tuning that asks for another keeps its launches.
+constexpr int64_t kTogetherPerLaunch = 3500, kTogetherMax = 16384;
+bool tiers_in_one_launch(const Plan& p, int64_t groups) {
+    int64_t wgs = (int64_t)p.hub_chunks.size(), launches = p.hub_chunks.empty() ? 0 : 1;
+    bool blocks = false;
+    for (int c = 0; c < p.nclasses; ++c) {
+        wgs += (int64_t)p.block[c].size();
+        launches += p.block[c].empty() ? 0 : 1;
+        blocks |= !p.block[c].empty();
+    }
+    launches += (groups > 0) + !p.half.empty() + (p.wave_short > 0) + ((int64_t)p.wave.size() > p.wave_short);
+    wgs += ((int64_t)p.wave.size() / kWaveNV + (int64_t)p.half.size() / 2 + groups) / kTiersWaves;
+    if (p.tune.half_lanes == 16 && !p.half.empty()) return false;
+    if (p.tune.block_threads > kTiersThreads && blocks) return false;
+    return p.tune.fused_small == 0 && launches > 1 &&
+           wgs <= std::min(kTogetherMax, kTogetherPerLaunch * (launches - 1));
+}
+
 }  // namespace glp
 
 extern "C" int glp_tuning_set(const char* key, int32_t value) {

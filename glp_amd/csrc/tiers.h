@@ -716,7 +716,6 @@ __device__ __forceinline__ void half_body(const StepArgs& a, const int4* __restr
 // (4 per lane), so one round of branch-free loads covers it: the loads of all
 // kWaveNV vertices are issued first, then each vertex is counted in the
 // wave's LDS table in turn.
-constexpr int kWaveNV = 4;
 // EPL: edges loaded per lane (4 covers 256 edges; 2 serves vertices of at
 // most 128 edges without clamped duplicate loads)
 // The wave runs unit `wunit` (vertices [wunit kWaveNV, ...)) with its LDS
@@ -1379,9 +1378,7 @@ __global__ __launch_bounds__(256) void k_hub_mark(StepArgs a, HubArgs h) {
 // graphs every tier's launch takes 4-12 us, most of it starting and draining;
 // together they take about what the longest does.  A tier's registers and LDS
 // are the largest tier's, so a launch that fills the chip by itself is better
-// off alone (one_launch).
-constexpr int kTiersThreads = 512;
-constexpr int kTiersWaves = kTiersThreads / 64;
+// off alone (tiers_in_one_launch).
 constexpr size_t kTiersWaveLds = kWaveCap * 8;  // a wave's area (the wave tier's table)
 static_assert(sizeof(PackedLds) <= kTiersWaveLds && sizeof(HalfLds<32>) <= kTiersWaveLds, "wave areas");
 struct TierWork {
@@ -1538,25 +1535,6 @@ static uint32_t tier_work(const DeviceGraph& g, int32_t ng, TierWork& w, size_t*
     w.end_half = at += blocks(p.half.size(), kTiersWaves * 2);
     return at + blocks((size_t)ng, kTiersWaves);
 }
-// Whether a plan's tiers go in one launch (k_tiers): each launch saved is
-// worth about 5 us, and each workgroup runs with the largest tier's registers
-// and LDS.  12 steps, separate / together (thousands of workgroups, launches):
-// R-MAT scale 12 510 / 177 us, 16 873 / 437 us, 18 1,123 / 907 us (10, 10),
-// 19 1,737 / 2,362 us (20, 10); LFR 300,000 vertices 1,098 / 953 us (9, 5);
-// planted 65,536 525 / 494 us (2.3, 2), 100,000 of degree 38 463 / 484 us
-// (6, 2).
-constexpr int64_t kTogetherPerLaunch = 3500, kTogetherMax = 16384;
-static bool one_launch(const Plan& p, int32_t ng) {
-    int64_t wgs = (int64_t)p.hub_chunks.size(), launches = p.hub_chunks.empty() ? 0 : 1;
-    for (int c = 0; c < p.nclasses; ++c) {
-        wgs += (int64_t)p.block[c].size();
-        launches += p.block[c].empty() ? 0 : 1;
-    }
-    launches += (ng > 0) + !p.half.empty() + (p.wave_short > 0) + ((int64_t)p.wave.size() > p.wave_short);
-    wgs += ((int64_t)p.wave.size() / kWaveNV + (int64_t)p.half.size() / 2 + ng) / kTiersWaves;
-    return p.tune.fused_small == 0 && launches > 1 &&
-           wgs <= std::min(kTogetherMax, kTogetherPerLaunch * (launches - 1));
-}
 template <class H, bool W>
 static int launch_together(const DeviceGraph& g, const HubScratch& hs, const StepArgs& a, int32_t ng, hipStream_t s) {
     TierWork w;
@@ -1578,7 +1556,7 @@ static int launch_tiers(const DeviceGraph& g, const HubScratch& hs, const StepAr
                                                                        : (int64_t)p.groups.size());
     bool together = false;
     if constexpr (!G) {
-        together = !ev && one_launch(p, ng);  // (ev: the tiers are timed one by one)
+        together = !ev && tiers_in_one_launch(p, ng);  // (ev: the tiers are timed one by one)
         if (together) {
             const int rc = launch_together<H, W>(g, hs, a, ng, s);
             if (rc != GLP_OK) return rc;

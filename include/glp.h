@@ -114,7 +114,9 @@ int glp_device_count(int32_t* count);
  * wave_max_deg, block_max_deg, hub_chunk, part_keys, part_limit,
  * block_threads (256, the default: a single graph's block tier picks 256,
  * 512 or 1024 threads per workgroup by LDS table size, up to 16, 32 or
- * 64 KB; 512 or 1024: that many for every table size).                     */
+ * 64 KB; 512 or 1024: that many for every table size).  Small graphs count
+ * all tiers in one launch, of 32 lanes per vertex and 512 threads; half_lanes
+ * 16 and block_threads 1024 give them a launch per tier.                    */
 int glp_tuning_set(const char* key, int32_t value);
 int glp_tuning_get(const char* key, int32_t* value);
 /* Autotuner (no reference counterpart; replaces hand-picked constants):

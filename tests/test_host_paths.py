@@ -195,3 +195,46 @@ fake.fake_limit_device(0)
 s.set_gamma(0, 1)
 assert count(s) == [0, 0, 1]
 """)
+
+
+def test_one_launch_keeps_to_the_tuned_shapes(fake_hip):
+    """The launch of all tiers runs 32 lanes per half-tier vertex and 512
+    threads per block-tier vertex: other shapes asked for by tuning get their
+    own launches, and the autotuner times no value that the launch ignores."""
+    fake_hip("""
+def kernels(**tuned):
+    with G.tuning(**tuned):
+        s = G.Session(G.Graph.rmat(12, 16, seed=9))
+        s.step(1)  # (the first step has launches of its own kind)
+        log()
+        s.step(1)
+        return [x for x in log() if "ClassicHooks" in x]
+
+def has(seen, name):
+    return any(name in x for x in seen)
+
+for same in ({}, {"half_lanes": 32}, {"block_threads": 512}, {"half_lanes": 16, "half_max_deg": 0}):
+    seen = kernels(**same)
+    assert has(seen, "k_tiers") and not has(seen, "k_half") and not has(seen, "k_block"), (same, seen)
+seen = kernels(half_lanes=16)
+assert not has(seen, "k_tiers") and has(seen, "k_halfINS_12ClassicHooksELb0ELb0ELi1ELi16E"), seen
+seen = kernels(block_threads=1024)
+assert not has(seen, "k_tiers") and has(seen, "k_blockINS_12ClassicHooksELb0ELb0ELi1024E"), seen
+
+def tuned_runs(graph):  # per timed run of an autotuning: whether its steps were one launch each
+    log()
+    G.autotune(graph, G.make_params(), steps=2)
+    runs = []
+    for x in log():
+        if "k_reset" in x:
+            runs.append(False)
+        if "k_tiers" in x:
+            runs[-1] = True
+    return runs
+
+candidates = 1 + 4 + 2 + 2 + 3 + 4 + 2 + 2 + 2 + 1  # the tuning it begins with, and each key's other values
+runs = tuned_runs(G.Graph.rmat(12, 16, seed=9))
+assert len(runs) == candidates - 2  # (half_lanes 32 and block_threads 512)
+assert runs.count(False) == 3       # (half_lanes 16, block_threads 1024, fused_small 1)
+assert len(tuned_runs(G.Graph.rmat(19, 16, seed=9))) == candidates  # too large for one launch
+""")

@@ -96,6 +96,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
             if (r == GLP_OK) *ms = s->timing.steps_ms;
             delete s;
         }
+        base->ascending = dg->ascending;  // (found out by its first session)
         g->dev = base;
         return r;
     };

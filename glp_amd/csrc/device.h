@@ -105,7 +105,9 @@ struct DeviceGraph {
     InverseIndex inv;
     double upload_ms = 0, plan_ms = 0;
     size_t bytes = 0;
-    bool ascending = false;  // every neighbour list is strictly ascending (no repeats)
+    // 1: every neighbour list is strictly ascending (no repeats); 0: not; -1:
+    // not known (the first session that asks finds out)
+    int8_t ascending = -1;
     bool owns_csr = true;   // false: off/nbr/w borrowed from another DeviceGraph
     bool owns_plan = true;  // false: the d_* plan arrays live in memory the graph does not own
     Staging staging;        // of its sessions' copies to the caller
@@ -238,8 +240,9 @@ int inverse_index_build(const int32_t* nbr, int32_t n, int64_t m, int32_t* curso
 // (frontier control word 7); above it the gather rewrites every edge.
 int32_t push_edge_limit(int64_t m);
 // Whether every neighbour list of the device CSR is strictly ascending
-// (synchronises s).
-int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s, bool* yes);
+// (synchronises s; scratch: two counters).
+int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s,
+                         unsigned long long* scratch, bool* yes);
 // Random-read calibration: `reads` 4-byte reads of T (entries a power of
 // two) at uniform hashed indices; out holds out_entries int32 sums.
 int launch_calib_read(const int32_t* T, int64_t entries, int64_t reads, uint32_t seed, int32_t* out,

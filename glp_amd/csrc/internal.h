@@ -30,8 +30,7 @@ struct HostCSR {
     // vertex's out-neighbours, so it needs this); 0: not; -1: not yet known
     int8_t symmetric = -1;
     // 1: every neighbour list is strictly ascending (no repeats), so a first
-    // step needs no tables; 0: not; -1: not known (the device copy's upload
-    // checks it there)
+    // step needs no tables; 0: not; -1: not known (checked on the device copy)
     int8_t ascending = -1;
     bool weighted() const { return !weights.empty(); }
     void finish();  // computes max_degree

@@ -985,25 +985,21 @@ __global__ __launch_bounds__(256) void k_descents(const int32_t* __restrict__ of
     }
 }
 
-int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s, bool* yes) {
+int neighbours_ascending(const int32_t* off, const int32_t* nbr, int32_t n, int64_t m, hipStream_t s,
+                         unsigned long long* scratch, bool* yes) {
     *yes = true;
     if (m < 2) return GLP_OK;
-    unsigned long long* out = nullptr;
     unsigned long long got[2] = {0, 0};
-    GLP_HIP(hipMalloc(&out, sizeof got));
-    int rc = launch_zero_bytes(out, sizeof got, s);
-    hipError_t e = hipSuccess;
-    if (!rc) {
-        const unsigned grid = (unsigned)std::min<int64_t>(grid_for(m, 256), 256 * 32);
-        hipLaunchKernelGGL(k_descents, dim3(grid), dim3(256), 0, s, off, nbr, n, m, out);
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(got, out, sizeof got, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) rc = set_error(GLP_E_HIP, "neighbour order check: %s", hipGetErrorString(e));
-    }
-    (void)hipFree(out);
+    const int rc = launch_zero_bytes(scratch, sizeof got, s);
+    if (rc != GLP_OK) return rc;
+    const unsigned grid = (unsigned)std::min<int64_t>(grid_for(m, 256), 256 * 32);
+    hipLaunchKernelGGL(k_descents, dim3(grid), dim3(256), 0, s, off, nbr, n, m, scratch);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(got, scratch, sizeof got, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) return set_error(GLP_E_HIP, "neighbour order check: %s", hipGetErrorString(e));
     *yes = got[0] == got[1];
-    return rc;
+    return GLP_OK;
 }
 
 // Random 4-byte reads of a table with uniform fmix32 indices (the label

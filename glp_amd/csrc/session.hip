@@ -85,8 +85,7 @@ int device_graph_upload(const HostCSR& g, Plan&& plan, hipStream_t s, DeviceGrap
     if ((rc = upload(&dg->off, g.offsets.data(), (size_t)g.n + 1, s, bytes))) return rc;
     if ((rc = upload(&dg->nbr, g.neighbors.data(), (size_t)g.m, s, bytes))) return rc;
     if (g.weighted() && (rc = upload(&dg->w, g.weights.data(), (size_t)g.m, s, bytes))) return rc;
-    if (g.ascending >= 0) dg->ascending = g.ascending == 1;
-    else if ((rc = neighbours_ascending(dg->off, dg->nbr, g.n, g.m, s, &dg->ascending))) return rc;
+    dg->ascending = g.ascending;
     if ((rc = device_plan_upload(dg.get(), s))) return rc;
     double t2 = now_ms();
     dg->upload_ms = t2 - t1;
@@ -245,6 +244,13 @@ glp_session::~glp_session() {
 
 namespace glp {
 
+// Whether a session's step from L_0 is a first step (FirstHooks; the frontier
+// gather counts on the adj its steps fill, so gather sessions keep their form).
+static bool first_steps(Method method, const glp_params& prm) {
+    return !prm.gather && (method == Method::Layered || method == Method::Slpa ||
+                           (method == Method::Classic && !counting_method(prm.method)));
+}
+
 // Whether a session's steps look for a dominant label (k_dominant_edges):
 // unweighted classic counting on the labels themselves, the gather fused and
 // every vertex recomputed, on graphs with hubs (a label spreads over most of
@@ -374,6 +380,12 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
     s->bytes = session_bytes(g->csr, p, *prm);
     if (counting_method(prm->method) && (rc = counting_wide_list(s.get())) != GLP_OK) return rc;
     make_dominant(s.get());
+    if (g->dev->ascending < 0 && first_steps(s->method, *prm)) {
+        bool yes = false;
+        // (the ring is scratch until the reset clears it)
+        if ((rc = neighbours_ascending(dg.off, dg.nbr, dg.n, dg.m, s->stream, s->d_ring, &yes)) != GLP_OK) return rc;
+        g->dev->ascending = yes ? 1 : 0;
+    }
     for (int t = 0; t < 4; ++t) {
         s->timing.tier_vertices[t] = p.verts[t];
         s->timing.tier_edges[t] = p.edges[t];
@@ -387,8 +399,7 @@ int session_reset(glp_session* s) {
     const int64_t n = s->n;
     s->cur = 0;
     s->t = 0;
-    s->at_l0 = s->method == Method::Layered || s->method == Method::Slpa ||
-               (s->method == Method::Classic && !counting_method(s->p.method));
+    s->at_l0 = first_steps(s->method, s->p);
     s->timing.steps = 0;
     s->timing.steps_ms = 0;
     for (int i = 0; i < GLP_NTIERS; ++i) {
@@ -532,13 +543,11 @@ int enqueue_step(glp_session* s, hipEvent_t* ev, bool replayed) {
     // layered with gamma > 0: each neighbour's label travels with its
     // label's volume, and the tables accumulate scores (LayeredVolHooks)
     Method method = s->method;
-    // from L_0 no label is gathered (the frontier gather counts on the adj
-    // its steps fill, so gather sessions keep their form)
-    const bool first = s->at_l0 && !replayed && !s->p.gather;
+    const bool first = s->at_l0 && !replayed;  // from L_0 no label is gathered
     bool volumes = s->method == Method::Layered;  // still to be cleared
     if (first) {
         method = Method::First;
-        a.ascending = s->g->dev->ascending ? 1 : 0;
+        a.ascending = s->g->dev->ascending == 1 ? 1 : 0;
         a.write_isolated = s->method == Method::Slpa ? 1 : 0;
     } else if (s->method == Method::Layered && s->LV && s->p.gamma_num > 0) {
         method = Method::LayeredVol;

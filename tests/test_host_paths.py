@@ -238,3 +238,29 @@ assert len(runs) == candidates - 2  # (half_lanes 32 and block_threads 512)
 assert runs.count(False) == 3       # (half_lanes 16, block_threads 1024, fused_small 1)
 assert len(tuned_runs(G.Graph.rmat(19, 16, seed=9))) == candidates  # too large for one launch
 """)
+
+
+def test_neighbour_order_is_checked_where_it_is_used(fake_hip, tmp_path):
+    """Whether a file's neighbour lists ascend is found out for the first
+    session whose steps ask, once, without waiting for other work on the
+    device; serving such graphs does without."""
+    fake_hip("path = %r" % str(tmp_path / "g.bin") + """
+np.random.default_rng(3).integers(0, 300, (3000, 2)).astype(np.int32).tofile(path)
+g = G.Graph.load_bin(path)
+log()
+sv = G.Server(1 << 30, max_slots=4)
+gid = sv.add_graph(g)
+for jid in (sv.submit(g, 2), sv.submit_resident(gid, 2)):
+    sv.wait(jid, g.n)
+sv.close()
+a = G.Session(g, method=G.FREQUENT)
+b = G.Session(g, method=G.SEEDED)
+c = G.Session(g, gather=True)
+assert not any("k_descents" in x for x in log())
+sessions = [G.Session(g, method=m) for m in (G.LAYERED, G.CLASSIC, G.SLPA)]
+seen = log()
+assert sum("k_descents" in x for x in seen) == 1 and "hipFree" not in seen
+log()
+G.autotune(G.Graph.load_bin(path), G.make_params(), steps=1)
+assert sum("k_descents" in x for x in log()) == 1
+""")

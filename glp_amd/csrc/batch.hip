@@ -104,20 +104,27 @@ extern "C" int glp_batch_run(glp_batch* b, int32_t steps, int32_t mode, double* 
     clear_error();
     if (!b || steps < 0 || mode < 0 || mode > 2) return set_error(GLP_E_ARG, "bad batch run arguments");
     int rc;
-    auto t0 = std::chrono::steady_clock::now();
+    std::chrono::steady_clock::time_point t0;
+    // the time is that of the steps: what is queued before them (a reset) has ended
+    auto start = [&](glp_session* const* s, size_t count) {
+        for (size_t i = 0; ms && i < count; ++i) GLP_HIP(hipStreamSynchronize(s[i]->stream));
+        t0 = std::chrono::steady_clock::now();
+        return (int)GLP_OK;
+    };
     if (mode == 2) {
         if (b->plain.empty()) {
             b->plain.resize(b->graphs.size(), nullptr);
             for (size_t i = 0; i < b->graphs.size(); ++i)
                 if ((rc = session_create(b->graphs[i], &b->p, &b->plain[i])) != GLP_OK) return rc;
-            t0 = std::chrono::steady_clock::now();
         }
+        if ((rc = start(b->plain.data(), b->plain.size())) != GLP_OK) return rc;
         for (auto* s : b->plain) {
             if ((rc = session_step(s, steps)) != GLP_OK) return rc;
             if ((rc = session_sync(s)) != GLP_OK) return rc;
         }
     } else {
         if (!b->sess) return set_error(GLP_E_STATE, "the batch has no union session (autotune failed)");
+        if ((rc = start(&b->sess, 1)) != GLP_OK) return rc;
         rc = mode == 1 ? session_step_graph(b->sess, steps) : session_step(b->sess, steps);
         if (rc != GLP_OK) return rc;
         if ((rc = session_sync(b->sess)) != GLP_OK) return rc;

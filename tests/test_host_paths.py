@@ -264,3 +264,23 @@ log()
 G.autotune(G.Graph.load_bin(path), G.make_params(), steps=1)
 assert sum("k_descents" in x for x in log()) == 1
 """)
+
+
+def test_batch_time_begins_after_the_reset(fake_hip):
+    """A reset is queued and not waited for; the time that a batch's run
+    reports is that of its steps."""
+    fake_hip("""
+graphs = [G.Graph.planted(500, 5, 6.0, 2.0, seed=i) for i in range(3)]
+b = G.Batch(graphs)
+for mode, reset in ((0, False), (1, True), (2, True), (2, True), (0, True)):
+    if reset:
+        b.reset()
+    if mode == 2:
+        b.run(0, mode=2)  # (its sessions are made)
+        b.reset()
+    log()
+    b.run(2, mode=mode)
+    seen = log()
+    step = [i for i, x in enumerate(seen) if "k_tiers" in x or "k_packed" in x or x == "hipGraphLaunch"][0]
+    assert seen[:step].count("hipStreamSynchronize") >= (len(graphs) if mode == 2 else 1), (mode, seen)
+""")

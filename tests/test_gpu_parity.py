@@ -455,6 +455,35 @@ def test_dominant_label_settles_the_same_labels(sort):
     assert np.array_equal(dumps[0], dumps[1])
 
 
+@pytest.mark.parametrize("n,spread", [(1245184, 1), (1245185, 1), (1 << 22, 1), (1 << 22, 3), (41000003, 39)])
+def test_dominant_label_look_ups_of_large_vertex_ranges(n, spread):
+    """The edges pass looks a neighbour's bit up in LDS (all vertices up to
+    1,245,184; else the first ones), in a bit per block of 64 vertices (up to
+    39.8 M) or in memory: a graph of 2^20 vertices whose first 1,000 keep
+    their ids and whose others lie at the end of n, side by side or `spread`
+    apart.  The ids keep their order, so every step's labels are the small
+    graph's."""
+    g = G.Graph.rmat(20, 20, seed=14)
+    off, nbr, _ = g.csr()
+    steps = 8
+    want = gpu_steps(g, steps, gather=True)
+    assert np.bincount(want[steps - 2][nbr]).max() > 0.55 * g.m  # the last step has a dominant label
+    ids = n - spread * (g.n - np.arange(g.n, dtype=np.int64))
+    ids[:1000] = np.arange(1000)
+    deg = np.zeros(n, dtype=np.int64)
+    deg[ids] = np.diff(off)
+    ids = ids.astype(np.int32)
+    large = G.Graph.from_csr(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32), ids[nbr])
+    with G.Session(large) as s:
+        for t in range(steps):
+            s.step(1)
+            labels = np.arange(n, dtype=np.int32)
+            labels[ids] = ids[want[t]]
+            assert np.array_equal(s.labels(), labels), t
+        prev = np.vstack([np.arange(g.n, dtype=np.int32)[None], want[:-1]])
+        assert s.changes().tolist() == (want != prev).sum(axis=1).tolist()
+
+
 def test_dominant_label_counts_small_hubs_once():
     """With hubs from 129 edges on, the deciding pass leaves each of them to
     its own workgroup: the change counts are those of the labels."""

@@ -514,10 +514,6 @@ __device__ __forceinline__ uint64_t readlane_u64(uint32_t lo, uint32_t hi, int s
     return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)hi, src) << 32) |
            (uint32_t)__builtin_amdgcn_readlane((int)lo, src);
 }
-// Set bits of m below this lane.
-__device__ __forceinline__ uint32_t rank_below(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 constexpr int kTableBlk = 4;               // most chunks of 64 edges loaded together
 constexpr uint32_t kNoEdge = 0xfffffffeu;  // key of a lane past the last edge
@@ -631,7 +627,7 @@ __device__ __forceinline__ void table_chunk(uint32_t key, uint64_t all, uint64_t
                 uint64_t run = miss & ((d & (0ull - d)) - 1ull);  // d = 0: all of them
                 uint32_t n = (uint32_t)__popcll(run);
                 if (n > nfree) {
-                    const uint32_t r = rank_below(run);
+                    const uint32_t r = (uint32_t)lanes_below(run);
                     uint32_t skip = 0u;
                     if (live_n == 0ull) {
                         uint32_t turns = 0u, left = n;
@@ -694,12 +690,12 @@ __device__ __forceinline__ void table_chunk(uint32_t key, uint64_t all, uint64_t
         uint32_t* ks = lds;
         uint32_t* as = lds + 64;
         if (__builtin_amdgcn_inverse_ballot_w64(live_n)) {
-            const uint32_t r = rank_below(live_n);
+            const uint32_t r = (uint32_t)lanes_below(live_n);
             ks[r] = key;
             as[r] = An + (uint32_t)(__popc(mn_lo) + __popc(mn_hi));
         }
         wave_lds_sync();
-        const uint32_t r = rank_below(t.fr);
+        const uint32_t r = (uint32_t)lanes_below(t.fr);
         const bool takes = __builtin_amdgcn_inverse_ballot_w64(t.fr) && r < cnt;
         if (takes) {
             t.K = ks[r];

@@ -34,6 +34,11 @@ __device__ __forceinline__ T ld_stream(const T* p) {
     return __builtin_nontemporal_load(p);
 }
 
+// How many of the lanes below this one m holds.
+__device__ __forceinline__ int32_t lanes_below(uint64_t m) {
+    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
 // Reductions over the 64 lanes, every lane active; every lane receives the
 // result.  DPP moves combine each row of 16 (quad pairs, quad with mirror
 // quad, half-row with half-row), readlanes the four rows: about 15 vector and

@@ -307,11 +307,6 @@ struct PackedLds {
     unsigned long long best[64];         // per vertex slot: best packed score
 };
 
-// How many of the lanes below this one m holds.
-__device__ __forceinline__ int32_t lanes_below(unsigned long long m) {
-    return (int32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
 // Every lane's first and owner: a vertex's last edge lane takes a mark from
 // it (pushed by ds_permute; lanes nobody pushes to get 0), and an edge lane's
 // owner is the number of marks below it.  With vertices of no edges, that

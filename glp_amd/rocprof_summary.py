@@ -52,15 +52,26 @@ def read_counter(d, counter):
     return [(k, acc[k][0], acc[k][1]) for k in sorted(acc)]
 
 
-def split_steps(rows):
-    """Groups dispatches into steps closed by k_end_step; dispatches after the
-    last k_end_step are dropped."""
-    steps, cur = [], []
+STEP_ENDS = ("k_end_step", "k_end_steps")
+
+
+def split_steps(rows, begins=()):
+    """Groups dispatches into steps closed by k_end_step or k_end_steps;
+    dispatches after the last of them are dropped.  k_end_steps ends all steps
+    of a call: such steps come in one group, unless `begins` names the kernels
+    a step begins with (then dispatches before the first of them are
+    dropped)."""
+    steps, cur, begun = [], [], not begins
     for row in rows:
+        if row[1] in begins:
+            if begun:
+                steps.append(cur)
+            cur, begun = [], True
         cur.append(row)
-        if row[1] == "k_end_step":
-            steps.append(cur)
-            cur = []
+        if row[1] in STEP_ENDS:
+            if begun:
+                steps.append(cur)
+            cur, begun = [], not begins
     return steps
 
 
@@ -123,7 +134,7 @@ def cmd_traffic(a):
     per = {}
     for d, counter, scale in ((a.fetch_dir, "FETCH_SIZE", sc["fetch_scale"]),
                               (a.write_dir, "WRITE_SIZE", sc["write_scale"])):
-        steps = split_steps(read_counter(d, counter))
+        steps = split_steps(read_counter(d, counter), a.begins)
         need = a.warmup + a.steps + (1 + a.gather_steps if a.gather_steps else 0)
         if len(steps) < need:
             sys.exit("%s: %d steps found, %d expected" % (counter, len(steps), need))
@@ -163,7 +174,7 @@ def cmd_sizes(a):
     next to TCC_BUBBLE (the 128 B count FETCH_SIZE's formula uses)."""
     per = defaultdict(lambda: defaultdict(float))
     for c in SIZE_COUNTERS:
-        steps = split_steps(read_counter(a.dir, c))
+        steps = split_steps(read_counter(a.dir, c), a.begins)
         groups = {"main": steps[a.warmup:a.warmup + a.steps]}
         if a.gather_steps:
             g0 = a.warmup + a.steps + 1
@@ -204,8 +215,8 @@ def traffic_for(path, workload, session, families):
 
 def cmd_steps(a):
     """Per-step kernel time (ms per family) of the first LP session in a
-    --kernel-trace run: dispatches in start order, steps closed by
-    k_end_step, the first `steps` steps."""
+    --kernel-trace run: dispatches in start order, split_steps's steps, the
+    first `steps` of them."""
     files = _csvs(a.dir, "kernel_trace.csv")
     if not files:
         sys.exit("no kernel_trace.csv under %s" % a.dir)
@@ -216,11 +227,11 @@ def cmd_steps(a):
                 t0, t1 = int(r["Start_Timestamp"]), int(r["End_Timestamp"])
                 rows.append((t0, family(r["Kernel_Name"]), (t1 - t0) / 1e6))
     rows.sort()
-    steps = split_steps([(t, fam, ms) for t, fam, ms in rows])[: a.steps]
+    steps = split_steps([(t, fam, ms) for t, fam, ms in rows], a.begins)[: a.steps]
     fams = defaultdict(float)
     for st in steps:
         for _, fam, ms in st:
-            if fam != "k_end_step":
+            if fam not in STEP_ENDS:
                 fams[fam] += ms
     order = [f for f, _ in sorted(fams.items(), key=lambda kv: -kv[1])][: a.columns]
     out = ["# kernel time per LP step (ms, from the trace's start/end timestamps)",
@@ -313,6 +324,9 @@ def main():
     n.add_argument("dirs", nargs="+")
     n.add_argument("--match", action="append", default=[], help="keep kernels whose name holds this")
     n.add_argument("--command", required=True)
+    for q in (t, z, p):
+        q.add_argument("--begins", action="append", default=[],
+                       help="kernel that a step begins with (where steps are ended together)")
     a = ap.parse_args()
     {"stats": cmd_stats, "calibrate": cmd_calibrate, "traffic": cmd_traffic, "sizes": cmd_sizes,
      "steps": cmd_steps, "counters": cmd_counters}[a.cmd](a)

@@ -47,6 +47,19 @@ def test_split_steps_drops_the_unfinished_tail():
     assert [len(s) for s in steps] == [2, 2]
 
 
+def test_split_steps_ended_together():
+    """k_end_steps ends the steps of a call; named first kernels part them."""
+    call = [("k_volume_init", 0.0), ("k_a", 1.0), ("k_label_volumes", 0.0), ("k_a", 2.0), ("k_label_volumes", 0.0),
+            ("k_a", 3.0), ("k_end_steps", 0.0)]
+    rows = [(i, k, v) for i, (k, v) in enumerate([("k_reset", 0.0)] + call + call[2:] + [("k_end_step", 0.0)])]
+    assert [len(s) for s in RS.split_steps(rows)] == [8, 5, 1]
+    steps = RS.split_steps(rows, ("k_volume_init", "k_label_volumes"))
+    assert [[k for _, k, _ in s] for s in steps] == \
+        [["k_volume_init", "k_a"], ["k_label_volumes", "k_a"], ["k_label_volumes", "k_a", "k_end_steps"]] + \
+        [["k_label_volumes", "k_a"], ["k_label_volumes", "k_a", "k_end_steps"]]
+    assert [sum(v for _, _, v in s) for s in steps] == [1.0, 2.0, 3.0, 2.0, 3.0]
+
+
 def test_calibrate_and_traffic_windows(tmp_path):
     # calibration: copies of 1 MiB read as FETCH 512 KiB and WRITE 1024 KiB
     fc, wc = str(tmp_path / "cf"), str(tmp_path / "cw")

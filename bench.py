@@ -251,6 +251,7 @@ def layered_legs(args, G, g, n, m):
     out = {}
     for gn, gd in ((0, 1), (1, 4), (1, 1)):
         ls = G.Session(g, G.make_params(method=G.LAYERED, gamma=(gn, gd), profile=True))
+        ls.sync()
         t0 = time.perf_counter()
         ls.step(10)
         ls.sync()
@@ -293,8 +294,8 @@ def counting_legs(args, G, g, m):
                      ("buffer", {"method": G.BUFFER, "table_cap": 16})):
         s = G.Session(g, G.make_params(**kw))
         s.step(1)
-        s.sync()
         s.reset()
+        s.sync()
         t0 = time.perf_counter()
         s.step(3)
         s.sync()
@@ -313,6 +314,7 @@ def from_l0_and_parity(args, G, O, g, off, nbr, n, m):
     strided sample of every other tier, each from the GPU's labels of the
     step before."""
     s = G.Session(g, G.make_params(method=G.CLASSIC))
+    s.sync()
     t0 = time.perf_counter()
     s.step(10)
     s.sync()
@@ -425,7 +427,11 @@ def slpa_leg(args, G):
     ss = G.Session(lg, G.make_params(method=G.SLPA, slpa_T=20, slpa_r=(1, 10), seed=args.seed))
     ss.step(20)  # untimed pass: the kernels' first launches
     ss.sync()
+    t1 = time.perf_counter()
+    ss.slpa_post(8)  # the first post-processing makes the copies' pinned slots
+    first_pms = (time.perf_counter() - t1) * 1e3
     ss.reset()
+    ss.sync()
     t0 = time.perf_counter()
     ss.step(20)
     ss.sync()
@@ -435,7 +441,7 @@ def slpa_leg(args, G):
     pms = (time.perf_counter() - t1) * 1e3
     out = {"graph": "LFR-style n=2^20 (tau1 2.5, degrees [8,512], tau2 1.5, sizes [20,5000], mu 0.3), m=%d" % lg.m,
            "steps": 20, "ms_per_step": round(sms, 4), "GTEPS": round(lg.m / (sms / 1e3) / 1e9, 3),
-           "post_ms": round(pms, 2), "mean_communities_per_vertex": round(float(ns.mean()), 3),
+           "post_ms": round(pms, 2), "post_first_ms": round(first_pms, 2), "mean_communities_per_vertex": round(float(ns.mean()), 3),
            "algorithmic_bytes_per_step": 8 * lg.m + 16 * lg.n,
            "step_roofline_frac": round((8 * lg.m + 16 * lg.n) / (sms / 1e3) / 1e9 / HBM_PEAK_GBS, 4)}
     log("slpa LFR-1M: %.3f ms/step, post %.1f ms" % (sms, pms))
@@ -631,11 +637,13 @@ RR_READS = 1 << 28
 
 def bench_random_read(args, G):
     """Calibration of the label gather's access pattern: random 4-byte reads
-    from a 128 MiB and a 1 GiB table (library kernel k_calib_read)."""
+    (library kernel k_calib_read) from tables that fit an XCD's L2 (up to 4
+    MiB), and of 8 and 128 MiB and 1 GiB."""
     out = {"metric": "random 4-byte read calibration", "unit": "G reads/s", "reads_per_launch": RR_READS}
-    for entries in (RR_TABLE, 1 << 28):
+    for entries in (1 << 16, 1 << 18, 1 << 20, 1 << 21, RR_TABLE, 1 << 28):
         ms = G.calib_random_read(entries, RR_READS, 5)
-        out["table_%dMiB" % (entries * 4 >> 20)] = {"ms": round(ms, 4),
+        size = entries * 4
+        out["table_%dMiB" % (size >> 20) if size >> 20 else "table_%dKiB" % (size >> 10)] = {"ms": round(ms, 4),
                                                      "G_reads_per_s": round(RR_READS / (ms / 1e3) / 1e9, 2)}
     out["value"] = out["table_%dMiB" % (RR_TABLE * 4 >> 20)]["G_reads_per_s"]
     return out

@@ -93,8 +93,9 @@ static int check_tuning(const Tuning& t) {
         return set_error(GLP_E_ARG, "hub_chunk must be a multiple of 256 in [256, 8192]");
     if (t.part_keys < 256 || t.part_keys > 4096)
         return set_error(GLP_E_ARG, "part_keys must be in [256, 4096]");
-    // a pass stops after `limit` distinct labels (+ at most a workgroup's
-    // worth in flight): limit <= part_keys keeps that inside the table
+    // a pass stops after `limit` distinct labels and those then in flight (up
+    // to 1,024) or at a full table; with limit <= part_keys, half the slots,
+    // small tables mostly end by the limit
     if (t.part_limit < 0 || t.part_limit > t.part_keys)
         return set_error(GLP_E_ARG, "part_limit must be in [0, part_keys]");
     if (t.block_threads != 256 && t.block_threads != 512 && t.block_threads != 1024)

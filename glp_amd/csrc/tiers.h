@@ -520,8 +520,9 @@ __device__ __forceinline__ void packed_body(const StepArgs& a, const int2* __res
 // per launch like the packed tier's NG), their loads issued before any is
 // counted.  Group sums and maxima run over DPP rows (one shuffle more with 32
 // lanes) and both majority candidates share one sum: 244 -> 233 us a step
-// over 96 graphs' 1.6 M vertices of 33 to 64 edges, of which bringing the
-// label lines into L1 (about 300 G lines/s) takes 200.
+// over 96 graphs' 1.6 M vertices of 33 to 64 edges.  Latency bound: the L1s
+// wait for L2 63% of the time, at 124 G line requests/s of the 262 that random
+// reads get from L2.
 constexpr uint32_t kHalfCap = 2 * kHalfMaxDeg;
 
 // Per-wave LDS of the half tier: one (key << 32 | sum) table per lane group.
@@ -1043,7 +1044,8 @@ struct PartJob {
 // every wave walks them all and takes a quarter of the pairs.  `bounded`: the
 // table holds all of the part's pairs, and they all are in range.  Otherwise
 // it stops early (the caller halves the range) once more than `limit`
-// distinct keys arrived; the table has room for limit + kHubThreads.
+// distinct keys arrived; up to kU * kHubThreads more can come in before every
+// wave sees that, and a key that finds the table full stops it too.
 // Bound by its instructions (41% of the VALU's cycles, 62% of the LDS's):
 // marks take one permute and one look-up a pair where a binary search took
 // nine, which brought R-MAT scale 25 from 687 to 655 us a step and the

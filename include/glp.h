@@ -82,7 +82,9 @@ typedef struct glp_params {
 /* Per-tier timing and shape record.  Replaces header/test_result.h:5-23
  * (Test_result): times are milliseconds from HIP events, not host clocks.
  * The gather slot times the separate gather, or in a fused session the passes
- * that settle vertices by a dominant label. */
+ * that settle vertices by a dominant label.  With profile = 1 every tier is a
+ * launch of its own; without it small graphs count all tiers in one launch,
+ * whose time these slots do not give. */
 enum { GLP_TIER_PACKED = 0, GLP_TIER_WAVE = 1, GLP_TIER_BLOCK = 2, GLP_TIER_HUB = 3,
        GLP_TIER_GATHER = 4, GLP_TIER_PICK = 5, GLP_TIER_AUX = 6, GLP_NTIERS = 8 };
 typedef struct glp_timing {
@@ -176,7 +178,8 @@ int glp_run_seeded(glp_graph* g, const glp_params* p, const uint8_t* seeds, int3
 /* Uploads the CSR (once per graph), plans tiers and allocates label state;
  * labels start at L_0[v] = v (header/kernel.cuh:444-451 initialize_labels). */
 int glp_session_create(glp_graph* g, const glp_params* p, glp_session** out);
-/* Resets labels to L_0 and the step counter to 0.                           */
+/* Resets labels to L_0 and the step counter to 0 (queued on the session's
+ * stream, not waited for).                                                  */
 int glp_session_reset(glp_session* s);
 /* Enqueues `steps` steps on the session's stream (asynchronous).  One step is
  * the body of the reference loop prop/classicLprop.cuh:361-443: PickLabel,
@@ -245,7 +248,8 @@ int glp_batch_create(int32_t ngraphs, glp_graph* const* graphs,
                      const glp_params* p, glp_batch** out);
 /* mode 0: the union's launches, enqueued per step; mode 1: the same steps
  * replayed from a captured HIP graph; mode 2: plain per-graph session
- * launches (the comparison form).                                          */
+ * launches (the comparison form).  *ms: the steps' time, what was queued
+ * before them (a reset) excluded.                                          */
 int glp_batch_run(glp_batch* b, int32_t steps, int32_t mode, double* ms);
 int glp_batch_labels(glp_batch* b, int32_t graph, int32_t* out);
 int glp_batch_reset(glp_batch* b);

@@ -138,6 +138,7 @@ extern "C" int glp_autotune(glp_graph* g, const glp_params* p, int32_t steps, co
         dg->nbr = base->nbr;
         dg->w = base->w;
         dg->ascending = base->ascending;
+        dg->staging = base->staging;
         if ((rc = device_plan_upload(dg.get(), stream)) != GLP_OK) return rc;
         dg->owns_csr = true;
         base->owns_csr = false;

@@ -147,7 +147,7 @@ extern "C" int glp_batch_labels(glp_batch* b, int32_t graph, int32_t* out) {
     if (rc != GLP_OK) return rc;
     if (n == 0) return GLP_OK;
     const int32_t bs = (int32_t)b->base[graph];
-    rc = copy_to_host(b->uni->dev->staging, out, b->sess->L[b->sess->cur] + bs, sizeof(int32_t) * (size_t)n,
+    rc = copy_to_host(*b->sess->staging, out, b->sess->L[b->sess->cur] + bs, sizeof(int32_t) * (size_t)n,
                       b->sess->stream);
     for (int32_t v = 0; rc == GLP_OK && v < n; ++v) out[v] -= bs;
     return rc;

@@ -1196,9 +1196,9 @@ int slpa_post(glp_session* s, int32_t kmax, int32_t* dominant, int32_t* nsets, i
                        s->p.slpa_r_num, s->p.slpa_r_den, kmax, d_dom, d_ns, d_sets);
     GLP_HIP(hipGetLastError());
     int rc = GLP_OK;
-    if (dominant) rc = copy_to_host(s->g->dev->staging, dominant, d_dom, (size_t)n * 4, s->stream);
-    if (!rc && nsets) rc = copy_to_host(s->g->dev->staging, nsets, d_ns, (size_t)n * 4, s->stream);
-    if (!rc && kmax > 0 && sets) rc = copy_to_host(s->g->dev->staging, sets, d_sets, (size_t)n * kmax * 4, s->stream);
+    if (dominant) rc = copy_to_host(*s->staging, dominant, d_dom, (size_t)n * 4, s->stream);
+    if (!rc && nsets) rc = copy_to_host(*s->staging, nsets, d_ns, (size_t)n * 4, s->stream);
+    if (!rc && kmax > 0 && sets) rc = copy_to_host(*s->staging, sets, d_sets, (size_t)n * kmax * 4, s->stream);
     GLP_HIP(hipStreamSynchronize(s->stream));  // before the arrays go
     return rc;
 }

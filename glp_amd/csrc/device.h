@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "internal.h"
@@ -110,7 +111,7 @@ struct DeviceGraph {
     int8_t ascending = -1;
     bool owns_csr = true;   // false: off/nbr/w borrowed from another DeviceGraph
     bool owns_plan = true;  // false: the d_* plan arrays live in memory the graph does not own
-    Staging staging;        // of its sessions' copies to the caller
+    std::shared_ptr<Staging> staging;  // of its sessions' copies to the caller (the first one makes it)
     ~DeviceGraph();
 };
 int device_graph_create(const HostCSR& g, const Tuning& t, hipStream_t s, DeviceGraph** out);

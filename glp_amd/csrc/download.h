@@ -18,8 +18,8 @@ struct CopySlots {
 
 constexpr int kCopyWorkers = 4;
 // The pinned buffers and the stream of copies, made when copies repeat and
-// kept: a graph's, for all sessions on it, as long as its device copy, or a
-// server's (1 MB, and 16 MB once its copies are large).
+// kept: a graph's, for all sessions on it, as long as its device copy or one
+// of them is there, or a server's (1 MB, and 16 MB once its copies are large).
 struct Staging {
     std::mutex mu;  // held by the copy that uses them
     hipStream_t stream = nullptr;

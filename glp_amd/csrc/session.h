@@ -62,6 +62,7 @@ struct glp_session {
     hipEvent_t ev_start = nullptr, ev_stop = nullptr;
     hipGraphExec_t graph_exec[2] = {nullptr, nullptr};
     glp_timing timing{};
+    std::shared_ptr<glp::Staging> staging;  // the graph's, for copies to the caller
     std::vector<int64_t> host_changes;
     ~glp_session();
 };

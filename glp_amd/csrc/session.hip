@@ -323,6 +323,8 @@ int session_create(glp_graph* g, const glp_params* prm, glp_session** out) {
         s->timing.upload_ms = dg->upload_ms;
         s->timing.plan_ms = dg->plan_ms;
     }
+    if (!g->dev->staging) g->dev->staging = std::make_shared<Staging>();
+    s->staging = g->dev->staging;
     const DeviceGraph& dg = *g->dev;
     const Plan& p = dg.plan;
     const size_t n = (size_t)s->n;
@@ -695,7 +697,7 @@ int session_labels(glp_session* s, int32_t* out) {
     int rc = session_sync(s);
     if (rc != GLP_OK) return rc;
     const int32_t* src = s->method == Method::Slpa ? s->mem + (size_t)s->t * s->n : s->L[s->cur];
-    return copy_to_host(s->g->dev->staging, out, src, sizeof(int32_t) * (size_t)s->n, s->stream);
+    return copy_to_host(*s->staging, out, src, sizeof(int32_t) * (size_t)s->n, s->stream);
 }
 
 int session_changes(glp_session* s, int64_t* out, int32_t cap, int32_t* nsteps) {
@@ -854,14 +856,14 @@ extern "C" int glp_session_volume(glp_session* s, int32_t* out) {
     if (!s->V[0]) return set_error(GLP_E_STATE, "volume exists for layered sessions only");
     int rc = session_sync(s);
     if (rc != GLP_OK) return rc;
-    return copy_to_host(s->g->dev->staging, out, s->V[s->cur], sizeof(int32_t) * (size_t)s->n, s->stream);
+    return copy_to_host(*s->staging, out, s->V[s->cur], sizeof(int32_t) * (size_t)s->n, s->stream);
 }
 extern "C" int glp_session_slpa_memory(glp_session* s, int32_t* out) {
     GLP_GUARD(s);
     if (!s->mem) return set_error(GLP_E_STATE, "memory exists for SLPA sessions only");
     int rc = session_sync(s);
     if (rc != GLP_OK) return rc;
-    return copy_to_host(s->g->dev->staging, out, s->mem, sizeof(int32_t) * (size_t)(s->t + 1) * s->n, s->stream);
+    return copy_to_host(*s->staging, out, s->mem, sizeof(int32_t) * (size_t)(s->t + 1) * s->n, s->stream);
 }
 
 struct StateHeader {

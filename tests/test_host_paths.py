@@ -141,6 +141,25 @@ for n, slots in (((1 << 22) + 5, 4), (1 << 20, 1)):
 """)
 
 
+def test_results_are_read_after_the_graph_is_freed(fake_hip):
+    """A session's labels can still be copied when its graph has gone; the
+    slots go with the last of them."""
+    fake_hip("""
+n = (1 << 22) + 5
+g = edgeless(n)
+s = G.Session(g)
+lab = with_labels(s, n)
+for gone in (False, True):
+    if gone:
+        log()
+        g.free()
+        assert "hipHostFree" not in log()
+    assert np.array_equal(s.labels(), lab)
+s.free()
+assert log().count("hipHostFree") == 4
+""")
+
+
 def test_dominant_label_scratch_only_where_it_is_used(fake_hip):
     """Sessions on a large graph hold the dominant label's scratch, and end
     their steps one by one, while gamma is 0; where that memory cannot be had
